@@ -677,9 +677,10 @@ size_t mfma_ws_bytes(int kind, int op, int n_units, int k_t, int m_rows, const P
   // room for the split-K records, for the normalised rows of an RMSNorm prologue and, for a
   // plain prompt block, for the prefill kernel's per-group sums of x
   const size_t split = split_part_bytes(plan_gemm(kind, op, n_units, k_t, m_rows, P));
-  const size_t pf = op == GOP_PLAIN ? pf_ws_bytes(n_units, k_t, m_rows) : 0;
-  return Q4NX_WS_COUNTER_BYTES + align256(split) + align256((size_t)m_rows * k_t * kTileK * 2) +
-         pf;
+  const size_t pf = op == GOP_PLAIN ? pf_ws_bytes(kind, n_units, k_t, m_rows) : 0;
+  const size_t pq = kind == Q4NX_KIND_Q4 && op != GOP_QKV && m_rows >= kPqRows ? pq_ws_bytes(op, n_units, k_t, m_rows) : 0;
+  const size_t b = align256(split) + align256((size_t)m_rows * k_t * kTileK * 2) + pf;
+  return Q4NX_WS_COUNTER_BYTES + (pq > b ? pq : b);
 }
 
 bool mfma_norm_fits(int k_t, int m_rows, size_t ws_bytes) {
@@ -699,6 +700,14 @@ int mfma_launch(int kind, int op, GemmArgs& a, int n_units, void* ws, size_t ws_
   const size_t xn_b = a.norm_w != nullptr && a.xn_out == nullptr
                           ? align256((size_t)a.m_rows * K * 2) : 0;
   const bool ws_ok = ws != nullptr && Q4NX_ALIGNED(ws, 256);
+  // a prompt block of q4 tiles: the fp16-operand kernel, when the workspace holds what it keeps
+  // there (a K split that the policy names belongs to the batched kernel)
+  if (pq_use(kind, op, a) && ws_ok && P.gemm_ksplit == 0 &&
+      (a.norm_w == nullptr || (a.ssq_in != nullptr && K / kSsqRows <= 512)) &&
+      ws_bytes >= Q4NX_WS_COUNTER_BYTES + pq_ws_bytes(op, a.n_tr[0], a.k_t, a.m_rows)) {
+    pq_launch(op, a, (uint8_t*)ws + Q4NX_WS_COUNTER_BYTES, st);
+    return check_launch(what);
+  }
   if (split && (!ws_ok || ws_bytes < Q4NX_WS_COUNTER_BYTES + align256(split) + xn_b)) {
     split = 0;   // no (or too small a) workspace: whole K per workgroup
     p.ksplit = 1;
@@ -725,8 +734,8 @@ int mfma_launch(int kind, int op, GemmArgs& a, int n_units, void* ws, size_t ws_
   // a prompt block: the prefill kernel, when the workspace holds its per-group sums of x
   // (past the counters, the split records and the normalised rows); else the batched kernel
   const size_t pf_off = Q4NX_WS_COUNTER_BYTES + align256(split) + xn_b;
-  if (pf_use(op, a) && ws_ok && ws_bytes >= pf_off + pf_ws_bytes(a.n_tr[0], a.k_t, a.m_rows)) {
-    pf_launch(kind, a, (uint8_t*)ws + pf_off, st);
+  if (pf_use(kind, op, a) && ws_ok && ws_bytes >= pf_off + pf_ws_bytes(kind, a.n_tr[0], a.k_t, a.m_rows)) {
+    pf_launch(a, (uint8_t*)ws + pf_off, st);
     return check_launch(what);
   }
   // one m-tile reads x through a buffer resource with 32-bit byte offsets
@@ -764,9 +773,12 @@ size_t q4nx_gemm_ws_bytes(int kind, int n_tile_rows, int k_tiles, int m_rows,
       m_rows < 1 || !resolve_policy_quiet(policy, &P))
     return 0;
   const size_t split = gemm_split_bytes(plan_gemm(kind, GOP_PLAIN, n_tile_rows, k_tiles, m_rows, P));
-  const size_t pf = pf_ws_bytes(n_tile_rows, k_tiles, m_rows);
+  const size_t pf = pf_ws_bytes(kind, n_tile_rows, k_tiles, m_rows);
   // the prefill kernel's sums sit past the counters and the split records
-  return pf ? (split ? split : Q4NX_WS_COUNTER_BYTES) + pf : split;
+  const size_t b = pf ? (split ? split : Q4NX_WS_COUNTER_BYTES) + pf : split;
+  const size_t pq = kind == Q4NX_KIND_Q4 && m_rows >= kPqRows
+                        ? Q4NX_WS_COUNTER_BYTES + pq_ws_bytes(GOP_PLAIN, n_tile_rows, k_tiles, m_rows) : 0;
+  return pq > b ? pq : b;
 }
 
 int q4nx_gemm(int kind, const uint8_t* w, int n_tile_rows, int k_tiles, const uint16_t* x,

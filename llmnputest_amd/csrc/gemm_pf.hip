@@ -433,26 +433,25 @@ int pf_block_mtiles(int n_tile_rows, int m_rows) {
 
 }  // namespace
 
-size_t pf_ws_bytes(int n_tile_rows, int k_t, int m_rows) {
-  if (pf_block_mtiles(n_tile_rows, m_rows) == 0) return 0;
+size_t pf_ws_bytes(int kind, int n_tile_rows, int k_t, int m_rows) {
+  if (kind != Q4NX_KIND_Q8 || pf_block_mtiles(n_tile_rows, m_rows) == 0) return 0;
   return pf_align256((size_t)pf_mtiles(m_rows) * pf_chunks(k_t) * 3 * 64 * sizeof(u32x4_t));
 }
 
 // A plain contraction goes to the prefill kernel when it fills the chip (pf_block_mtiles), with
 // no sums-of-squares or argmax epilogue (those stay on the batched kernel).
-bool pf_use(int op, const GemmArgs& a) {
+bool pf_use(int kind, int op, const GemmArgs& a) {
   return op == GOP_PLAIN && a.ssq_out == nullptr && a.argmax_keys == nullptr &&
-         pf_ws_bytes(a.n_tr[0], a.k_t, a.m_rows) > 0;
+         pf_ws_bytes(kind, a.n_tr[0], a.k_t, a.m_rows) > 0;
 }
 
-void pf_launch(int kind, const GemmArgs& a, void* sums, hipStream_t st) {
+void pf_launch(const GemmArgs& a, void* sums, hipStream_t st) {
   const int n_ch = pf_chunks(a.k_t);
   hipLaunchKernelGGL(pf_sums_kernel, dim3((unsigned)(pf_mtiles(a.m_rows) * n_ch)), dim3(256), 0,
                      st, a.x, a.x_stride, a.m_rows, a.k_t * 8, n_ch, (u32x4_t*)sums);
   const bool big = pf_block_mtiles(a.n_tr[0], a.m_rows) == kPfMT;
   const u32x4_t* sp = (const u32x4_t*)sums;
-  if (kind == Q4NX_KIND_Q4) big ? pf_go<4, kPfMT>(a, sp, st) : pf_go<4, kPfMT / 2>(a, sp, st);
-  else big ? pf_go<8, kPfMT>(a, sp, st) : pf_go<8, kPfMT / 2>(a, sp, st);
+  big ? pf_go<8, kPfMT>(a, sp, st) : pf_go<8, kPfMT / 2>(a, sp, st);
 }
 
 }  // namespace q4nx

@@ -1,0 +1,885 @@
+// Prompt-block contraction of q4 tiles on the matrix cores (gfx950), weights and activations
+// as fp16 operands: Y[m][n] = R[m][n] + sum_k W[n][k] X[m][k], and [gate, up, SwiGLU].
+//
+// Replaces, for prompt blocks, the torch fallback that reference/npu.py:118-122, 138-140 takes
+// for more than one row.
+//
+// Arithmetic. Per column n and 32-K group g, with the Q4_1 factoring of granite_gemv.h:19-29 and
+// an offset o[n][g] near 7.5 d[n][g],
+//   y[m][n] = sum_k (d[n][g] c[n][k] - o[n][g]) x[m][k] + sum_g u[n][g] S[m][g]
+//   S[m][g] = sum_{k in g} x[m][k]     u[n][g] = m[n][g] + o[n][g]
+// A code's four bits under a fixed fp16 exponent are the value B + c (B = 1024 for a low nibble,
+// 64 for a high one), so d c - o is one fp16 multiply-add, d (B + c) + A with A the fp16 value
+// of -(B + 7.5) d. d has 8 significant bits and A is a multiple of at most 128 of their last
+// place, so the result is a multiple of that place below 2^11 of them: exact. A's own rounding
+// is in o = -(B d + A), hence in u. x is an exact fp16 value under a power of two per row, d
+// under one per column (an entry 2^28 below its row's largest loses bits, 2^-39 of that
+// largest). The first sum is therefore v_mfma_f32_16x16x32_f16 alone, one per 16x16 block and
+// group with exact products: no per-group scale on the VALU, and no large offset to cancel
+// afterwards. The second sum is a contraction over the groups (32 per MFMA), S and u each in two
+// fp16 terms (the product of the two low terms, 2^-22, is left out). A one-hot row still gives
+// the float32 dequantised column bit for bit.
+//
+// What bounds it: see pq_kernel.
+#include "common.h"
+#include "gemm.h"
+#include "gemm_fmt.h"
+
+namespace q4nx {
+
+namespace {
+
+typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
+typedef unsigned short us2_t __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ f32x4_t mfma_f16(const u32x4_t& a, const u32x4_t& b, f32x4_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a),
+                                                __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ uint32_t pk_max_u16(uint32_t a, uint32_t b) {
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(us2_t, a),
+                                                                __builtin_bit_cast(us2_t, b)));
+}
+// two fp32 values that fp16 holds exactly (or far below the scale's largest), packed
+__device__ __forceinline__ uint32_t pk_f16(float lo, float hi) {
+  return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(lo, hi));
+}
+// v = hi + lo to 2^-22: the two terms of a pair of values as packed fp16 words
+__device__ __forceinline__ void split2(float v0, float v1, uint32_t& hi, uint32_t& lo) {
+  const half2_t h = {(_Float16)v0, (_Float16)v1};
+  const half2_t r = {(_Float16)(v0 - (float)h.x), (_Float16)(v1 - (float)h.y)};
+  hi = h2_bits(h);
+  lo = h2_bits(r);
+}
+
+constexpr int kPqChunkTiles = 4;      // K-tiles (32 groups) per minimum-term contraction
+constexpr int kPqHalf = 2560;         // LDS bytes of half a tile: codes of 128 K, their scales
+constexpr int kPqXTop = 141;          // 141 - exponent field: the row's largest x in [2^14, 2^15)
+constexpr int kPqWTop = 135;          // |u| of a column below 2^9, its 8 |d| below 2^8
+constexpr int kPqSum = 6;             // S is kept 2^6 below its row's scale, u 2^6 above its column's
+constexpr float kPqLow = -1031.5f, kPqHigh = -71.5f;   // A / d of the low and the high nibbles
+constexpr int kPqSlack = 64 << 10;    // bytes after x that steps past its end read (never used)
+
+// The pre-pass's output (workspace), all in the order the contraction's operands take it: x as
+// fp16, its group sums, every column's u, and the powers of two.
+struct PqX {
+  u32x4_t* xt;      // [m-tile][32-K step][row % 16][k / 8 ^ row / 2 % 4]: 8 fp16 values; after
+                    // the steps, two of sums (hi, lo) per chunk of 32 groups, k the group
+  u32x4_t* u;       // [tensor][tile-row][chunk][hi, lo][even, odd column][lane]
+  uint2* scale;     // [tensor][tile-row][group][lane % 16]: fp16 d of the even and odd column, A
+  int* xshift;      // [row]: the power of two of x
+  int* wshift;      // [tensor][column]: that of d, A and u
+};
+
+// The larger of each lane's value and its DPP / permlane partner's, over the whole wave
+template <int CTRL>
+__device__ __forceinline__ uint32_t umax_dpp(uint32_t v) {
+  const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, false);
+  return pk_max_u16(v, o);
+}
+__device__ __forceinline__ uint32_t rows_max(uint32_t v) {    // across the four rows of 16 lanes
+  const auto a = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  v = pk_max_u16(a[0], a[1]);
+  const auto b = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  return pk_max_u16(b[0], b[1]);
+}
+
+// 2^e as a float, -126 <= e <= 127
+__device__ __forceinline__ float exp2i(int e) { return __int_as_float((e + 127) << 23); }
+
+constexpr int kPrepThreads = 256;
+
+// One row of x per workgroup: x (or RMSNorm of the fp32 residual, to bf16 first, as every
+// consumer rounds it) to fp16 under the row's power of two, and the sums per 32-K group. Each
+// thread keeps C chunks of 8 entries (K <= 2048 C; longer rows are read again for the second
+// pass). Every load is unconditional, through a buffer resource over the row: entries past its
+// end read zeros. Rows past m_rows stay unwritten: a row of an operand reaches its own row of
+// the result only. The code is kept short: a wave runs it once, so its instruction fetches are
+// not amortised (eight rows per workgroup, a wave each with up to 16 chunks, took 2.5 times as
+// long).
+template <bool NORM, int C>
+__device__ __forceinline__ void prep_row(const GemmArgs& a, const PqX& o, int row,
+                                         float* __restrict__ sg, uint32_t* __restrict__ smx) {
+  const int tid = threadIdx.x, l = tid & 63, wave = tid >> 6;
+  const int K = a.k_t * kTileK, n_q = K / 8;
+  const int n_ch = (a.k_t + kPqChunkTiles - 1) / kPqChunkTiles;
+  auto ld = [](__amdgpu_buffer_rsrc_t r, uint32_t off) {
+    const v4i_t t = __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0);
+    return u32x4_t{(uint32_t)t.x, (uint32_t)t.y, (uint32_t)t.z, (uint32_t)t.w};
+  };
+  const __amdgpu_buffer_rsrc_t xr =
+      NORM ? make_rsrc(a.hres + (int64_t)row * a.x_stride, (uint32_t)K * 4u)
+           : make_rsrc(a.x + (int64_t)row * a.x_stride, (uint32_t)K * 2u);
+  u32x4_t v[C];
+  uint32_t mx = 0;
+  auto see = [&](const u32x4_t& w) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) mx = pk_max_u16(mx, w[j] & 0x7FFF7FFFu);
+  };
+  if constexpr (NORM) {
+    const __amdgpu_buffer_rsrc_t wr = make_rsrc(a.norm_w, (uint32_t)K * 2u);
+    const int n_ss = K / kSsqRows;              // <= 512
+    u32x4_t h0[C], h1[C], w[C];
+#pragma unroll
+    for (int i = 0; i < C; ++i) {
+      const uint32_t q = tid + kPrepThreads * i;
+      h0[i] = ld(xr, 32 * q);
+      h1[i] = ld(xr, 32 * q + 16);
+      w[i] = ld(wr, 16 * q);
+    }
+    float4 sq[2];
+    ssq_load<2>(a.ssq_in + (int64_t)row * n_ss, l, n_ss, sq);
+    const float inv = rms_inv(wave_sum(ssq_lane_sum<2>(sq, l, n_ss)), K, a.eps);
+#pragma unroll
+    for (int i = 0; i < C; ++i) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const u32x4_t& h = j < 2 ? h0[i] : h1[i];
+        const int e = (j & 1) * 2;
+        v[i][j] = pack_bf16x2((__uint_as_float(h[e]) * inv) * bf16lo(w[i][j]),
+                              (__uint_as_float(h[e + 1]) * inv) * bf16hi(w[i][j]));
+      }
+      const int q = tid + kPrepThreads * i;
+      if (a.xn_out != nullptr && q < n_q)
+        *(u32x4_t*)(a.xn_out + (int64_t)row * a.x_stride + 8 * q) = v[i];
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < C; ++i) v[i] = ld(xr, 16 * (tid + kPrepThreads * i));
+    for (int q = tid + kPrepThreads * C; q < n_q; q += kPrepThreads) see(ld(xr, 16 * q));
+  }
+#pragma unroll
+  for (int i = 0; i < C; ++i) see(v[i]);
+  mx = umax_dpp<kDppXor1>(mx);
+  mx = umax_dpp<kDppXor2>(mx);
+  mx = umax_dpp<kDppHalfMirror>(mx);
+  mx = rows_max(umax_dpp<kDppRor8>(mx));
+  if (l == 0) smx[wave] = mx;
+  __syncthreads();
+  mx = pk_max_u16(pk_max_u16(smx[0], smx[1]), pk_max_u16(smx[2], smx[3]));
+  // exponent field of the row's largest entry; a row with an infinity or a NaN is left
+  // unscaled (its sums carry the NaN into every output of the row)
+  const int ex = (int)max(mx >> 16, mx & 0xFFFFu) >> 7;
+  const int sh = ex == 255 ? 0 : min(kPqXTop - max(ex, 1), 127);
+  const float sc = exp2i(sh), ss = exp2i(sh - kPqSum);
+  if (tid == 0) o.xshift[row] = sh;
+  const int r16 = row & 15, swz = (r16 >> 1) & 3;
+  u32x4_t* xt = o.xt + (size_t)(row >> 4) * (a.k_t * 8 + n_ch * 2) * 64 + r16 * 4;
+  u32x4_t* sm = xt + (size_t)a.k_t * 8 * 64;
+  for (int i0 = 0; i0 * 8 * kPrepThreads < K; i0 += C) {
+    if (i0 > 0) __syncthreads();                // the sums of the section before are read
+#pragma unroll
+    for (int i = 0; i < C; ++i) {
+      const int q = tid + kPrepThreads * (i0 + i);
+      u32x4_t w = v[i];
+      if (!NORM && i0 > 0) w = ld(xr, 16 * q);
+      u32x4_t h;
+      float s = 0.f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        // entries k, k + 2 of a group of four share a word, as the codes do (below)
+        const int e = j & 2;
+        const float x0 = (j & 1) ? bf16hi(w[e]) : bf16lo(w[e]);
+        const float x1 = (j & 1) ? bf16hi(w[e + 1]) : bf16lo(w[e + 1]);
+        h[j] = pk_f16(x0 * sc, x1 * sc);
+        s += x0 + x1;
+      }
+      if (q < n_q) xt[(size_t)(q >> 2) * 64 + ((q & 3) ^ swz)] = h;
+      s += dpp<kDppXor1>(s);
+      s += dpp<kDppXor2>(s);                    // the group's sum, in its four lanes
+      if ((l & 3) == 0) sg[64 * i + (tid >> 2)] = s;
+    }
+    __syncthreads();
+    // eight groups per thread (groups past K hold zeros, which the last chunk keeps)
+    const int g = 64 * i0 + 8 * tid;
+    if (tid < 8 * C && g < 32 * n_ch) {
+      u32x4_t hi, lo;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        uint32_t th, tl;
+        split2(sg[8 * tid + 2 * j] * ss, sg[8 * tid + 2 * j + 1] * ss, th, tl);
+        hi[j] = th;
+        lo[j] = tl;
+      }
+      u32x4_t* d = sm + (size_t)(g >> 5) * 2 * 64 + (((g >> 3) & 3) ^ swz);
+      d[0] = hi;
+      d[64] = lo;
+    }
+  }
+}
+
+// Weight tile-row: its columns' powers of two and u = m + 8 d in the minimum term's B operand
+// order. Four waves per tile-row, a chunk of 32 groups each: lane (c, s) holds columns
+// (c / 8) 16 + 2 (c % 8), + 1 at groups 8 s + j (K-tile 4 ch + s).
+__device__ __forceinline__ void prep_tile_row(const GemmArgs& a, const PqX& o, int tensor, int tr,
+                                              uint32_t* __restrict__ sm) {
+  constexpr int CACHED = 2;                     // chunks a wave keeps: K <= 8192
+  const int l = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = l & 15, s = l >> 4, n_tr = a.n_tr[0];
+  const int n_ch = (a.k_t + kPqChunkTiles - 1) / kPqChunkTiles;
+  const uint8_t* wr = a.w[tensor] + (size_t)tr * a.k_t * kQ4TileBytes +
+                      2 * ((c >> 3) * 16 + 2 * (c & 7));
+  uint32_t dv[CACHED][8], mv[CACHED][8], dm = 0, mm = 0;
+  auto fetch = [&](int ch, uint32_t (&d)[8], uint32_t (&m)[8]) {
+    const int kt = kPqChunkTiles * ch + s;
+    const uint8_t* t = wr + (size_t)min(kt, a.k_t - 1) * kQ4TileBytes;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      d[j] = *(const uint32_t*)(t + j * 64);
+      m[j] = *(const uint32_t*)(t + kMetaBytes + j * 64);
+    }
+  };
+  auto clip = [&](int ch, uint32_t (&d)[8], uint32_t (&m)[8]) {   // groups past K: zero
+    const bool in = kPqChunkTiles * ch + s < a.k_t;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      d[j] = in ? d[j] : 0u;
+      m[j] = in ? m[j] : 0u;
+    }
+  };
+  auto see = [&](const uint32_t (&d)[8], const uint32_t (&m)[8]) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      dm = pk_max_u16(dm, d[j] & 0x7FFF7FFFu);
+      mm = pk_max_u16(mm, m[j] & 0x7FFF7FFFu);
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < CACHED; ++i)
+    if (w + 4 * i < n_ch) fetch(w + 4 * i, dv[i], mv[i]);
+#pragma unroll
+  for (int i = 0; i < CACHED; ++i)
+    if (w + 4 * i < n_ch) {
+      clip(w + 4 * i, dv[i], mv[i]);
+      see(dv[i], mv[i]);
+    }
+  for (int ch = w + 4 * CACHED; ch < n_ch; ch += 4) {
+    uint32_t d[8], m[8];
+    fetch(ch, d, m);
+    clip(ch, d, m);
+    see(d, m);
+  }
+  dm = rows_max(dm);
+  mm = rows_max(mm);
+  if (l < 16) {
+    sm[w * 32 + l] = dm;
+    sm[w * 32 + 16 + l] = mm;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    dm = pk_max_u16(dm, sm[i * 32 + c]);
+    mm = pk_max_u16(mm, sm[i * 32 + 16 + c]);
+  }
+  int sh[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int ed = (int)((dm >> (16 * h + 7)) & 0xFF), em = (int)((mm >> (16 * h + 7)) & 0xFF);
+    // |u| <= |m| + 8 |d| < 2^(max(em, ed + 3) + 1 - 126)
+    sh[h] = ed < 255 && em < 255 ? min(kPqWTop - 1 - max(max(em, ed + 3), 1), 127 - kPqSum) : 0;
+  }
+  if (w == 0 && l < 16)
+    *(int2*)(o.wshift + ((size_t)tensor * n_tr + tr) * 32 + (c >> 3) * 16 + 2 * (c & 7)) =
+        make_int2(sh[0], sh[1]);
+  const float sd[2] = {exp2i(sh[0]), exp2i(sh[1])};
+  auto put = [&](int ch, const uint32_t (&d)[8], const uint32_t (&m)[8]) {
+    u32x4_t* du = o.u + ((((size_t)tensor * n_tr + tr) * n_ch + ch) * 4) * 64 + l;
+    uint2* ds = o.scale + (((size_t)tensor * n_tr + tr) * a.k_t + kPqChunkTiles * ch + s) * 128 + c;
+    u32x4_t hi[2], lo[2];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float u[2][2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const uint32_t dd = d[2 * j + e], mw = m[2 * j + e];
+        const float d0 = bf16lo(dd) * sd[0], d1 = bf16hi(dd) * sd[1];
+        const uint32_t dp = pk_f16(d0, d1), ap = pk_f16(d0 * kPqLow, d1 * kPqHigh);
+        const half2_t dh = as_h2(dp), ah = as_h2(ap);
+        if (kPqChunkTiles * ch + s < a.k_t) ds[(2 * j + e) * 16] = make_uint2(dp, ap);
+        u[0][e] = (bf16lo(mw) * sd[0] - fmaf(1024.f, (float)dh.x, (float)ah.x)) * (1 << kPqSum);
+        u[1][e] = (bf16hi(mw) * sd[1] - fmaf(64.f, (float)dh.y, (float)ah.y)) * (1 << kPqSum);
+      }
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        uint32_t th, tl;
+        split2(u[h][0], u[h][1], th, tl);
+        hi[h][j] = th;
+        lo[h][j] = tl;
+      }
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      du[h * 64] = hi[h];
+      du[(2 + h) * 64] = lo[h];
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < CACHED; ++i)
+    if (w + 4 * i < n_ch) put(w + 4 * i, dv[i], mv[i]);
+  for (int ch = w + 4 * CACHED; ch < n_ch; ch += 4) {
+    uint32_t d[8], m[8];
+    fetch(ch, d, m);
+    clip(ch, d, m);
+    put(ch, d, m);
+  }
+}
+
+// Workgroups [0, m_rows): a row of x each; the rest: a weight tile-row each, over both tensors
+// of [gate, up].
+template <bool NORM, int C>
+__global__ __launch_bounds__(kPrepThreads) void pq_prep_kernel(GemmArgs a, PqX o) {
+  __shared__ float sg[64 * C];
+  __shared__ uint32_t sm[128];
+  if ((int)blockIdx.x < a.m_rows) {
+    prep_row<NORM, C>(a, o, blockIdx.x, sg, sm);
+  } else {
+    const int t = blockIdx.x - a.m_rows, n = a.n_tr[0];
+    prep_tile_row(a, o, t / n, t % n, sm);
+  }
+}
+
+constexpr int vm_wait_pq(int n) {
+  return (n & 15) | (7 << 4) | (15 << 8) | ((n >> 4) & 3) << 14;
+}
+
+// The workgroup's waves meet; nothing is waited for (the reads of LDS in flight are of buffers
+// that are written again a whole step later at the earliest, after their use)
+__device__ __forceinline__ void step_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" ::: "memory");
+}
+
+// 16 bytes (4: one dword) per lane from uniform base + offset + lane offset to LDS at lds + off
+// + 16 (4) lane
+template <int OFF>
+__device__ __forceinline__ void ldl16(const void* base, uint32_t voff, uint32_t lds, int add) {
+  asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 offset:%4"
+               :: "s"(lds), "v"(voff), "s"(base), "i"(add - OFF), "i"(OFF) : "memory", "scc");
+}
+__device__ __forceinline__ void ldl16d(const void* base, uint32_t voff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               :: "s"(lds), "v"(voff), "s"(base) : "memory");
+}
+template <int OFF>
+__device__ __forceinline__ void ldl4(const void* base, uint32_t voff, uint32_t lds, int add) {
+  asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2 offset:%4"
+               :: "s"(lds), "v"(voff), "s"(base), "i"(add - OFF), "i"(OFF) : "memory", "scc");
+}
+
+// A workgroup of WN x WK waves takes 16 MT rows of X; wave (wn, wk) owns RT tile-rows (GATEUP:
+// the same tile-row of gate and of up) over K part wk, so nothing is shared between waves but
+// the staged x of their K part, and the parts are added through LDS at the end in part order.
+// x (a ring of RING 32-K steps) and the codes (a K-tile in two halves) go from memory to LDS by
+// direct loads, counted by hand, with no registers in between; the step's operands are built
+// beside its MFMAs, in 18 VALU instructions per tile-row, so the matrix cores set the pace.
+// What bounds it: two workgroups of the 128-row tile run the main loop at 1.76 PFLOP/s (an MFMA
+// loop with random operands and nothing else reaches 1.6-1.9 here, held by the power limit); the
+// pre-pass, the first loads and the outputs, all of a launch's at once, are not overlapped with
+// it. N x K, rows, before (scale after the MFMA, one FMA per output and group; below 512
+// workgroups the batched kernel) and now, pre-pass included: 8192 x 2560, 2048 rows 149 -> 95 us
+// (575 -> 905 TFLOP/s); 2560 x 8192, 333 rows 62 -> 37; [gate, up] 8192 x 2560, 500 rows 126 ->
+// 57 us, 2048 rows 477 -> 193. Error against 64 bits: 2048 rows, K = 2560 1.06e-6 -> 3.2e-7, 333
+// rows, K = 8192 3.1e-7 -> 1.2e-7.
+template <int OP, int MT, int RT, int WN, int WK, int RING, int OCC>
+__global__ __launch_bounds__(64 * WN * WK, OCC) void pq_kernel(GemmArgs a, PqX p) {
+  constexpr int TB = kQ4TileBytes;
+  constexpr int U = MT / WN;                   // x units (1 KB: one m-tile, one step) per wave
+  constexpr int XD = RING - 1;                 // steps of x in flight ahead of use
+  constexpr bool LOOK = RING == 8;             // x read from LDS ahead across the step boundary
+  constexpr int WL = 4 * RT;                   // direct loads of half a weight tile
+  static_assert(MT % WN == 0, "every wave stages as many m-tiles");
+  static_assert(8 % RING == 0, "a step's ring slot is known at compile time");
+  static_assert(OP == GOP_PLAIN || RT == 2, "gate and up");
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+
+  const int tid = threadIdx.x, l = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wn = wave % WN, wk = wave / WN;
+  const int c = l & 15, s = l >> 4;
+  const int n_tr = a.n_tr[0];
+  const int n_ch = (a.k_t + kPqChunkTiles - 1) / kPqChunkTiles;
+  const int unit_steps = a.k_t * 8 + n_ch * 2;  // per m-tile: the steps of x, then of the sums
+  const int unit = blockIdx.x * WN + wn;       // RT tile-rows, or one pair
+  const int m0 = blockIdx.y * 16 * MT;
+  // this wave's K part (a wave whose part ends early, or is empty, keeps the others' barriers)
+  const int kq = (a.k_t + WK - 1) / WK;
+  const int kt0 = min(wk * kq, a.k_t - 1), kt1 = min(a.k_t, wk * kq + kq);
+  const int nt = kt1 - wk * kq;                // its K-tiles (0 or less: none)
+  const uint8_t* wr[RT];
+  int tr[RT], col0[RT];
+#pragma unroll
+  for (int r = 0; r < RT; ++r) {
+    const int ten = OP == GOP_PLAIN ? 0 : r;
+    tr[r] = OP == GOP_PLAIN ? unit * RT + r : unit;
+    const int trc = min(tr[r], n_tr - 1);
+    wr[r] = a.w[ten] + (size_t)trc * a.k_t * TB;
+    col0[r] = ten * n_tr + trc;
+  }
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
+  const uint32_t xring = wk * RING * MT * 1024;                       // this part's x ring
+  constexpr int WBUF = RT * 2 * kPqHalf;       // one K-tile of the wave's tile-rows
+  const uint32_t wslot = WK * RING * MT * 1024 + wave * WBUF;
+  const uint32_t l16 = 16 * l, l4 = 4 * l;
+  const uint32_t xm0 = lds0 + xring + wn * 1024, wm0 = lds0 + wslot;
+  const uint8_t* xp[U];                        // m-tile wn + WN j at a multiple of four steps
+#pragma unroll
+  for (int j = 0; j < U; ++j)
+    xp[j] = (const uint8_t*)p.xt +
+            ((size_t)(blockIdx.y * MT + wn + WN * j) * unit_steps + kt0 * 8) * 1024;
+  // the part's chunks of the minimum term, and from its last x step to its sums
+  const int ch0 = kt0 / kPqChunkTiles, nc = nt > 0 ? (kt1 + kPqChunkTiles - 1) / kPqChunkTiles - ch0 : 0;
+  const int64_t to_sums = (int64_t)((a.k_t - kt1) * 8 + ch0 * 2 + 4) * 1024;
+  const uint8_t *up[RT], *sp[RT];              // its u, its scales
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+  {
+    up[r] = (const uint8_t*)(p.u + ((size_t)col0[r] * n_ch + ch0) * 4 * 64);
+    sp[r] = (const uint8_t*)(p.scale + (size_t)col0[r] * a.k_t * 128);
+  }
+
+  // x of a step, `ks` (mod 8) its place in its K-tile; the part's sums follow its last K-tile,
+  // and loads past them read the next bytes of the workspace, never used
+  auto x_load = [&](auto ksc, bool last) {
+    constexpr int ks = decltype(ksc)::value;
+    if constexpr ((ks & 3) == 0) {
+      const int64_t go = ks == 0 && last ? to_sums : 4096;
+#pragma unroll
+      for (int j = 0; j < U; ++j) xp[j] += go;
+    }
+#pragma unroll
+    for (int j = 0; j < U; ++j)
+      ldl16<(ks & 3) * 1024>(xp[j], l16, xm0, ((ks % RING) * MT + WN * j) * 1024);
+  };
+  // half of the part's K-tile t: 128 K of codes and their scales; after the last tile, the high (low) terms of the part's first chunk of u in their place, in as many
+  // loads
+  auto w_load = [&](int t, auto halfc) {
+    constexpr int half = decltype(halfc)::value;
+    const bool more = t < nt;
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      const uint8_t* w = wr[r] + (size_t)(kt0 + t) * TB;
+      const uint8_t* u = up[r] + half * 2048;
+      const int d = (r * 2 + half) * kPqHalf;
+      ldl16<0>(more ? w + 1024 + half * 1024 : u, l16, wm0, d);
+      ldl16<0>(more ? w + 3072 + half * 1024 : u + 1024, l16, wm0, d + 1024);
+      const uint8_t* q = more ? sp[r] + (size_t)(kt0 + t) * 1024 + half * 512 : u;
+      ldl4<0>(q, l4, wm0, d + 2048);
+      ldl4<256>(q, l4, wm0, d + 2304);
+    }
+  };
+#pragma unroll
+  for (int j = 0; j < U; ++j) xp[j] -= 4096;
+  x_load(std::integral_constant<int, 0>{}, false);
+  w_load(0, std::integral_constant<int, 0>{});
+  w_load(0, std::integral_constant<int, 1>{});
+  static_for<1, XD>([&](auto i) { x_load(i, false); });
+
+  f32x4_t acc[RT][MT][2];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) acc[r][mt][0] = acc[r][mt][1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  // Short accumulation chains where the registers allow: a K-tile's sum starts from zero and is
+  // added to the total on the VALU (the matrix cores' own accumulation rounds more coarsely: K =
+  // 8192 in one chain is 5.9e-7 off the 64-bit result, in tiles 1.2e-7 .. 1.6e-7; the kernel of
+  // this shape before, 1.9e-6)
+  constexpr bool FLUSH = MT * RT <= 8;
+  f32x4_t prt[FLUSH ? RT : 1][FLUSH ? MT : 1][2];
+  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+  int shw[RT][2];                              // the columns' powers of two
+#pragma unroll
+  for (int r = 0; r < RT; ++r) {
+    const int2 v = *(const int2*)(p.wshift + (size_t)col0[r] * 32 + (c >> 3) * 16 + 2 * (c & 7));
+    shw[r][0] = v.x;
+    shw[r][1] = v.y;
+  }
+  // ---- operands: the transposing LDS read gives lane (c, s) the 8 code bytes of row pair
+  // c % 8 of row-block c / 8 at k = 8 s ..; low nibbles are the even row, high the odd one
+  const uint8_t* const trp = lds + wslot + (c & 1) * 1024 + (8 * s + (c >> 1)) * 8;
+  const uint8_t* const scp = lds + wslot + 2048 + 8 * c;
+  struct Raw {
+    i32x2_t cb;
+    uint2 sc;                                  // fp16 (d even, d odd), (A even, A odd)
+  } raw[2][RT];                                // of steps of either parity
+  auto read_raw = [&](int kb) {
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      const int b = (r * 2 + (kb >> 2)) * kPqHalf;
+      raw[kb & 1][r].cb = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
+          (lds_i32x2_t*)(trp + b + (kb & 3) * 256));
+      raw[kb & 1][r].sc = *(const uint2*)(scp + b + (kb & 3) * 128);
+    }
+  };
+  // The operands of a step, in 8 RT half pieces: the first half of a piece takes the low and the
+  // high nibbles of two code bytes (bytes 0 and 2, or 1 and 3, of word h) to fp16 B + c, the
+  // second multiplies and adds.
+  u32x4_t ops[2][RT][2];
+  uint32_t msk_l, msk_h, exp_l, exp_h, tE = 0, tO = 0;
+  asm("v_mov_b32 %0, 0x000f000f" : "=v"(msk_l));
+  asm("v_mov_b32 %0, 0x00f000f0" : "=v"(msk_h));
+  asm("s_mov_b32 %0, 0x64006400" : "=s"(exp_l));
+  asm("s_mov_b32 %0, 0x54005400" : "=s"(exp_h));
+  auto half_piece = [&](int b, int i) {        // into ops[b] from raw[b]
+    const int r = i >> 3, h = (i >> 2) & 1, q = (i >> 1) & 1;
+    if ((i & 1) == 0) {
+      const uint32_t w = (h ? (uint32_t)raw[b][r].cb.y : (uint32_t)raw[b][r].cb.x) >> (8 * q);
+      tE = (w & msk_l) | exp_l;
+      tO = (w & msk_h) | exp_h;
+    } else {
+      const half2_t d = as_h2(raw[b][r].sc.x), A = as_h2(raw[b][r].sc.y);
+      const half2_t dE = {d.x, d.x}, dO = {d.y, d.y}, aE = {A.x, A.x}, aO = {A.y, A.y};
+      ops[b][r][0][2 * h + q] = h2_bits(__builtin_elementwise_fma(as_h2(tE), dE, aE));
+      ops[b][r][1][2 * h + q] = h2_bits(__builtin_elementwise_fma(as_h2(tO), dO, aO));
+    }
+  };
+
+  __builtin_amdgcn_s_waitcnt(vm_wait_pq(0));
+  __syncthreads();
+  read_raw(0);
+  read_raw(1);
+#pragma unroll
+  for (int i = 0; i < 8 * RT; ++i) half_piece(0, i);
+  // x fragments are read from LDS D m-tiles ahead of their use (LOOK: across the step boundary
+  // too) and a step's operand data two steps ahead
+  constexpr int D = MT < 3 ? MT : 3;
+  u32x4_t xa[4];
+  const uint8_t* const xl = lds + xring + c * 64 + ((s ^ (c >> 1)) & 3) * 16;
+  if constexpr (LOOK) {
+#pragma unroll
+    for (int f = 0; f < D; ++f) xa[f] = *(const u32x4_t*)(xl + f * 1024);
+  }
+
+  // ---- main loop over the part's K-tiles
+  for (int t = 0; t < nt; ++t) {
+    static_for<0, 8>([&](auto kbc) {
+      constexpr int kb = decltype(kbc)::value;
+      constexpr int cur = kb & 1, nxt = cur ^ 1;
+      constexpr int cs = (kb % RING) * MT * 1024, ns = ((kb + 1) % RING) * MT * 1024;
+      if constexpr (!LOOK) {
+#pragma unroll
+        for (int f = 0; f < D; ++f) xa[(kb * MT + f) & 3] = *(const u32x4_t*)(xl + cs + f * 1024);
+      }
+      read_raw((kb + 2) & 7);
+      x_load(std::integral_constant<int, (kb + XD) & 7>{}, t == nt - 1);
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        if (mt + D < MT) xa[(kb * MT + mt + D) & 3] = *(const u32x4_t*)(xl + cs + (mt + D) * 1024);
+        else if (LOOK) xa[(kb * MT + mt + D) & 3] = *(const u32x4_t*)(xl + ns + (mt + D - MT) * 1024);
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const u32x4_t& x = xa[(kb * MT + mt) & 3];
+            if constexpr (!FLUSH) acc[r][mt][h] = mfma_f16(x, ops[cur][r][h], acc[r][mt][h]);
+            else prt[r][mt][h] = mfma_f16(x, ops[cur][r][h], kb == 0 ? zero : prt[r][mt][h]);
+            // one MFMA, then the part of the operand build that fits beside it: a wave issues in
+            // order, so MFMAs back to back would hold the build up until the last has started
+            const int n = (mt * RT + r) * 2 + h;
+#pragma unroll
+            for (int i = n * 4 / MT; i < (n + 1) * 4 / MT; ++i) half_piece(nxt, i);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        // the half tile whose last operand data this step's build has used is loaded again
+        if constexpr (kb == 2) {
+          if (mt == 0) w_load(t + 1, std::integral_constant<int, 0>{});
+        } else if constexpr (kb == 6) {
+          if (mt == 0) w_load(t + 1, std::integral_constant<int, 1>{});
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if constexpr (FLUSH && kb == 7) {
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) acc[r][mt][h][e] += prt[r][mt][h][e];
+      }
+      // x of the steps that the next step reads (its own, and with LOOK the one after it) has
+      // landed when at most the loads issued after it are in flight: x of the LATE steps last
+      // issued, and the half tiles loaded since; the half tile whose operand data the next step
+      // begins to read (kb 2, 6) when x of three steps is all that follows it
+      constexpr int LATE = LOOK ? XD - 2 : XD - 1, AGO = (kb - 2) & 3;
+      constexpr int X = LATE * U + ((AGO <= LATE) + (AGO + 4 <= LATE)) * WL;
+      constexpr int N = AGO == 3 && X > 3 * U ? 3 * U : X;
+      __builtin_amdgcn_s_waitcnt(vm_wait_pq(N));
+      step_barrier();
+    });
+  }
+  for (int t = nt > 0 ? nt : 0; t < kq; ++t)   // a shorter part: the others' barriers
+#pragma unroll
+    for (int kb = 0; kb < 8; ++kb) step_barrier();
+
+  // ---- the minimum term, in the same scale: A holds the S terms (ring steps after the last of
+  // x), B u of the lane's two columns at groups 32 ch + 8 s + j (K-tile 4 ch + s; zero outside
+  // the part). The next chunk's are loaded while this one's are used.
+  const int nc_all = WK == 1 ? nc : (kq + 2 * kPqChunkTiles - 2) / kPqChunkTiles;   // any part's, at most
+  const uint8_t* sx[U];
+#pragma unroll
+  for (int j = 0; j < U; ++j)
+    sx[j] = (const uint8_t*)p.xt + ((size_t)(blockIdx.y * MT + wn + WN * j) * unit_steps +
+                                    a.k_t * 8 + ch0 * 2) * 1024;
+  for (int i = 0; i < nc_all; ++i) {
+    __builtin_amdgcn_s_waitcnt(vm_wait_pq(0));
+    __syncthreads();
+    if (i >= nc) continue;
+    const int kt = kPqChunkTiles * (ch0 + i) + s;
+    const bool in = WK == 1 || (kt >= kt0 && kt < kt1);
+    u32x4_t uu[RT][2][2];                      // [hi, lo][even, odd column]
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const u32x4_t v = *(const u32x4_t*)(lds + wslot + (r * 2 + (e >> 1)) * kPqHalf +
+                                            (e & 1) * 1024 + l16);
+        uu[r][e >> 1][e & 1] = in ? v : u32x4_t{0, 0, 0, 0};
+      }
+    if (i + 1 < nc) {
+#pragma unroll
+      for (int e = 2; e < 4; ++e)
+#pragma unroll
+        for (int j = 0; j < U; ++j)
+          ldl16d(sx[j] + (size_t)(2 * i + e) * 1024, l16,
+                 xm0 + (((2 * i + e) & (RING - 1)) * MT + WN * j) * 1024);
+    }
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {              // the sums' high terms, then the low ones
+      const uint8_t* xs = xl + ((2 * i + e) & (RING - 1)) * MT * 1024;
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        const u32x4_t x = *(const u32x4_t*)(xs + mt * 1024);
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            f32x4_t& t = FLUSH ? prt[FLUSH ? r : 0][FLUSH ? mt : 0][h] : acc[r][mt][h];
+            if (e == 0) t = mfma_f16(x, uu[r][1][h], FLUSH && i == 0 ? zero : t);
+            t = mfma_f16(x, uu[r][0][h], t);
+          }
+      }
+      if (e == 0 && i + 1 < nc) {              // u is in registers: its slots are free
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+            ldl16d(up[r] + (size_t)(i + 1) * 4096 + k * 1024, l16,
+                   wm0 + (r * 2 + (k >> 1)) * kPqHalf + (k & 1) * 1024);
+      }
+    }
+  }
+  if constexpr (FLUSH) {
+    if (nc > 0) {
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[r][mt][h][e] += prt[r][mt][h][e];
+    }
+  }
+  __builtin_amdgcn_s_waitcnt(vm_wait_pq(0));   // the loads past the end have landed
+  __syncthreads();
+
+  // ---- to the true scale: rows 4 s + e of each m-tile
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    const int4 xs = *(const int4*)(p.xshift + m0 + 16 * mt + 4 * s);
+    const int xsh[4] = {xs.x, xs.y, xs.z, xs.w};
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          acc[r][mt][h][e] = ldexpf(acc[r][mt][h][e], -(shw[r][h] + xsh[e]));
+  }
+
+  // ---- the K parts, added in part order by part 0's wave
+  if constexpr (WK > 1) {
+    constexpr int REC = RT * MT * 2;           // f32x4 per lane
+    f32x4_t* red = (f32x4_t*)lds;
+    if (wk > 0) {
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+            red[(((wk - 1) * WN + wn) * REC + (r * MT + mt) * 2 + h) * 64 + l] = acc[r][mt][h];
+    }
+    __syncthreads();
+    if (wk > 0) return;
+#pragma unroll 1
+    for (int k = 1; k < WK; ++k)
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const f32x4_t v = red[(((k - 1) * WN + wn) * REC + (r * MT + mt) * 2 + h) * 64 + l];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[r][mt][h][e] += v[e];
+          }
+  }
+
+  // ---- outputs: the lane's two columns are adjacent, so the 16 lanes of a row write 128
+  // contiguous bytes (64 of bf16)
+  const int col = (c >> 3) * 16 + 2 * (c & 7);
+  auto store = [&](auto fullc) {               // full: every row of the block is one of X
+    constexpr bool FULL = decltype(fullc)::value;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int m = m0 + 16 * mt + 4 * s + e;
+        const bool row_live = FULL || m < a.m_rows;
+        if constexpr (OP == GOP_PLAIN) {
+#pragma unroll
+          for (int r = 0; r < RT; ++r) {
+            if (tr[r] >= n_tr) continue;
+            float2 v = make_float2(acc[r][mt][0][e], acc[r][mt][1][e]);
+            const int64_t o = (int64_t)m * a.y_stride + (int64_t)tr[r] * 32 + col;
+            if (row_live) {
+              if (a.residual != nullptr) {
+                const float2 rr = *(const float2*)(a.residual + o);
+                v.x += rr.x;
+                v.y += rr.y;
+              }
+              if (a.y != nullptr) *(float2*)(a.y + o) = v;
+            }
+            if (a.ssq_out != nullptr) {        // per 16-row block: 8 lanes
+              float q = fmaf(v.x, v.x, v.y * v.y);
+              q += dpp<kDppXor1>(q);
+              q += dpp<kDppXor2>(q);
+              q += dpp<kDppHalfMirror>(q);
+              if (row_live && (c & 7) == 0)
+                a.ssq_out[(int64_t)m * n_tr * 2 + tr[r] * 2 + (c >> 3)] = q;
+            }
+          }
+        } else {
+          if (tr[0] >= n_tr || !row_live) continue;
+          const int64_t N = (int64_t)n_tr * 32, n = (int64_t)tr[0] * 32 + col;
+          const float g0 = acc[0][mt][0][e], g1 = acc[0][mt][1][e];
+          const float u0 = acc[1][mt][0][e], u1 = acc[1][mt][1][e];
+          *(uint32_t*)(a.h_out + (int64_t)m * a.h_stride + n) =
+              pack_bf16x2(swiglu(round_bf16_op(g0), round_bf16_op(u0)),
+                          swiglu(round_bf16_op(g1), round_bf16_op(u1)));
+          if (a.raw_out != nullptr) {
+            *(float2*)(a.raw_out + (int64_t)m * 2 * N + n) = make_float2(g0, g1);
+            *(float2*)(a.raw_out + (int64_t)m * 2 * N + N + n) = make_float2(u0, u1);
+          }
+        }
+      }
+  };
+  if (m0 + 16 * MT <= a.m_rows) store(std::true_type{});
+  else store(std::false_type{});
+}
+
+// ---------------------------------------------------------------- host side
+
+size_t pq_align(size_t b) { return (b + 255) & ~(size_t)255; }
+int pq_chunks(int k_t) { return (k_t + kPqChunkTiles - 1) / kPqChunkTiles; }
+int pq_mtiles(int m_rows) { return (m_rows + 127) / 128 * 8; }   // whole 128-row blocks
+
+// The pre-pass's buffers in a workspace (nullptr: their total size)
+size_t pq_layout(void* ws, int tensors, int n_tr, int k_t, int m_rows, PqX* x) {
+  const size_t mt = pq_mtiles(m_rows), ch = pq_chunks(k_t), tr = (size_t)tensors * n_tr;
+  size_t off = 0;
+  auto take = [&](size_t bytes) {
+    uint8_t* b = (uint8_t*)ws + off;
+    off += pq_align(bytes);
+    return b;
+  };
+  x->xt = (u32x4_t*)take(mt * (k_t * 8 + ch * 2) * 1024 + kPqSlack);
+  x->u = (u32x4_t*)take(tr * ch * 4 * 1024);
+  x->scale = (uint2*)take(tr * k_t * 1024);
+  x->xshift = (int*)take(mt * 16 * 4);
+  x->wshift = (int*)take(tr * 32 * 4);
+  return off;
+}
+
+template <int OP, int MT, int RT, int WN, int WK, int RING, int OCC>
+void pq_go(const GemmArgs& a, const PqX& x, hipStream_t st) {
+  constexpr int ring = WK * RING * MT * 1024 + WN * WK * RT * 2 * kPqHalf;
+  constexpr int red = (WK - 1) * WN * RT * MT * 2 * 1024;
+  constexpr int lds = ring > red ? ring : red;
+  static_assert(lds <= 160 * 1024);
+  const int units = OP == GOP_PLAIN ? (a.n_tr[0] + RT - 1) / RT : a.n_tr[0];
+  const dim3 grid((unsigned)((units + WN - 1) / WN), (unsigned)((a.m_rows + 16 * MT - 1) / (16 * MT)));
+  hipLaunchKernelGGL((pq_kernel<OP, MT, RT, WN, WK, RING, OCC>), grid, dim3(64 * WN * WK), lds, st, a, x);
+}
+
+}  // namespace
+
+size_t pq_ws_bytes(int op, int n_tile_rows, int k_t, int m_rows) {
+  PqX x;
+  return pq_layout(nullptr, op == GOP_GATEUP ? 2 : 1, n_tile_rows, k_t, m_rows, &x);
+}
+
+bool pq_use(int kind, int op, const GemmArgs& a) {
+  if (kind != Q4NX_KIND_Q4 || op == GOP_QKV || a.m_rows < kPqRows || a.argmax_keys != nullptr)
+    return false;
+  // [gate, up] stores pairs of bf16 outputs as one word
+  return op == GOP_PLAIN || (Q4NX_ALIGNED(a.h_out, 4) && a.h_stride % 2 == 0);
+}
+
+void pq_launch(int op, const GemmArgs& a, void* ws, hipStream_t st) {
+  PqX x;
+  const int tensors = op == GOP_GATEUP ? 2 : 1;
+  pq_layout(ws, tensors, a.n_tr[0], a.k_t, a.m_rows, &x);
+  const dim3 pg((unsigned)(a.m_rows + a.n_tr[0] * tensors)), pb(kPrepThreads);
+  if (a.norm_w != nullptr) {
+    if (a.k_t <= 16) hipLaunchKernelGGL((pq_prep_kernel<true, 2>), pg, pb, 0, st, a, x);
+    else hipLaunchKernelGGL((pq_prep_kernel<true, 4>), pg, pb, 0, st, a, x);
+  } else {
+    if (a.k_t <= 16) hipLaunchKernelGGL((pq_prep_kernel<false, 2>), pg, pb, 0, st, a, x);
+    else hipLaunchKernelGGL((pq_prep_kernel<false, 4>), pg, pb, 0, st, a, x);
+  }
+  // Tile by the workgroups it gives a chip of 256 CUs: the largest that fills it. Measured over
+  // K x N of 512 x 1024 to 12288 x 4096 and 65 to 3000 rows; us at the side of each line where
+  // the two are closest (N x K, rows):
+  const auto wgs = [&](int rows, int trs) {
+    return ((a.m_rows + rows - 1) / rows) * ((a.n_tr[0] + trs - 1) / trs);
+  };
+  if (op == GOP_PLAIN) {
+    // 128 rows x 8 tile-rows against 64 x 4: 8192 x 2560, 1000 rows (256) 57 / 61, 640 rows
+    // (160) 53 / 47; a short K does not repay the larger block's epilogue (6144 x 1024, 1500
+    // rows (288) 44 / 38), and with fewer rows than the block has the others are as fast and add
+    // up in shorter chains (the error against 64 bits 1.2e-7, not 2.8e-7)
+    const int w0 = a.m_rows < 128 ? 0 : wgs(128, 8);
+    if (w0 >= 512 || (w0 >= 240 && a.k_t >= 8)) pq_go<GOP_PLAIN, 8, 2, 4, 1, 4, 2>(a, x, st);
+    // 64 x 4 against 64 x 2 with K in two parts: 2560 x 8192, 1500 rows (480) 90 / 99, 1000 rows
+    // (320) 80 / 72
+    else if (wgs(64, 4) >= 440) pq_go<GOP_PLAIN, 4, 1, 4, 1, 8, 2>(a, x, st);
+    // two parts against four: 2560 x 8192, 400 rows (280) 50 / 56, 256 rows (160) 40 / 36
+    else if (wgs(64, 2) > 256) pq_go<GOP_PLAIN, 4, 1, 2, 2, 4, 2>(a, x, st);
+    // 64 x 2 in four parts against 32 x 2: 2560 x 8192, 256 rows (160) 36 / 48, 192 rows (120)
+    // 35 / 31
+    else if (wgs(64, 2) >= 160) pq_go<GOP_PLAIN, 4, 1, 2, 4, 4, 2>(a, x, st);
+    // 32 x 2 in four parts against 32 x 1 in eight: 2560 x 2560, 128 rows (320) 16 / 22, 96 rows
+    // (240) 16 / 14
+    else if (wgs(32, 1) > 256) pq_go<GOP_PLAIN, 2, 1, 2, 4, 8, 2>(a, x, st);
+    else pq_go<GOP_PLAIN, 2, 1, 1, 8, 4, 2>(a, x, st);
+  } else {
+    // 128 rows x 4 pairs against 64 x 2 in two parts: 8192 x 2560, 400 rows (256) 55 / 64, 192
+    // rows (128) 51 / 39
+    if (wgs(128, 4) >= 192) pq_go<GOP_GATEUP, 8, 2, 4, 1, 4, 2>(a, x, st);
+    // 64 x 2 against 32 x 2 in four parts: 2560 x 8192, 256 rows (160) 58 / 70, 192 rows (120)
+    // 58 / 44
+    else if (wgs(64, 2) >= 160) pq_go<GOP_GATEUP, 4, 2, 2, 2, 4, 2>(a, x, st);
+    // 32 x 2 against 32 x 1 in eight parts: 2560 x 2560, 128 rows (320) 23 / 28, 96 rows (240)
+    // 22 / 18
+    else if (wgs(32, 1) > 256) pq_go<GOP_GATEUP, 2, 2, 2, 4, 4, 2>(a, x, st);
+    else pq_go<GOP_GATEUP, 2, 2, 1, 8, 4, 2>(a, x, st);
+  }
+}
+
+}  // namespace q4nx

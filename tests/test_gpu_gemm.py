@@ -307,3 +307,123 @@ def test_gemm_prefill_without_workspace(dev):
         _lib.call("q4nx_gemm", 4, w.data_ptr(), n // 32, k // 256, xd.data_ptr(), k, m,
                   y.data_ptr(), n, None, wp, wn, None, ops._stream())
         _check_rows(y.cpu().numpy(), ref)
+
+
+# ------------------------------------------------------------------ q4 prompt blocks on fp16 operands
+# From 65 rows q4 launches take the fp16-operand kernel, whose workgroup tile follows from the
+# workgroups each size would give: 128 rows x 8 tile-rows, 64 x 4, 64 x 2 with K in two or four
+# parts, 32 x 2 in four, 32 x 1 in eight. Its operands d (B + c) + A are exact and its sums fp32,
+# so every row is held to the GEMV bar; minima unrelated to the scales (every other case here has
+# m = -8 d) make the minimum term carry a full share of the result.
+
+def _free_minima(raw, rng):
+    m = synth.f32_to_bf16_bits((rng.standard_normal((raw.shape[0], 256)) * 0.1).astype(np.float32))
+    raw = raw.copy()
+    raw[:, 512:1024] = m.view(np.uint8).reshape(raw.shape[0], 512)
+    return raw
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (65, 32, 256),        # 32 x 1: one tile-row, seven of eight K parts empty
+    (80, 544, 2816),      # 32 x 1: 11 K-tiles over eight parts of two, the last ones empty
+    (129, 2080, 768),     # 32 x 2 (325 workgroups of 32 x 1): a last workgroup with one tile-row
+    (257, 2080, 1280),    # 64 x 2 in four parts: five K-tiles in parts of two, one empty
+    (449, 2592, 768),     # 64 x 2 in two parts, ragged rows
+    (1500, 2464, 256),    # 64 x 4: one K-tile, fewer steps than the ring holds ahead
+    (3900, 2016, 2048),   # 128 x 8, ragged rows, a last workgroup of seven tile-rows
+    (130, 128, 8448),     # rows longer than the pre-pass keeps in registers
+])
+def test_gemm_fp16_operands_parity(dev, m, n, k):
+    raw, rng = _tiles("q4", n, k, 51 + m)
+    raw = _free_minima(raw, rng)
+    x = synth.random_bf16(rng, (m, k))
+    res = rng.standard_normal((m, n)).astype(np.float32)
+    w, xd = _dev_u8(raw, dev), _dev_bf16(x, dev)
+    y = ops.gemm(w, "q4", xd, n // 32, k // 256, residual=torch.from_numpy(res).to(dev))
+    rows = np.unique(np.concatenate([np.arange(0, m, max(1, m // 48)), [m - 1]]))
+    ref = qo.gemv(raw, "q4", x[rows], n // 32, k // 256, acc=np.float64) + res[rows]
+    _check_rows(y.cpu().numpy()[rows], ref)
+    ssq = torch.full((m, n // 16), float("nan"), device=dev)
+    y2 = ops.gemv_ex(w, "q4", xd, n // 32, k // 256, residual=torch.from_numpy(res).to(dev),
+                     ssq_out=ssq)
+    assert torch.equal(y, y2)
+    want = y2.double().view(m, -1, 16).square().sum(-1)
+    # 16 squares added in fp32: 16 roundings of 2^-24 at most
+    assert ((ssq.double() - want).abs() <= 16 * 2.0 ** -24 * want).all()
+
+
+def test_gemm_fp16_operands_range(dev):
+    """Scales over the whole bf16 exponent range between a tile's columns, zero scales and
+    minima, all-zero rows and rows of very different size, exactly as the 64-bit result has
+    them; an infinity or a NaN in a row of x reaches every output of that row and no other."""
+    m, n, k = 72, 96, 512
+    raw, rng = _tiles("q4", n, k, 61)
+    raw = _free_minima(raw, rng)
+    e = (10.0 ** rng.uniform(-25, 25, (1, 8, 32))).astype(np.float32)   # one size per column
+    for p in (0, 512):
+        v = qo.bf16_to_f32(raw[:, p:p + 512].copy().view(np.uint16)).reshape(-1, 8, 32) * e[:, :1]
+        v[:, :, 5] = 0.0
+        raw[:, p:p + 512] = synth.f32_to_bf16_bits(v.reshape(-1, 256).astype(np.float32)).view(
+            np.uint8).reshape(-1, 512)
+    xf = rng.standard_normal((m, k)).astype(np.float32)
+    xf *= (10.0 ** rng.uniform(-6, 6, (m, 1))).astype(np.float32)
+    xf[3] = 0.0
+    x = qo.bf16_round(xf)
+    w, xd = _dev_u8(raw, dev), _dev_bf16(x, dev)
+    y = ops.gemm(w, "q4", xd, n // 32, k // 256).cpu().numpy().astype(np.float64)
+    ref = qo.gemv(raw, "q4", x, n // 32, k // 256, acc=np.float64)
+    assert (y[3] == 0).all() and (y[:, 5] == 0).all() and (y[:, 37] == 0).all()
+    # columns differ by up to 2^166: each output against its own terms' size, K roundings of
+    # 2^-24 at most
+    wabs = np.abs(qo.dequant_matrix(raw, "q4", n // 32, k // 256).astype(np.float64))
+    size = np.abs(qo.bf16_to_f32(x).astype(np.float64)) @ (wabs.T + 16 * wabs.max(1))
+    assert (np.abs(y - ref) <= k * 2.0 ** -24 * size).all()
+    bad = xd.clone()
+    bad[7, 100], bad[20, 3], bad[64, 511] = float("inf"), float("nan"), float("-inf")
+    yb = ops.gemm(w, "q4", bad, n // 32, k // 256).cpu().numpy()
+    hit = np.zeros(m, bool)
+    hit[[7, 20, 64]] = True
+    assert not np.isfinite(yb[hit]).any()
+    assert np.array_equal(yb[~hit].view(np.uint32), y[~hit].astype(np.float32).view(np.uint32))
+
+
+@pytest.mark.parametrize("batch,n,k,norm", [
+    (65, 96, 256, False),      # 32 x 1 pairs
+    (200, 1312, 768, True),    # 32 x 2 pairs (287 workgroups of 32 x 1)
+    (300, 2080, 2816, True),   # 64 x 2 pairs in two parts
+    (1300, 2464, 512, True),   # 128 x 4 pairs, ragged both ways
+])
+def test_gate_up_fp16_operands(dev, batch, n, k, norm):
+    """[RMSNorm, gate, up, SwiGLU] on the fp16-operand kernel: the fp32 gate and up values at the
+    GEMV bar on the prologue's own bf16 output, h their SwiGLU's rounding."""
+    rng = np.random.default_rng(71 + batch)
+    g = _free_minima(synth.q4_tiles(rng, n, k).reshape(-1, qo.Q4_TILE_BYTES), rng)
+    u = synth.q4_tiles(rng, n, k).reshape(-1, qo.Q4_TILE_BYTES)
+    xn = torch.empty((batch, k), dtype=torch.bfloat16, device=dev)
+    raw_out = torch.empty((batch, 2 * n), dtype=torch.float32, device=dev)
+    kw = {}
+    if norm:
+        h = (rng.standard_normal((batch, k)) * 5).astype(np.float32)
+        x = torch.from_numpy(h).to(dev)
+        kw = dict(norm_w=_dev_bf16(synth.random_bf16(rng, k), dev), xn_out=xn,
+                  ssq_in=x.view(batch, -1, 16).square().sum(-1).contiguous())
+    else:
+        x = _dev_bf16(synth.random_bf16(rng, (batch, k)), dev)
+        xn.copy_(x)
+    h_out = ops.gate_up_swiglu(_dev_u8(g, dev), _dev_u8(u, dev), n // 32, k // 256, x,
+                               raw_out=raw_out, **kw)
+    if norm:   # the prologue against the batched kernel's: the same bits
+        xn2 = torch.empty_like(xn)
+        ops.gate_up_swiglu(_dev_u8(g, dev), _dev_u8(u, dev), n // 32, k // 256, x,
+                           policy=ops.Policy(gemm_ksplit=1), **dict(kw, xn_out=xn2))
+        assert torch.equal(xn, xn2)
+    rows = np.unique(np.concatenate([np.arange(0, batch, max(1, batch // 32)), [batch - 1]]))
+    xb = xn.view(torch.int16).cpu().numpy().view(np.uint16)[rows]
+    got = raw_out.cpu().numpy()
+    _check_rows(got[rows, :n], qo.gemv(g, "q4", xb, n // 32, k // 256, acc=np.float64))
+    _check_rows(got[rows, n:], qo.gemv(u, "q4", xb, n // 32, k // 256, acc=np.float64))
+    narrow = lambda t: t.to(torch.bfloat16).double()
+    gv, uv = narrow(raw_out[:, :n]), narrow(raw_out[:, n:])
+    want = (gv / (1 + torch.exp(-gv)) * uv)
+    # one bf16 rounding (2^-9 of the value's binade) and the fp32 formula's own few ulps
+    assert ((h_out.double() - want).abs() <= want.abs() * (2.0 ** -8 + 2.0 ** -20) + 1e-38).all()
