@@ -666,3 +666,72 @@ def test_gqa_decode_random_shapes(dev, apath, case):
     assert not of[empty].any()                           # no positions: zeros
     if (~empty).any():
         assert_close(of[~empty], ref[~empty])
+
+
+# ------------------------------------------------------------------ 16-byte elementwise kernels
+# Aligned operands of whole 16-byte pieces take kernels with eight (embed: four) entries per
+# thread, others one entry per thread; the two agree on every shape both take.
+
+def _off(t):
+    """The same values one entry past an aligned address: the one-entry kernels."""
+    flat = torch.empty(t.numel() + 8, dtype=t.dtype, device=t.device)[1:1 + t.numel()]
+    return flat.view(t.shape).copy_(t)
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 8), (3, 264), (5, 2048), (2, 2056), (300, 2560),
+                                       (2, 8192), (2, 8200), (3, 2561)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_rmsnorm_wide_equals_narrow(dev, rows, cols, dtype):
+    g = torch.Generator(device=dev).manual_seed(rows * cols)
+    x = (torch.randn((rows, cols), device=dev, generator=g) * 3).to(dtype)
+    w = torch.randn(cols, device=dev, generator=g).to(torch.bfloat16)
+    y, yf = ops.rmsnorm(x, w, want_f32=True)
+    z, zf = ops.rmsnorm(_off(x), w, want_f32=True)
+    # the row's squares are added in another order: cols roundings of 2^-24 under a square root
+    assert ((yf - zf).abs() <= (cols + 8) * 2.0 ** -24 * zf.abs()).all()
+    assert torch.equal(y, yf.to(torch.bfloat16)) and torch.equal(z, zf.to(torch.bfloat16))
+    assert torch.equal(ops.rmsnorm(x, w), y)
+
+
+@pytest.mark.parametrize("b,h,d", [(1, 1, 16), (3, 5, 64), (257, 8, 64), (2, 3, 24), (40, 40, 64)])
+def test_rope_wide_equals_narrow(dev, b, h, d):
+    g = torch.Generator(device=dev).manual_seed(b * h)
+    x = torch.randn((b, h, d), device=dev, generator=g).to(torch.bfloat16)
+    pos = torch.randint(-1, 101, (b,), dtype=torch.int32, device=dev, generator=g)
+    tab = ops.rope_table(100, d)
+    y, yf = ops.rope(x, pos, tab, want_f32=True)
+    z, zf = ops.rope(_off(x), pos, tab, want_f32=True)
+    assert torch.equal(y.view(torch.int16), z.view(torch.int16))
+    assert torch.equal(yf.isnan(), zf.isnan()) and torch.equal(yf.nan_to_num(), zf.nan_to_num())
+    bad = (pos < 0) | (pos >= 100)
+    assert y[bad].isnan().all() and not y[~bad].isnan().any()
+
+
+@pytest.mark.parametrize("shape", [(1, 8), (3, 40), (1, 2050), (7, 8191), (300, 1032)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_swiglu_wide_equals_narrow(dev, shape, dtype):
+    g = torch.Generator(device=dev).manual_seed(shape[1])
+    a, u = ((torch.randn(shape, device=dev, generator=g) * 30).to(dtype) for _ in range(2))
+    a.view(-1)[:3] = torch.tensor([float("inf"), float("-inf"), float("nan")])
+    y, yf = ops.swiglu(a, u, want_f32=True)
+    z, zf = ops.swiglu(_off(a), u, want_f32=True)
+    assert torch.equal(y.nan_to_num(), z.nan_to_num()) and torch.equal(yf.nan_to_num(), zf.nan_to_num())
+    assert torch.equal(y.isnan(), z.isnan())
+
+
+@pytest.mark.parametrize("kind", ["q8", "q4", "bf16"])
+def test_embed_wide_equals_narrow(dev, kind):
+    rng = np.random.default_rng(29)
+    vocab, hid = 96, 768
+    if kind == "bf16":
+        table = bf16_dev(synth.random_bf16(rng, (vocab, hid)), dev)
+    else:
+        table = torch.from_numpy((synth.q8_tiles if kind == "q8" else synth.q4_tiles)(
+            rng, vocab, hid).reshape(-1)).to(dev)
+    toks = torch.arange(-1, vocab + 1, dtype=torch.int32, device=dev)
+    h = ops.embed(table, kind, toks, vocab, hid)
+    ss = torch.empty((toks.numel(), hid // 16), device=dev)
+    for other in (ops.embed(table, kind, toks, vocab, hid, ssq_out=ss),
+                  ops.embed(_off(table), kind, toks, vocab, hid)):
+        assert torch.equal(h[1:-1], other[1:-1])
+        assert other[[0, -1]].isnan().all() and h[[0, -1]].isnan().all()
