@@ -55,28 +55,18 @@ bool mfma_use(int kind, int rows, const Policy& P);
 size_t mfma_ws_bytes(int kind, int op, int n_units, int k_t, int m_rows, const Policy& P);
 // whether ws_bytes holds the normalised rows an RMSNorm prologue needs on this path
 bool mfma_norm_fits(int k_t, int m_rows, size_t ws_bytes);
-// The prefill kernel (gemm_pf.hip) takes plain q8 contractions from this many rows.
-constexpr int kPrefillRows = 128;
-// workspace bytes the prefill kernel keeps its per-group sums of x in (past the counters,
-// the split records and the normalised rows), or 0 when the shape does not take that kernel
-size_t pf_ws_bytes(int kind, int n_tile_rows, int k_t, int m_rows);
-// whether a launch of op `op` described by `a` has the prefill kernel's shape
-bool pf_use(int kind, int op, const GemmArgs& a);
-// launches `a` on the prefill kernel (whole K per workgroup, no split): the per-group sums
-// of x into `sums` (pf_ws_bytes of them, 256-byte aligned), then the contraction
-void pf_launch(const GemmArgs& a, void* sums, hipStream_t st);
-// The fp16-operand prompt-block kernel (gemm_pq.hip) takes q4 contractions past the batched
-// kernel's 64-row workgroups (80 rows, batched / here in us: 8192 x 2560 30 / 21, 2560 x 8192
-// 38 / 21, [gate, up] 43 / 31; at 64 rows 19 / 19, 22 / 20 and 28 / 27, most shapes the batched
-// kernel's).
+// The fp16-operand prompt-block kernel (gemm_pq.hip) takes contractions past the batched
+// kernel's 64-row workgroups (80 rows, batched / here in us: q4 8192 x 2560 30 / 21, 2560 x 8192
+// 38 / 21, [gate, up] 43 / 31; q8 2560 x 2560 20 / 14; at 64 rows q4 19 / 19, 22 / 20 and 28 /
+// 27, most shapes the batched kernel's).
 constexpr int kPqRows = 65;
 // workspace bytes it keeps the fp16 x, sums and column terms in (past the counters)
-size_t pq_ws_bytes(int op, int n_tile_rows, int k_t, int m_rows);
+size_t pq_ws_bytes(int kind, int op, int n_tile_rows, int k_t, int m_rows);
 // whether a launch of op `op` described by `a` takes that kernel
-bool pq_use(int kind, int op, const GemmArgs& a);
+bool pq_use(int op, const GemmArgs& a);
 // launches `a` on it (with its RMSNorm prologue, if any): the pre-pass over x into `ws`
 // (pq_ws_bytes of it, 256-byte aligned), then the contraction
-void pq_launch(int op, const GemmArgs& a, void* ws, hipStream_t st);
+void pq_launch(int kind, int op, const GemmArgs& a, void* ws, hipStream_t st);
 // launches `a` (all but the split-K fields filled in); returns Q4NX_OK or an error code
 int mfma_launch(int kind, int op, GemmArgs& a, int n_units, void* ws, size_t ws_bytes,
                 const Policy& P, hipStream_t st, const char* what);

@@ -674,12 +674,11 @@ bool mfma_use(int kind, int rows, const Policy& P) {
 }
 
 size_t mfma_ws_bytes(int kind, int op, int n_units, int k_t, int m_rows, const Policy& P) {
-  // room for the split-K records, for the normalised rows of an RMSNorm prologue and, for a
-  // plain prompt block, for the prefill kernel's per-group sums of x
+  // room for the split-K records and the normalised rows of an RMSNorm prologue or, for a prompt
+  // block, for what the fp16-operand kernel keeps
   const size_t split = split_part_bytes(plan_gemm(kind, op, n_units, k_t, m_rows, P));
-  const size_t pf = op == GOP_PLAIN ? pf_ws_bytes(kind, n_units, k_t, m_rows) : 0;
-  const size_t pq = kind == Q4NX_KIND_Q4 && op != GOP_QKV && m_rows >= kPqRows ? pq_ws_bytes(op, n_units, k_t, m_rows) : 0;
-  const size_t b = align256(split) + align256((size_t)m_rows * k_t * kTileK * 2) + pf;
+  const size_t pq = op != GOP_QKV && m_rows >= kPqRows ? pq_ws_bytes(kind, op, n_units, k_t, m_rows) : 0;
+  const size_t b = align256(split) + align256((size_t)m_rows * k_t * kTileK * 2);
   return Q4NX_WS_COUNTER_BYTES + (pq > b ? pq : b);
 }
 
@@ -700,12 +699,20 @@ int mfma_launch(int kind, int op, GemmArgs& a, int n_units, void* ws, size_t ws_
   const size_t xn_b = a.norm_w != nullptr && a.xn_out == nullptr
                           ? align256((size_t)a.m_rows * K * 2) : 0;
   const bool ws_ok = ws != nullptr && Q4NX_ALIGNED(ws, 256);
-  // a prompt block of q4 tiles: the fp16-operand kernel, when the workspace holds what it keeps
+  // The fp16-operand kernel takes two launches; up to K = 512 they do not repay themselves while
+  // the batched kernel's one fits the chip at once or the columns are few (a stream of calls, us,
+  // batched / fp16 operands; N x K, rows): q8 1024 x 512, 1000 rows (256 workgroups) 10.8 / 12.4,
+  // 1500 rows (384) 15.0 / 13.1; q4 2048 x 512, 96 rows 11.8 / 12.3, 128 rows 13.0 / 12.4; 512 x
+  // 512, 3000 rows q4 13.8 / 16.9, q8 15.1 / 15.9
+  const bool short_k = op == GOP_PLAIN && a.k_t <= 2 &&
+                       (a.n_tr[0] <= 16 || (kind == Q4NX_KIND_Q8 ? p.groups * p.m_blocks <= 256
+                                                                 : a.m_rows <= 96));
+  // a prompt block: the fp16-operand kernel, when the workspace holds what it keeps
   // there (a K split that the policy names belongs to the batched kernel)
-  if (pq_use(kind, op, a) && ws_ok && P.gemm_ksplit == 0 &&
+  if (pq_use(op, a) && ws_ok && P.gemm_ksplit == 0 && !short_k &&
       (a.norm_w == nullptr || (a.ssq_in != nullptr && K / kSsqRows <= 512)) &&
-      ws_bytes >= Q4NX_WS_COUNTER_BYTES + pq_ws_bytes(op, a.n_tr[0], a.k_t, a.m_rows)) {
-    pq_launch(op, a, (uint8_t*)ws + Q4NX_WS_COUNTER_BYTES, st);
+      ws_bytes >= Q4NX_WS_COUNTER_BYTES + pq_ws_bytes(kind, op, a.n_tr[0], a.k_t, a.m_rows)) {
+    pq_launch(kind, op, a, (uint8_t*)ws + Q4NX_WS_COUNTER_BYTES, st);
     return check_launch(what);
   }
   if (split && (!ws_ok || ws_bytes < Q4NX_WS_COUNTER_BYTES + align256(split) + xn_b)) {
@@ -730,13 +737,6 @@ int mfma_launch(int kind, int op, GemmArgs& a, int n_units, void* ws, size_t ws_
                        a.ssq_in, a.norm_w, a.eps, K, xn, xs);
     a.x = xn;
     a.x_stride = xs;
-  }
-  // a prompt block: the prefill kernel, when the workspace holds its per-group sums of x
-  // (past the counters, the split records and the normalised rows); else the batched kernel
-  const size_t pf_off = Q4NX_WS_COUNTER_BYTES + align256(split) + xn_b;
-  if (pf_use(kind, op, a) && ws_ok && ws_bytes >= pf_off + pf_ws_bytes(kind, a.n_tr[0], a.k_t, a.m_rows)) {
-    pf_launch(a, (uint8_t*)ws + pf_off, st);
-    return check_launch(what);
   }
   // one m-tile reads x through a buffer resource with 32-bit byte offsets
   Q4NX_REQUIRE(p.mt != 1 || (int64_t)a.m_rows * a.x_stride * 2 < ((int64_t)1 << 31),
@@ -773,12 +773,9 @@ size_t q4nx_gemm_ws_bytes(int kind, int n_tile_rows, int k_tiles, int m_rows,
       m_rows < 1 || !resolve_policy_quiet(policy, &P))
     return 0;
   const size_t split = gemm_split_bytes(plan_gemm(kind, GOP_PLAIN, n_tile_rows, k_tiles, m_rows, P));
-  const size_t pf = pf_ws_bytes(kind, n_tile_rows, k_tiles, m_rows);
-  // the prefill kernel's sums sit past the counters and the split records
-  const size_t b = pf ? (split ? split : Q4NX_WS_COUNTER_BYTES) + pf : split;
-  const size_t pq = kind == Q4NX_KIND_Q4 && m_rows >= kPqRows
-                        ? Q4NX_WS_COUNTER_BYTES + pq_ws_bytes(GOP_PLAIN, n_tile_rows, k_tiles, m_rows) : 0;
-  return pq > b ? pq : b;
+  const size_t pq = m_rows >= kPqRows
+                        ? Q4NX_WS_COUNTER_BYTES + pq_ws_bytes(kind, GOP_PLAIN, n_tile_rows, k_tiles, m_rows) : 0;
+  return pq > split ? pq : split;
 }
 
 int q4nx_gemm(int kind, const uint8_t* w, int n_tile_rows, int k_tiles, const uint16_t* x,

@@ -1,6 +1,5 @@
 // q4nx tile formats as the matrix-core kernels stage and read them: per-kind tile sizes and
-// the code -> bf16 operand conversions shared by the batched (gemm.hip) and prefill
-// (gemm_pf.hip) contractions.
+// the code -> bf16 operand conversions of the batched contraction (gemm.hip).
 #pragma once
 
 #include "common.h"

@@ -1,10 +1,10 @@
-// Prompt-block contraction of q4 tiles on the matrix cores (gfx950), weights and activations
+// Prompt-block contraction of q4nx tiles on the matrix cores (gfx950), weights and activations
 // as fp16 operands: Y[m][n] = R[m][n] + sum_k W[n][k] X[m][k], and [gate, up, SwiGLU].
 //
 // Replaces, for prompt blocks, the torch fallback that reference/npu.py:118-122, 138-140 takes
 // for more than one row.
 //
-// Arithmetic. Per column n and 32-K group g, with the Q4_1 factoring of granite_gemv.h:19-29 and
+// Arithmetic, q4. Per column n and 32-K group g, with the Q4_1 factoring of granite_gemv.h:19-29 and
 // an offset o[n][g] near 7.5 d[n][g],
 //   y[m][n] = sum_k (d[n][g] c[n][k] - o[n][g]) x[m][k] + sum_g u[n][g] S[m][g]
 //   S[m][g] = sum_{k in g} x[m][k]     u[n][g] = m[n][g] + o[n][g]
@@ -19,6 +19,13 @@
 // afterwards. The second sum is a contraction over the groups (32 per MFMA), S and u each in two
 // fp16 terms (the product of the two low terms, 2^-22, is left out). A one-hot row still gives
 // the float32 dequantised column bit for bit.
+//
+// Arithmetic, q8: y[m][n] = sum_g s[n][g] sum_{k in g} q[n][k] x[m][k]. s q has 15 bits, more than
+// one fp16 value holds, so the operand is the code alone (q = (1152 + q) - 1152, the byte under a
+// fixed exponent less a constant) and one MFMA from zero per 16x16 block and group gives the
+// inner sum, which four FMAs per lane scale into the total. (Two MFMAs on s = s1 + s2, four bits
+// each, and no FMA took 555 us for 512 rows of 248320 x 1024, this 471.) x and s under powers of two
+// as above.
 //
 // What bounds it: see pq_kernel.
 #include "common.h"
@@ -53,10 +60,13 @@ __device__ __forceinline__ void split2(float v0, float v1, uint32_t& hi, uint32_
 }
 
 constexpr int kPqChunkTiles = 4;      // K-tiles (32 groups) per minimum-term contraction
-constexpr int kPqHalf = 2560;         // LDS bytes of half a tile: codes of 128 K, their scales
+// LDS bytes of half a tile: codes of 128 K, then their scales
+template <int KIND>
+constexpr int kPqHalf = KIND == 4 ? 2560 : 4352;
 constexpr int kPqXTop = 141;          // 141 - exponent field: the row's largest x in [2^14, 2^15)
 constexpr int kPqWTop = 135;          // |u| of a column below 2^9, its 8 |d| below 2^8
 constexpr int kPqSum = 6;             // S is kept 2^6 below its row's scale, u 2^6 above its column's
+constexpr int kPqSTop = 131;          // a q8 column's largest scale in [2^4, 2^5)
 constexpr float kPqLow = -1031.5f, kPqHigh = -71.5f;   // A / d of the low and the high nibbles
 constexpr int kPqSlack = 64 << 10;    // bytes after x that steps past its end read (never used)
 
@@ -67,8 +77,11 @@ struct PqX {
                     // the steps, two of sums (hi, lo) per chunk of 32 groups, k the group
   u32x4_t* u;       // [tensor][tile-row][chunk][hi, lo][even, odd column][lane]
   uint2* scale;     // [tensor][tile-row][group][lane % 16]: fp16 d of the even and odd column, A
+                    // (q4 only)
   int* xshift;      // [row]: the power of two of x
-  int* wshift;      // [tensor][column]: that of d, A and u
+  int* wshift;      // [tensor][column]: that of d, A and u (q8: of s)
+  int m_blocks, c_groups;   // the launch's row blocks, its groups of columns
+  bool rows_first;  // the order of its workgroups: row blocks first, within an eighth of them
 };
 
 // The larger of each lane's value and its DPP / permlane partner's, over the whole wave
@@ -87,22 +100,30 @@ __device__ __forceinline__ uint32_t rows_max(uint32_t v) {    // across the four
 // 2^e as a float, -126 <= e <= 127
 __device__ __forceinline__ float exp2i(int e) { return __int_as_float((e + 127) << 23); }
 
-constexpr int kPrepThreads = 256;
+// chunks of 32 groups of the minimum term (q8 has none)
+template <int KIND>
+__host__ __device__ constexpr int pq_chunks(int k_t) {
+  return KIND == 4 ? (k_t + kPqChunkTiles - 1) / kPqChunkTiles : 0;
+}
 
-// One row of x per workgroup: x (or RMSNorm of the fp32 residual, to bf16 first, as every
+// One row of x per NT threads (a workgroup, or one wave of it): x (or RMSNorm of the fp32 residual, to bf16 first, as every
 // consumer rounds it) to fp16 under the row's power of two, and the sums per 32-K group. Each
-// thread keeps C chunks of 8 entries (K <= 2048 C; longer rows are read again for the second
+// thread keeps C chunks of 8 entries (K <= 8 NT C; longer rows are read again for the second
 // pass). Every load is unconditional, through a buffer resource over the row: entries past its
 // end read zeros. Rows past m_rows stay unwritten: a row of an operand reaches its own row of
 // the result only. The code is kept short: a wave runs it once, so its instruction fetches are
 // not amortised (eight rows per workgroup, a wave each with up to 16 chunks, took 2.5 times as
 // long).
-template <bool NORM, int C>
+template <int KIND, bool NORM, int C, int NT>
 __device__ __forceinline__ void prep_row(const GemmArgs& a, const PqX& o, int row,
                                          float* __restrict__ sg, uint32_t* __restrict__ smx) {
-  const int tid = threadIdx.x, l = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x & (NT - 1), l = tid & 63, wave = tid >> 6;
+  auto meet = [] {                              // of the row's threads
+    if constexpr (NT > 64) __syncthreads();
+    else __builtin_amdgcn_wave_barrier();
+  };
   const int K = a.k_t * kTileK, n_q = K / 8;
-  const int n_ch = (a.k_t + kPqChunkTiles - 1) / kPqChunkTiles;
+  const int n_ch = pq_chunks<KIND>(a.k_t);
   auto ld = [](__amdgpu_buffer_rsrc_t r, uint32_t off) {
     const v4i_t t = __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0);
     return u32x4_t{(uint32_t)t.x, (uint32_t)t.y, (uint32_t)t.z, (uint32_t)t.w};
@@ -122,7 +143,7 @@ __device__ __forceinline__ void prep_row(const GemmArgs& a, const PqX& o, int ro
     u32x4_t h0[C], h1[C], w[C];
 #pragma unroll
     for (int i = 0; i < C; ++i) {
-      const uint32_t q = tid + kPrepThreads * i;
+      const uint32_t q = tid + NT * i;
       h0[i] = ld(xr, 32 * q);
       h1[i] = ld(xr, 32 * q + 16);
       w[i] = ld(wr, 16 * q);
@@ -139,14 +160,14 @@ __device__ __forceinline__ void prep_row(const GemmArgs& a, const PqX& o, int ro
         v[i][j] = pack_bf16x2((__uint_as_float(h[e]) * inv) * bf16lo(w[i][j]),
                               (__uint_as_float(h[e + 1]) * inv) * bf16hi(w[i][j]));
       }
-      const int q = tid + kPrepThreads * i;
+      const int q = tid + NT * i;
       if (a.xn_out != nullptr && q < n_q)
         *(u32x4_t*)(a.xn_out + (int64_t)row * a.x_stride + 8 * q) = v[i];
     }
   } else {
 #pragma unroll
-    for (int i = 0; i < C; ++i) v[i] = ld(xr, 16 * (tid + kPrepThreads * i));
-    for (int q = tid + kPrepThreads * C; q < n_q; q += kPrepThreads) see(ld(xr, 16 * q));
+    for (int i = 0; i < C; ++i) v[i] = ld(xr, 16 * (tid + NT * i));
+    for (int q = tid + NT * C; q < n_q; q += NT) see(ld(xr, 16 * q));
   }
 #pragma unroll
   for (int i = 0; i < C; ++i) see(v[i]);
@@ -154,9 +175,12 @@ __device__ __forceinline__ void prep_row(const GemmArgs& a, const PqX& o, int ro
   mx = umax_dpp<kDppXor2>(mx);
   mx = umax_dpp<kDppHalfMirror>(mx);
   mx = rows_max(umax_dpp<kDppRor8>(mx));
-  if (l == 0) smx[wave] = mx;
-  __syncthreads();
-  mx = pk_max_u16(pk_max_u16(smx[0], smx[1]), pk_max_u16(smx[2], smx[3]));
+  if constexpr (NT > 64) {
+    if (l == 0) smx[wave] = mx;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NT / 64; ++i) mx = pk_max_u16(mx, smx[i]);
+  }
   // exponent field of the row's largest entry; a row with an infinity or a NaN is left
   // unscaled (its sums carry the NaN into every output of the row)
   const int ex = (int)max(mx >> 16, mx & 0xFFFFu) >> 7;
@@ -166,11 +190,11 @@ __device__ __forceinline__ void prep_row(const GemmArgs& a, const PqX& o, int ro
   const int r16 = row & 15, swz = (r16 >> 1) & 3;
   u32x4_t* xt = o.xt + (size_t)(row >> 4) * (a.k_t * 8 + n_ch * 2) * 64 + r16 * 4;
   u32x4_t* sm = xt + (size_t)a.k_t * 8 * 64;
-  for (int i0 = 0; i0 * 8 * kPrepThreads < K; i0 += C) {
-    if (i0 > 0) __syncthreads();                // the sums of the section before are read
+  for (int i0 = 0; i0 * 8 * NT < K; i0 += C) {
+    if (KIND == 4 && i0 > 0) meet();   // the sums of the section before are read
 #pragma unroll
     for (int i = 0; i < C; ++i) {
-      const int q = tid + kPrepThreads * (i0 + i);
+      const int q = tid + NT * (i0 + i);
       u32x4_t w = v[i];
       if (!NORM && i0 > 0) w = ld(xr, 16 * q);
       u32x4_t h;
@@ -185,14 +209,17 @@ __device__ __forceinline__ void prep_row(const GemmArgs& a, const PqX& o, int ro
         s += x0 + x1;
       }
       if (q < n_q) xt[(size_t)(q >> 2) * 64 + ((q & 3) ^ swz)] = h;
-      s += dpp<kDppXor1>(s);
-      s += dpp<kDppXor2>(s);                    // the group's sum, in its four lanes
-      if ((l & 3) == 0) sg[64 * i + (tid >> 2)] = s;
+      if constexpr (KIND == 4) {
+        s += dpp<kDppXor1>(s);
+        s += dpp<kDppXor2>(s);                  // the group's sum, in its four lanes
+        if ((l & 3) == 0) sg[NT / 4 * i + (tid >> 2)] = s;
+      }
     }
-    __syncthreads();
+    if constexpr (KIND != 4) continue;
+    meet();
     // eight groups per thread (groups past K hold zeros, which the last chunk keeps)
-    const int g = 64 * i0 + 8 * tid;
-    if (tid < 8 * C && g < 32 * n_ch) {
+    const int g = NT / 4 * i0 + 8 * tid;
+    if (tid < NT / 32 * C && g < 32 * n_ch) {
       u32x4_t hi, lo;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -209,14 +236,15 @@ __device__ __forceinline__ void prep_row(const GemmArgs& a, const PqX& o, int ro
 }
 
 // Weight tile-row: its columns' powers of two and u = m + 8 d in the minimum term's B operand
-// order. Four waves per tile-row, a chunk of 32 groups each: lane (c, s) holds columns
+// order. NW waves per tile-row, a chunk of 32 groups each: lane (c, s) holds columns
 // (c / 8) 16 + 2 (c % 8), + 1 at groups 8 s + j (K-tile 4 ch + s).
+template <int NW>
 __device__ __forceinline__ void prep_tile_row(const GemmArgs& a, const PqX& o, int tensor, int tr,
                                               uint32_t* __restrict__ sm) {
-  constexpr int CACHED = 2;                     // chunks a wave keeps: K <= 8192
+  constexpr int CACHED = 2;                     // chunks a wave keeps: K <= 2048 NW
   const int l = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c = l & 15, s = l >> 4, n_tr = a.n_tr[0];
-  const int n_ch = (a.k_t + kPqChunkTiles - 1) / kPqChunkTiles;
+  const int n_ch = pq_chunks<4>(a.k_t);
   const uint8_t* wr = a.w[tensor] + (size_t)tr * a.k_t * kQ4TileBytes +
                       2 * ((c >> 3) * 16 + 2 * (c & 7));
   uint32_t dv[CACHED][8], mv[CACHED][8], dm = 0, mm = 0;
@@ -246,14 +274,14 @@ __device__ __forceinline__ void prep_tile_row(const GemmArgs& a, const PqX& o, i
   };
 #pragma unroll
   for (int i = 0; i < CACHED; ++i)
-    if (w + 4 * i < n_ch) fetch(w + 4 * i, dv[i], mv[i]);
+    if (w + NW * i < n_ch) fetch(w + NW * i, dv[i], mv[i]);
 #pragma unroll
   for (int i = 0; i < CACHED; ++i)
-    if (w + 4 * i < n_ch) {
-      clip(w + 4 * i, dv[i], mv[i]);
+    if (w + NW * i < n_ch) {
+      clip(w + NW * i, dv[i], mv[i]);
       see(dv[i], mv[i]);
     }
-  for (int ch = w + 4 * CACHED; ch < n_ch; ch += 4) {
+  for (int ch = w + NW * CACHED; ch < n_ch; ch += NW) {
     uint32_t d[8], m[8];
     fetch(ch, d, m);
     clip(ch, d, m);
@@ -267,7 +295,7 @@ __device__ __forceinline__ void prep_tile_row(const GemmArgs& a, const PqX& o, i
   }
   __syncthreads();
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < NW; ++i) {
     dm = pk_max_u16(dm, sm[i * 32 + c]);
     mm = pk_max_u16(mm, sm[i * 32 + 16 + c]);
   }
@@ -315,8 +343,8 @@ __device__ __forceinline__ void prep_tile_row(const GemmArgs& a, const PqX& o, i
   };
 #pragma unroll
   for (int i = 0; i < CACHED; ++i)
-    if (w + 4 * i < n_ch) put(w + 4 * i, dv[i], mv[i]);
-  for (int ch = w + 4 * CACHED; ch < n_ch; ch += 4) {
+    if (w + NW * i < n_ch) put(w + NW * i, dv[i], mv[i]);
+  for (int ch = w + NW * CACHED; ch < n_ch; ch += NW) {
     uint32_t d[8], m[8];
     fetch(ch, d, m);
     clip(ch, d, m);
@@ -324,17 +352,56 @@ __device__ __forceinline__ void prep_tile_row(const GemmArgs& a, const PqX& o, i
   }
 }
 
-// Workgroups [0, m_rows): a row of x each; the rest: a weight tile-row each, over both tensors
-// of [gate, up].
-template <bool NORM, int C>
-__global__ __launch_bounds__(kPrepThreads) void pq_prep_kernel(GemmArgs a, PqX o) {
-  __shared__ float sg[64 * C];
-  __shared__ uint32_t sm[128];
-  if ((int)blockIdx.x < a.m_rows) {
-    prep_row<NORM, C>(a, o, blockIdx.x, sg, sm);
+// Of a q8 tile-row: the columns' powers of two. Each wave takes K-tiles, lane (c, s) the scales of
+// columns 2 c and 2 c + 1 at groups 2 s and 2 s + 1.
+template <int NW>
+__device__ __forceinline__ void prep_tile_row_q8(const GemmArgs& a, const PqX& o, int tr,
+                                                 uint32_t* __restrict__ sm) {
+  const int l = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = l & 15, s = l >> 4;
+  const uint8_t* wr = a.w[0] + (size_t)tr * a.k_t * kQ8TileBytes + 128 * s + 4 * c;
+  uint32_t mx = 0;
+  for (int kt = w; kt < a.k_t; kt += NW)
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+      mx = pk_max_u16(mx, *(const uint32_t*)(wr + (size_t)kt * kQ8TileBytes + 64 * e) & 0x7FFF7FFFu);
+  mx = rows_max(mx);
+  if (l < 16) sm[w * 16 + l] = mx;
+  __syncthreads();
+  if (w > 0 || l >= 16) return;
+#pragma unroll
+  for (int i = 1; i < NW; ++i) mx = pk_max_u16(mx, sm[16 * i + c]);
+  int sh[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int e = (int)((mx >> (16 * h + 7)) & 0xFF);
+    sh[h] = e < 255 ? min(kPqSTop - max(e, 1), 127) : 0;
+  }
+  *(int2*)(o.wshift + (size_t)tr * 32 + 2 * c) = make_int2(sh[0], sh[1]);
+}
+
+// First a weight tile-row per workgroup, over both tensors of [gate, up] -- the longer ones -- then
+// ROWS rows of x each.
+// What bounds it: the latency of one workgroup (3 us launched empty-handed; 80 tile-rows of K =
+// 8192 took 8.9 us in four waves, 5.4 in the eight of K > 4096) and, with many rows, their bytes
+// (2048 x 2560, 21 MB in and out, 8.2 us). Rows of K <= 1024 leave most of a workgroup idle and
+// are a wave each, so a workgroup's 64-byte pieces of x also fill whole cache lines (3000 rows of
+// K = 512 8.2 -> 6.8 us, and with 12288 columns the contraction after it 61 -> 57); two or four
+// longer rows per workgroup gain nothing (2048 x 2560 9.1 -> 10.1, 9.9).
+template <int KIND, bool NORM, int C, int NT, int ROWS>
+__global__ __launch_bounds__(NT) void pq_prep_kernel(GemmArgs a, PqX o, int tile_rows) {
+  __shared__ float sg[KIND == 4 ? NT / 4 * C : 1];
+  __shared__ uint32_t sm[NT / 2];
+  const int t = blockIdx.x, n = a.n_tr[0];
+  if (t >= tile_rows) {
+    constexpr int TR = NT / ROWS;                 // threads of a row: one wave, or all
+    const int sub = ROWS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / TR);
+    // (past the last row: that row again, in step with the others)
+    prep_row<KIND, NORM, C, TR>(a, o, min((t - tile_rows) * ROWS + sub, a.m_rows - 1),
+                                sg + (KIND == 4 ? TR / 4 * C * sub : 0), sm + TR / 64 * sub);
   } else {
-    const int t = blockIdx.x - a.m_rows, n = a.n_tr[0];
-    prep_tile_row(a, o, t / n, t % n, sm);
+    if constexpr (KIND == 4) prep_tile_row<NT / 64>(a, o, t / n, t % n, sm);
+    else prep_tile_row_q8<NT / 64>(a, o, t, sm);
   }
 }
 
@@ -351,6 +418,8 @@ __device__ __forceinline__ void step_barrier() {
   __builtin_amdgcn_sched_barrier(0);
   asm volatile("" ::: "memory");
 }
+
+__device__ __forceinline__ void pin_acc(f32x4_t& v) { asm volatile("" : "+v"(v)); }
 
 // 16 bytes (4: one dword) per lane from uniform base + offset + lane offset to LDS at lds + off
 // + 16 (4) lane
@@ -383,16 +452,18 @@ __device__ __forceinline__ void ldl4(const void* base, uint32_t voff, uint32_t l
 // (575 -> 905 TFLOP/s); 2560 x 8192, 333 rows 62 -> 37; [gate, up] 8192 x 2560, 500 rows 126 ->
 // 57 us, 2048 rows 477 -> 193. Error against 64 bits: 2048 rows, K = 2560 1.06e-6 -> 3.2e-7, 333
 // rows, K = 8192 3.1e-7 -> 1.2e-7.
-template <int OP, int MT, int RT, int WN, int WK, int RING, int OCC>
+template <int KIND, int OP, int MT, int RT, int WN, int WK, int RING, int OCC>
 __global__ __launch_bounds__(64 * WN * WK, OCC) void pq_kernel(GemmArgs a, PqX p) {
-  constexpr int TB = kQ4TileBytes;
+  constexpr int TB = GemmFmt<KIND>::kTile, HALF = kPqHalf<KIND>;
+  constexpr int NR = KIND == 4 ? 1 : 2;        // transposing reads of a step's codes
+  constexpr int NC = KIND == 4 ? 2 : 4;        // direct loads of half a tile's codes
   constexpr int U = MT / WN;                   // x units (1 KB: one m-tile, one step) per wave
   constexpr int XD = RING - 1;                 // steps of x in flight ahead of use
   constexpr bool LOOK = RING == 8;             // x read from LDS ahead across the step boundary
-  constexpr int WL = 4 * RT;                   // direct loads of half a weight tile
+  constexpr int WL = (NC + (KIND == 4 ? 2 : 1)) * RT;            // direct loads of half a weight tile
   static_assert(MT % WN == 0, "every wave stages as many m-tiles");
   static_assert(8 % RING == 0, "a step's ring slot is known at compile time");
-  static_assert(OP == GOP_PLAIN || RT == 2, "gate and up");
+  static_assert(OP == GOP_PLAIN || (KIND == 4 && RT == 2), "gate and up");
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
 
   const int tid = threadIdx.x, l = tid & 63;
@@ -400,10 +471,20 @@ __global__ __launch_bounds__(64 * WN * WK, OCC) void pq_kernel(GemmArgs a, PqX p
   const int wn = wave % WN, wk = wave / WN;
   const int c = l & 15, s = l >> 4;
   const int n_tr = a.n_tr[0];
-  const int n_ch = (a.k_t + kPqChunkTiles - 1) / kPqChunkTiles;
+  const int n_ch = pq_chunks<KIND>(a.k_t);
   const int unit_steps = a.k_t * 8 + n_ch * 2;  // per m-tile: the steps of x, then of the sums
-  const int unit = blockIdx.x * WN + wn;       // RT tile-rows, or one pair
-  const int m0 = blockIdx.y * 16 * MT;
+  int cgrp, mblk;
+  if (p.rows_first) {
+    const int tile = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    cgrp = tile / p.m_blocks;
+    mblk = tile - cgrp * p.m_blocks;
+  } else {
+    mblk = blockIdx.x / p.c_groups;
+    cgrp = blockIdx.x - mblk * p.c_groups;
+  }
+  const int unit = cgrp * WN + wn;             // RT tile-rows, or one pair
+  if (cgrp >= p.c_groups || mblk >= p.m_blocks) return;   // the grid is a multiple of 8
+  const int m0 = mblk * 16 * MT;
   // this wave's K part (a wave whose part ends early, or is empty, keeps the others' barriers)
   const int kq = (a.k_t + WK - 1) / WK;
   const int kt0 = min(wk * kq, a.k_t - 1), kt1 = min(a.k_t, wk * kq + kq);
@@ -420,7 +501,7 @@ __global__ __launch_bounds__(64 * WN * WK, OCC) void pq_kernel(GemmArgs a, PqX p
   }
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
   const uint32_t xring = wk * RING * MT * 1024;                       // this part's x ring
-  constexpr int WBUF = RT * 2 * kPqHalf;       // one K-tile of the wave's tile-rows
+  constexpr int WBUF = RT * 2 * HALF;       // one K-tile of the wave's tile-rows
   const uint32_t wslot = WK * RING * MT * 1024 + wave * WBUF;
   const uint32_t l16 = 16 * l, l4 = 4 * l;
   const uint32_t xm0 = lds0 + xring + wn * 1024, wm0 = lds0 + wslot;
@@ -428,14 +509,13 @@ __global__ __launch_bounds__(64 * WN * WK, OCC) void pq_kernel(GemmArgs a, PqX p
 #pragma unroll
   for (int j = 0; j < U; ++j)
     xp[j] = (const uint8_t*)p.xt +
-            ((size_t)(blockIdx.y * MT + wn + WN * j) * unit_steps + kt0 * 8) * 1024;
+            ((size_t)(mblk * MT + wn + WN * j) * unit_steps + kt0 * 8) * 1024;
   // the part's chunks of the minimum term, and from its last x step to its sums
   const int ch0 = kt0 / kPqChunkTiles, nc = nt > 0 ? (kt1 + kPqChunkTiles - 1) / kPqChunkTiles - ch0 : 0;
-  const int64_t to_sums = (int64_t)((a.k_t - kt1) * 8 + ch0 * 2 + 4) * 1024;
+  const int64_t to_sums = KIND == 4 ? (int64_t)((a.k_t - kt1) * 8 + ch0 * 2 + 4) * 1024 : 4096;
   const uint8_t *up[RT], *sp[RT];              // its u, its scales
 #pragma unroll
-  for (int r = 0; r < RT; ++r)
-  {
+  for (int r = 0; r < RT; ++r) {
     up[r] = (const uint8_t*)(p.u + ((size_t)col0[r] * n_ch + ch0) * 4 * 64);
     sp[r] = (const uint8_t*)(p.scale + (size_t)col0[r] * a.k_t * 128);
   }
@@ -453,21 +533,32 @@ __global__ __launch_bounds__(64 * WN * WK, OCC) void pq_kernel(GemmArgs a, PqX p
     for (int j = 0; j < U; ++j)
       ldl16<(ks & 3) * 1024>(xp[j], l16, xm0, ((ks % RING) * MT + WN * j) * 1024);
   };
-  // half of the part's K-tile t: 128 K of codes and their scales; after the last tile, the high (low) terms of the part's first chunk of u in their place, in as many
-  // loads
+  // half of the part's K-tile t: 128 K of codes and their scales; after the last tile, in as many
+  // loads, the high (low) terms of the part's first chunk of u in their place (q8: that tile
+  // again, never used)
   auto w_load = [&](int t, auto halfc) {
     constexpr int half = decltype(halfc)::value;
     const bool more = t < nt;
+    const int kt = KIND == 4 ? kt0 + t : kt0 + (more ? t : max(nt - 1, 0));
 #pragma unroll
     for (int r = 0; r < RT; ++r) {
-      const uint8_t* w = wr[r] + (size_t)(kt0 + t) * TB;
-      const uint8_t* u = up[r] + half * 2048;
-      const int d = (r * 2 + half) * kPqHalf;
-      ldl16<0>(more ? w + 1024 + half * 1024 : u, l16, wm0, d);
-      ldl16<0>(more ? w + 3072 + half * 1024 : u + 1024, l16, wm0, d + 1024);
-      const uint8_t* q = more ? sp[r] + (size_t)(kt0 + t) * 1024 + half * 512 : u;
-      ldl4<0>(q, l4, wm0, d + 2048);
-      ldl4<256>(q, l4, wm0, d + 2304);
+      const uint8_t* w = wr[r] + (size_t)kt * TB;
+      const uint8_t* q = sp[r] + (size_t)kt * 1024 + half * 512;
+      const int d = (r * 2 + half) * HALF;
+      if constexpr (KIND == 4) {
+        const uint8_t* u = up[r] + half * 2048;
+        ldl16<0>(more ? w + 1024 + half * 1024 : u, l16, wm0, d);
+        ldl16<0>(more ? w + 3072 + half * 1024 : u + 1024, l16, wm0, d + 1024);
+        q = more ? q : u;
+        ldl4<256>(q, l4, wm0, d + NC * 1024 + 256);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)            // each row block's 2 KB
+          ldl16<0>(w + kMetaBytes + (i >> 1) * 4096 + half * 2048 + (i & 1) * 1024, l16, wm0,
+                   d + i * 1024);
+        q = w + half * 256;
+      }
+      ldl4<0>(q, l4, wm0, d + NC * 1024);
     }
   };
 #pragma unroll
@@ -486,36 +577,54 @@ __global__ __launch_bounds__(64 * WN * WK, OCC) void pq_kernel(GemmArgs a, PqX p
   // added to the total on the VALU (the matrix cores' own accumulation rounds more coarsely: K =
   // 8192 in one chain is 5.9e-7 off the 64-bit result, in tiles 1.2e-7 .. 1.6e-7; the kernel of
   // this shape before, 1.9e-6)
-  constexpr bool FLUSH = MT * RT <= 8;
+  constexpr bool FLUSH = KIND == 4 && MT * RT <= 8;
   f32x4_t prt[FLUSH ? RT : 1][FLUSH ? MT : 1][2];
   const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+  // the lane's two columns of a tile-row (its even and odd column, or column c of each row block)
+  const int cols[2] = {KIND == 4 ? (c >> 3) * 16 + 2 * (c & 7) : c,
+                       KIND == 4 ? (c >> 3) * 16 + 2 * (c & 7) + 1 : 16 + c};
   int shw[RT][2];                              // the columns' powers of two
 #pragma unroll
   for (int r = 0; r < RT; ++r) {
-    const int2 v = *(const int2*)(p.wshift + (size_t)col0[r] * 32 + (c >> 3) * 16 + 2 * (c & 7));
-    shw[r][0] = v.x;
-    shw[r][1] = v.y;
+    shw[r][0] = p.wshift[(size_t)col0[r] * 32 + cols[0]];
+    shw[r][1] = p.wshift[(size_t)col0[r] * 32 + cols[1]];
   }
-  // ---- operands: the transposing LDS read gives lane (c, s) the 8 code bytes of row pair
-  // c % 8 of row-block c / 8 at k = 8 s ..; low nibbles are the even row, high the odd one
-  const uint8_t* const trp = lds + wslot + (c & 1) * 1024 + (8 * s + (c >> 1)) * 8;
-  const uint8_t* const scp = lds + wslot + 2048 + 8 * c;
+  // q8: the inner sums on their way to the totals (each LAG MFMAs after its own), the scales of
+  // the steps of either parity, the columns' powers of two
+  constexpr int LAG = 3;
+  f32x4_t inner[4] = {zero, zero, zero, zero};
+  float scl[2][RT][2] = {}, wsc[RT][2];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) wsc[r][h] = exp2i(shw[r][h]);
+  // ---- operands: the transposing LDS read gives lane (c, s) the 8 code bytes at k = 8 s .. of
+  // row pair c % 8 of row-block c / 8, low nibbles the even row, high the odd one (q8: of row c
+  // of one row block per read)
+  const uint8_t* const trp = lds + wslot + (KIND == 4 ? (c & 1) * 1024 + (8 * s + (c >> 1)) * 8
+                                                      : (8 * s + (c >> 1)) * 16 + (c & 1) * 8);
+  const uint8_t* const scp = lds + wslot + NC * 1024 + (KIND == 4 ? 8 : 2) * c;
   struct Raw {
-    i32x2_t cb;
-    uint2 sc;                                  // fp16 (d even, d odd), (A even, A odd)
+    i32x2_t cb[NR];
+    uint2 sc;                                  // fp16 (d even, d odd), (A even, A odd); q8: bf16
   } raw[2][RT];                                // of steps of either parity
   auto read_raw = [&](int kb) {
 #pragma unroll
     for (int r = 0; r < RT; ++r) {
-      const int b = (r * 2 + (kb >> 2)) * kPqHalf;
-      raw[kb & 1][r].cb = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
-          (lds_i32x2_t*)(trp + b + (kb & 3) * 256));
-      raw[kb & 1][r].sc = *(const uint2*)(scp + b + (kb & 3) * 128);
+      const int b = (r * 2 + (kb >> 2)) * HALF;
+#pragma unroll
+      for (int h = 0; h < NR; ++h)
+        raw[kb & 1][r].cb[h] = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
+            (lds_i32x2_t*)(trp + b + h * 2048 + (kb & 3) * (KIND == 4 ? 256 : 512)));
+      if constexpr (KIND == 4) raw[kb & 1][r].sc = *(const uint2*)(scp + b + (kb & 3) * 128);
+      else
+        raw[kb & 1][r].sc = make_uint2(*(const uint16_t*)(scp + b + (kb & 3) * 64),
+                                       *(const uint16_t*)(scp + b + (kb & 3) * 64 + 32));
     }
   };
-  // The operands of a step, in 8 RT half pieces: the first half of a piece takes the low and the
-  // high nibbles of two code bytes (bytes 0 and 2, or 1 and 3, of word h) to fp16 B + c, the
-  // second multiplies and adds.
+  // The operands of a step, in 8 NR RT half pieces: the first half of a piece takes two code
+  // bytes (0 and 2, or 1 and 3) of a word to fp16 B + c -- their low and their high nibbles (q8:
+  // the bytes) -- the second multiplies and adds (q8: subtracts).
   u32x4_t ops[2][RT][2];
   uint32_t msk_l, msk_h, exp_l, exp_h, tE = 0, tO = 0;
   asm("v_mov_b32 %0, 0x000f000f" : "=v"(msk_l));
@@ -523,17 +632,45 @@ __global__ __launch_bounds__(64 * WN * WK, OCC) void pq_kernel(GemmArgs a, PqX p
   asm("s_mov_b32 %0, 0x64006400" : "=s"(exp_l));
   asm("s_mov_b32 %0, 0x54005400" : "=s"(exp_h));
   auto half_piece = [&](int b, int i) {        // into ops[b] from raw[b]
-    const int r = i >> 3, h = (i >> 2) & 1, q = (i >> 1) & 1;
-    if ((i & 1) == 0) {
-      const uint32_t w = (h ? (uint32_t)raw[b][r].cb.y : (uint32_t)raw[b][r].cb.x) >> (8 * q);
-      tE = (w & msk_l) | exp_l;
-      tO = (w & msk_h) | exp_h;
-    } else {
+    const int r = i / (8 * NR), col = (i >> 3) & (NR - 1), h = (i >> 2) & 1, q = (i >> 1) & 1;
+    const i32x2_t cb = raw[b][r].cb[col];
+    if constexpr (KIND == 4) {
+      const uint32_t w = h ? (uint32_t)cb.y : (uint32_t)cb.x;
+      if ((i & 1) == 0) {
+        tE = ((w >> (8 * q)) & msk_l) | exp_l;
+        tO = ((w >> (8 * q)) & msk_h) | exp_h;
+        return;
+      }
       const half2_t d = as_h2(raw[b][r].sc.x), A = as_h2(raw[b][r].sc.y);
       const half2_t dE = {d.x, d.x}, dO = {d.y, d.y}, aE = {A.x, A.x}, aO = {A.y, A.y};
       ops[b][r][0][2 * h + q] = h2_bits(__builtin_elementwise_fma(as_h2(tE), dE, aE));
       ops[b][r][1][2 * h + q] = h2_bits(__builtin_elementwise_fma(as_h2(tO), dO, aO));
+    } else {
+      if ((i & 3) == 0) tO = (h ? (uint32_t)cb.y : (uint32_t)cb.x) ^ 0x80808080u;
+      if ((i & 1) == 0) {
+        tE = __builtin_amdgcn_perm(exp_l, tO, q ? 0x07030701u : 0x07020700u);   // 0x64 code bytes
+        return;
+      }
+      const half2_t k = {(_Float16)1152.f, (_Float16)1152.f};
+      uint32_t o = h2_bits(as_h2(tE) - k);
+      asm volatile("" : "+v"(o));
+      ops[b][r][col][2 * h + q] = o;
     }
+  };
+  auto scales = [&](int b) {                   // q8: scl[b] from raw[b]
+    if constexpr (KIND == 8)
+#pragma unroll
+      for (int r = 0; r < RT; ++r) {
+        scl[b][r][0] = __uint_as_float(raw[b][r].sc.x << 16) * wsc[r][0];
+        scl[b][r][1] = __uint_as_float(raw[b][r].sc.y << 16) * wsc[r][1];
+      }
+  };
+  // q8: MFMA f's inner sums, a step of parity b, into the totals
+  auto fold = [&](int f, int b) {
+    const int h = f & 1, r = (f >> 1) % RT, mt = (f >> 1) / RT;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[r][mt][h][e] = fmaf(scl[b][r][h], inner[f & 3][e], acc[r][mt][h][e]);
+    pin_acc(acc[r][mt][h]);
   };
 
   __builtin_amdgcn_s_waitcnt(vm_wait_pq(0));
@@ -541,7 +678,8 @@ __global__ __launch_bounds__(64 * WN * WK, OCC) void pq_kernel(GemmArgs a, PqX p
   read_raw(0);
   read_raw(1);
 #pragma unroll
-  for (int i = 0; i < 8 * RT; ++i) half_piece(0, i);
+  for (int i = 0; i < 8 * NR * RT; ++i) half_piece(0, i);
+  scales(0);
   // x fragments are read from LDS D m-tiles ahead of their use (LOOK: across the step boundary
   // too) and a step's operand data two steps ahead
   constexpr int D = MT < 3 ? MT : 3;
@@ -572,14 +710,23 @@ __global__ __launch_bounds__(64 * WN * WK, OCC) void pq_kernel(GemmArgs a, PqX p
         for (int r = 0; r < RT; ++r)
 #pragma unroll
           for (int h = 0; h < 2; ++h) {
+            constexpr int F = MT * RT * 2;
+            const int f = (mt * RT + r) * 2 + h;
             const u32x4_t& x = xa[(kb * MT + mt) & 3];
-            if constexpr (!FLUSH) acc[r][mt][h] = mfma_f16(x, ops[cur][r][h], acc[r][mt][h]);
-            else prt[r][mt][h] = mfma_f16(x, ops[cur][r][h], kb == 0 ? zero : prt[r][mt][h]);
+            if constexpr (KIND == 8) {
+              inner[f & 3] = mfma_f16(x, ops[cur][r][h], zero);
+              if (f >= LAG) fold(f - LAG, cur);
+              else fold(F + f - LAG, nxt);     // the step before's (before the first: zeros)
+              if (f == LAG) scales(nxt);
+            } else if constexpr (!FLUSH) {
+              acc[r][mt][h] = mfma_f16(x, ops[cur][r][h], acc[r][mt][h]);
+            } else {
+              prt[r][mt][h] = mfma_f16(x, ops[cur][r][h], kb == 0 ? zero : prt[r][mt][h]);
+            }
             // one MFMA, then the part of the operand build that fits beside it: a wave issues in
             // order, so MFMAs back to back would hold the build up until the last has started
-            const int n = (mt * RT + r) * 2 + h;
 #pragma unroll
-            for (int i = n * 4 / MT; i < (n + 1) * 4 / MT; ++i) half_piece(nxt, i);
+            for (int i = f * 4 * NR / MT; i < (f + 1) * 4 * NR / MT; ++i) half_piece(nxt, i);
             __builtin_amdgcn_sched_barrier(0);
           }
         // the half tile whose last operand data this step's build has used is loaded again
@@ -611,6 +758,9 @@ __global__ __launch_bounds__(64 * WN * WK, OCC) void pq_kernel(GemmArgs a, PqX p
       step_barrier();
     });
   }
+  if constexpr (KIND == 8)
+#pragma unroll
+    for (int f = MT * RT * 2 - LAG; f < MT * RT * 2; ++f) fold(f, 1);
   for (int t = nt > 0 ? nt : 0; t < kq; ++t)   // a shorter part: the others' barriers
 #pragma unroll
     for (int kb = 0; kb < 8; ++kb) step_barrier();
@@ -618,11 +768,11 @@ __global__ __launch_bounds__(64 * WN * WK, OCC) void pq_kernel(GemmArgs a, PqX p
   // ---- the minimum term, in the same scale: A holds the S terms (ring steps after the last of
   // x), B u of the lane's two columns at groups 32 ch + 8 s + j (K-tile 4 ch + s; zero outside
   // the part). The next chunk's are loaded while this one's are used.
-  const int nc_all = WK == 1 ? nc : (kq + 2 * kPqChunkTiles - 2) / kPqChunkTiles;   // any part's, at most
+  const int nc_all = KIND != 4 ? 0 : WK == 1 ? nc : (kq + 2 * kPqChunkTiles - 2) / kPqChunkTiles;   // any part's, at most
   const uint8_t* sx[U];
 #pragma unroll
   for (int j = 0; j < U; ++j)
-    sx[j] = (const uint8_t*)p.xt + ((size_t)(blockIdx.y * MT + wn + WN * j) * unit_steps +
+    sx[j] = (const uint8_t*)p.xt + ((size_t)(mblk * MT + wn + WN * j) * unit_steps +
                                     a.k_t * 8 + ch0 * 2) * 1024;
   for (int i = 0; i < nc_all; ++i) {
     __builtin_amdgcn_s_waitcnt(vm_wait_pq(0));
@@ -635,7 +785,7 @@ __global__ __launch_bounds__(64 * WN * WK, OCC) void pq_kernel(GemmArgs a, PqX p
     for (int r = 0; r < RT; ++r)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const u32x4_t v = *(const u32x4_t*)(lds + wslot + (r * 2 + (e >> 1)) * kPqHalf +
+        const u32x4_t v = *(const u32x4_t*)(lds + wslot + (r * 2 + (e >> 1)) * HALF +
                                             (e & 1) * 1024 + l16);
         uu[r][e >> 1][e & 1] = in ? v : u32x4_t{0, 0, 0, 0};
       }
@@ -668,11 +818,11 @@ __global__ __launch_bounds__(64 * WN * WK, OCC) void pq_kernel(GemmArgs a, PqX p
 #pragma unroll
           for (int k = 0; k < 4; ++k)
             ldl16d(up[r] + (size_t)(i + 1) * 4096 + k * 1024, l16,
-                   wm0 + (r * 2 + (k >> 1)) * kPqHalf + (k & 1) * 1024);
+                   wm0 + (r * 2 + (k >> 1)) * HALF + (k & 1) * 1024);
       }
     }
   }
-  if constexpr (FLUSH) {
+  if constexpr (FLUSH && KIND == 4) {
     if (nc > 0) {
 #pragma unroll
       for (int r = 0; r < RT; ++r)
@@ -731,50 +881,70 @@ __global__ __launch_bounds__(64 * WN * WK, OCC) void pq_kernel(GemmArgs a, PqX p
   }
 
   // ---- outputs: the lane's two columns are adjacent, so the 16 lanes of a row write 128
-  // contiguous bytes (64 of bf16)
-  const int col = (c >> 3) * 16 + 2 * (c & 7);
+  // contiguous bytes (64 of bf16; q8: 64 bytes per row block)
+  // (an output's address is a uniform row 16 mt + e plus the lane's 32-bit offset)
+  const uint32_t ly = (uint32_t)(4 * s * (OP == GOP_PLAIN ? a.y_stride : a.h_stride) + cols[0]);
   auto store = [&](auto fullc) {               // full: every row of the block is one of X
     constexpr bool FULL = decltype(fullc)::value;
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int m = m0 + 16 * mt + 4 * s + e;
+        const int mu = m0 + 16 * mt + e, m = mu + 4 * s;
         const bool row_live = FULL || m < a.m_rows;
         if constexpr (OP == GOP_PLAIN) {
 #pragma unroll
           for (int r = 0; r < RT; ++r) {
             if (tr[r] >= n_tr) continue;
+            const int64_t o = (int64_t)mu * a.y_stride + (int64_t)tr[r] * 32;
             float2 v = make_float2(acc[r][mt][0][e], acc[r][mt][1][e]);
-            const int64_t o = (int64_t)m * a.y_stride + (int64_t)tr[r] * 32 + col;
             if (row_live) {
               if (a.residual != nullptr) {
-                const float2 rr = *(const float2*)(a.residual + o);
-                v.x += rr.x;
-                v.y += rr.y;
+                const float* rr = a.residual + o;
+                if constexpr (KIND == 4) {
+                  const float2 t = *(const float2*)(rr + ly);
+                  v.x += t.x;
+                  v.y += t.y;
+                } else {
+                  v.x += rr[ly];
+                  v.y += rr[ly + 16];
+                }
               }
-              if (a.y != nullptr) *(float2*)(a.y + o) = v;
+              if (a.y != nullptr) {
+                float* yy = a.y + o;
+                if constexpr (KIND == 4) *(float2*)(yy + ly) = v;
+                else {
+                  yy[ly] = v.x;
+                  yy[ly + 16] = v.y;
+                }
+              }
             }
-            if (a.ssq_out != nullptr) {        // per 16-row block: 8 lanes
-              float q = fmaf(v.x, v.x, v.y * v.y);
-              q += dpp<kDppXor1>(q);
-              q += dpp<kDppXor2>(q);
-              q += dpp<kDppHalfMirror>(q);
-              if (row_live && (c & 7) == 0)
-                a.ssq_out[(int64_t)m * n_tr * 2 + tr[r] * 2 + (c >> 3)] = q;
+            if (a.ssq_out != nullptr) {        // per 16-row block: 8 lanes (q8: 16, a column each)
+              float* so = a.ssq_out + (int64_t)m * n_tr * 2 + tr[r] * 2;
+              if constexpr (KIND == 4) {
+                float q = fmaf(v.x, v.x, v.y * v.y);
+                q += dpp<kDppXor1>(q);
+                q += dpp<kDppXor2>(q);
+                q += dpp<kDppHalfMirror>(q);
+                if (row_live && (c & 7) == 0) so[c >> 3] = q;
+              } else {
+                const float q0 = group16_sum(v.x * v.x), q1 = group16_sum(v.y * v.y);
+                if (row_live && c == 0) so[0] = q0, so[1] = q1;
+              }
             }
           }
         } else {
           if (tr[0] >= n_tr || !row_live) continue;
-          const int64_t N = (int64_t)n_tr * 32, n = (int64_t)tr[0] * 32 + col;
+          const int64_t N = (int64_t)n_tr * 32, n = (int64_t)tr[0] * 32;
           const float g0 = acc[0][mt][0][e], g1 = acc[0][mt][1][e];
           const float u0 = acc[1][mt][0][e], u1 = acc[1][mt][1][e];
-          *(uint32_t*)(a.h_out + (int64_t)m * a.h_stride + n) =
+          *(uint32_t*)(a.h_out + (int64_t)mu * a.h_stride + n + ly) =
               pack_bf16x2(swiglu(round_bf16_op(g0), round_bf16_op(u0)),
                           swiglu(round_bf16_op(g1), round_bf16_op(u1)));
           if (a.raw_out != nullptr) {
-            *(float2*)(a.raw_out + (int64_t)m * 2 * N + n) = make_float2(g0, g1);
-            *(float2*)(a.raw_out + (int64_t)m * 2 * N + N + n) = make_float2(u0, u1);
+            float* ro = a.raw_out + (int64_t)m * 2 * N + n + cols[0];
+            *(float2*)ro = make_float2(g0, g1);
+            *(float2*)(ro + N) = make_float2(u0, u1);
           }
         }
       }
@@ -786,12 +956,12 @@ __global__ __launch_bounds__(64 * WN * WK, OCC) void pq_kernel(GemmArgs a, PqX p
 // ---------------------------------------------------------------- host side
 
 size_t pq_align(size_t b) { return (b + 255) & ~(size_t)255; }
-int pq_chunks(int k_t) { return (k_t + kPqChunkTiles - 1) / kPqChunkTiles; }
 int pq_mtiles(int m_rows) { return (m_rows + 127) / 128 * 8; }   // whole 128-row blocks
 
 // The pre-pass's buffers in a workspace (nullptr: their total size)
-size_t pq_layout(void* ws, int tensors, int n_tr, int k_t, int m_rows, PqX* x) {
-  const size_t mt = pq_mtiles(m_rows), ch = pq_chunks(k_t), tr = (size_t)tensors * n_tr;
+size_t pq_layout(void* ws, int kind, int tensors, int n_tr, int k_t, int m_rows, PqX* x) {
+  const size_t mt = pq_mtiles(m_rows), tr = (size_t)tensors * n_tr;
+  const size_t ch = kind == Q4NX_KIND_Q4 ? pq_chunks<4>(k_t) : pq_chunks<8>(k_t);
   size_t off = 0;
   auto take = [&](size_t bytes) {
     uint8_t* b = (uint8_t*)ws + off;
@@ -800,86 +970,127 @@ size_t pq_layout(void* ws, int tensors, int n_tr, int k_t, int m_rows, PqX* x) {
   };
   x->xt = (u32x4_t*)take(mt * (k_t * 8 + ch * 2) * 1024 + kPqSlack);
   x->u = (u32x4_t*)take(tr * ch * 4 * 1024);
-  x->scale = (uint2*)take(tr * k_t * 1024);
+  x->scale = (uint2*)take(kind == Q4NX_KIND_Q4 ? tr * k_t * 1024 : 0);
   x->xshift = (int*)take(mt * 16 * 4);
   x->wshift = (int*)take(tr * 32 * 4);
   return off;
 }
 
-template <int OP, int MT, int RT, int WN, int WK, int RING, int OCC>
-void pq_go(const GemmArgs& a, const PqX& x, hipStream_t st) {
-  constexpr int ring = WK * RING * MT * 1024 + WN * WK * RT * 2 * kPqHalf;
+template <int KIND, int OP, int MT, int RT, int WN, int WK, int RING, int OCC>
+void pq_go(const GemmArgs& a, PqX x, hipStream_t st) {
+  constexpr int ring = WK * RING * MT * 1024 + WN * WK * RT * 2 * kPqHalf<KIND>;
   constexpr int red = (WK - 1) * WN * RT * MT * 2 * 1024;
   constexpr int lds = ring > red ? ring : red;
   static_assert(lds <= 160 * 1024);
   const int units = OP == GOP_PLAIN ? (a.n_tr[0] + RT - 1) / RT : a.n_tr[0];
-  const dim3 grid((unsigned)((units + WN - 1) / WN), (unsigned)((a.m_rows + 16 * MT - 1) / (16 * MT)));
-  hipLaunchKernelGGL((pq_kernel<OP, MT, RT, WN, WK, RING, OCC>), grid, dim3(64 * WN * WK), lds, st, a, x);
+  x.m_blocks = (a.m_rows + 16 * MT - 1) / (16 * MT);
+  x.c_groups = (units + WN - 1) / WN;
+  // Weights beyond the eight L2s (4 MB each) would be read from memory again for every row block.
+  // The dispatcher deals workgroups to the XCDs in turn, so each XCD then takes an eighth of the
+  // tiles, all row blocks of a group of columns before the next group. 512 x 248320 x 1024 (q8)
+  // 620 -> 562 us, 102 x 163200 x 2048 (q4) 146 -> 138; smaller weights stay in column order:
+  // 1000 x 2560 x 8192 (q4) 73, rows first 82.
+  x.rows_first = (size_t)a.n_tr[0] * (OP == GOP_PLAIN ? 1 : 2) * a.k_t * GemmFmt<KIND>::kTile > (32u << 20);
+  const int tiles = x.c_groups * x.m_blocks;
+  const dim3 grid((unsigned)((tiles + 7) / 8 * 8));
+  hipLaunchKernelGGL((pq_kernel<KIND, OP, MT, RT, WN, WK, RING, OCC>), grid, dim3(64 * WN * WK),
+                     lds, st, a, x);
+}
+
+template <int KIND, bool NORM>
+void pq_prep(const GemmArgs& a, const PqX& x, int tensors, hipStream_t st) {
+  const int tile_rows = a.n_tr[0] * tensors;
+  const auto go = [&](auto rows, auto threads) {
+    constexpr int ROWS = decltype(rows)::value, NT = decltype(threads)::value;
+    hipLaunchKernelGGL((pq_prep_kernel<KIND, NORM, 2, NT, ROWS>),
+                       dim3((unsigned)((a.m_rows + ROWS - 1) / ROWS + tile_rows)), dim3(NT), 0, st,
+                       a, x, tile_rows);
+  };
+  if (a.k_t <= 4) go(std::integral_constant<int, 4>{}, std::integral_constant<int, 256>{});
+  else if (a.k_t <= 16) go(std::integral_constant<int, 1>{}, std::integral_constant<int, 256>{});
+  else go(std::integral_constant<int, 1>{}, std::integral_constant<int, 512>{});
 }
 
 }  // namespace
 
-size_t pq_ws_bytes(int op, int n_tile_rows, int k_t, int m_rows) {
+size_t pq_ws_bytes(int kind, int op, int n_tile_rows, int k_t, int m_rows) {
   PqX x;
-  return pq_layout(nullptr, op == GOP_GATEUP ? 2 : 1, n_tile_rows, k_t, m_rows, &x);
+  return pq_layout(nullptr, kind, op == GOP_GATEUP ? 2 : 1, n_tile_rows, k_t, m_rows, &x);
 }
 
-bool pq_use(int kind, int op, const GemmArgs& a) {
-  if (kind != Q4NX_KIND_Q4 || op == GOP_QKV || a.m_rows < kPqRows || a.argmax_keys != nullptr)
-    return false;
-  // [gate, up] stores pairs of bf16 outputs as one word
-  return op == GOP_PLAIN || (Q4NX_ALIGNED(a.h_out, 4) && a.h_stride % 2 == 0);
+bool pq_use(int op, const GemmArgs& a) {
+  if (op == GOP_QKV || a.m_rows < kPqRows || a.argmax_keys != nullptr) return false;
+  // a lane's offset in its 16 rows has 32 bits; [gate, up] stores pairs of bf16 as one word
+  constexpr int64_t kMaxStride = 1 << 25;
+  if (op == GOP_PLAIN) return a.y_stride < kMaxStride;
+  return a.h_stride < kMaxStride && Q4NX_ALIGNED(a.h_out, 4) && a.h_stride % 2 == 0;
 }
 
-void pq_launch(int op, const GemmArgs& a, void* ws, hipStream_t st) {
-  PqX x;
-  const int tensors = op == GOP_GATEUP ? 2 : 1;
-  pq_layout(ws, tensors, a.n_tr[0], a.k_t, a.m_rows, &x);
-  const dim3 pg((unsigned)(a.m_rows + a.n_tr[0] * tensors)), pb(kPrepThreads);
-  if (a.norm_w != nullptr) {
-    if (a.k_t <= 16) hipLaunchKernelGGL((pq_prep_kernel<true, 2>), pg, pb, 0, st, a, x);
-    else hipLaunchKernelGGL((pq_prep_kernel<true, 4>), pg, pb, 0, st, a, x);
-  } else {
-    if (a.k_t <= 16) hipLaunchKernelGGL((pq_prep_kernel<false, 2>), pg, pb, 0, st, a, x);
-    else hipLaunchKernelGGL((pq_prep_kernel<false, 4>), pg, pb, 0, st, a, x);
-  }
-  // Tile by the workgroups it gives a chip of 256 CUs: the largest that fills it. Measured over
-  // K x N of 512 x 1024 to 12288 x 4096 and 65 to 3000 rows; us at the side of each line where
-  // the two are closest (N x K, rows):
+// Tile by the workgroups it gives a chip of 256 CUs, two on each: the largest that fills it.
+// Measured over N x K of 512 x 1024 to 12288 x 4096 (q8: to 248320 x 1024) and 65 to 3000 rows; us
+// at the side of each line where the two are closest (N x K, rows):
+template <int KIND>
+static void pq_plain(const GemmArgs& a, const PqX& x, hipStream_t st) {
   const auto wgs = [&](int rows, int trs) {
     return ((a.m_rows + rows - 1) / rows) * ((a.n_tr[0] + trs - 1) / trs);
   };
-  if (op == GOP_PLAIN) {
+  const int w64 = wgs(64, 4);
+  if constexpr (KIND == 4) {
     // 128 rows x 8 tile-rows against 64 x 4: 8192 x 2560, 1000 rows (256) 57 / 61, 640 rows
     // (160) 53 / 47; a short K does not repay the larger block's epilogue (6144 x 1024, 1500
     // rows (288) 44 / 38), and with fewer rows than the block has the others are as fast and add
     // up in shorter chains (the error against 64 bits 1.2e-7, not 2.8e-7)
     const int w0 = a.m_rows < 128 ? 0 : wgs(128, 8);
-    if (w0 >= 512 || (w0 >= 240 && a.k_t >= 8)) pq_go<GOP_PLAIN, 8, 2, 4, 1, 4, 2>(a, x, st);
+    if (w0 >= 512 || (w0 >= 240 && a.k_t >= 8)) return pq_go<4, GOP_PLAIN, 8, 2, 4, 1, 4, 2>(a, x, st);
     // 64 x 4 against 64 x 2 with K in two parts: 2560 x 8192, 1500 rows (480) 90 / 99, 1000 rows
     // (320) 80 / 72
-    else if (wgs(64, 4) >= 440) pq_go<GOP_PLAIN, 4, 1, 4, 1, 8, 2>(a, x, st);
-    // two parts against four: 2560 x 8192, 400 rows (280) 50 / 56, 256 rows (160) 40 / 36
-    else if (wgs(64, 2) > 256) pq_go<GOP_PLAIN, 4, 1, 2, 2, 4, 2>(a, x, st);
-    // 64 x 2 in four parts against 32 x 2: 2560 x 8192, 256 rows (160) 36 / 48, 192 rows (120)
-    // 35 / 31
-    else if (wgs(64, 2) >= 160) pq_go<GOP_PLAIN, 4, 1, 2, 4, 4, 2>(a, x, st);
-    // 32 x 2 in four parts against 32 x 1 in eight: 2560 x 2560, 128 rows (320) 16 / 22, 96 rows
-    // (240) 16 / 14
-    else if (wgs(32, 1) > 256) pq_go<GOP_PLAIN, 2, 1, 2, 4, 8, 2>(a, x, st);
-    else pq_go<GOP_PLAIN, 2, 1, 1, 8, 4, 2>(a, x, st);
+    if (w64 >= 440) return pq_go<4, GOP_PLAIN, 4, 1, 4, 1, 8, 2>(a, x, st);
   } else {
-    // 128 rows x 4 pairs against 64 x 2 in two parts: 8192 x 2560, 400 rows (256) 55 / 64, 192
-    // rows (128) 51 / 39
-    if (wgs(128, 4) >= 192) pq_go<GOP_GATEUP, 8, 2, 4, 1, 4, 2>(a, x, st);
-    // 64 x 2 against 32 x 2 in four parts: 2560 x 8192, 256 rows (160) 58 / 70, 192 rows (120)
-    // 58 / 44
-    else if (wgs(64, 2) >= 160) pq_go<GOP_GATEUP, 4, 2, 2, 2, 4, 2>(a, x, st);
-    // 32 x 2 against 32 x 1 in eight parts: 2560 x 2560, 128 rows (320) 23 / 28, 96 rows (240)
-    // 22 / 18
-    else if (wgs(32, 1) > 256) pq_go<GOP_GATEUP, 2, 2, 2, 4, 4, 2>(a, x, st);
-    else pq_go<GOP_GATEUP, 2, 2, 1, 8, 4, 2>(a, x, st);
+    // 128 rows x 4 tile-rows (eight would take the LDS of both workgroups of a CU) against the
+    // next: 8192 x 2560, 1000 rows (512) 68 / 79, 768 rows (384) 65 / 65, 640 rows (320) 64 / 60
+    if (wgs(128, 4) >= 384) return pq_go<8, GOP_PLAIN, 8, 1, 4, 1, 4, 2>(a, x, st);
+    // 64 x 4 when it fills the chip once, against 64 x 2 with K in two parts: 8192 x 2560, 400
+    // rows (448) 40 / 43, 320 rows (320) 39 / 37, 640 rows (640) 62 / 60
+    if (w64 >= 440 && w64 <= 512) return pq_go<8, GOP_PLAIN, 4, 1, 4, 1, 8, 2>(a, x, st);
   }
+  // two parts against four: 2560 x 8192, 400 rows (280) q4 50 / 56, q8 61 / 68, 256 rows (160)
+  // q4 40 / 36, q8 46 / 40
+  if (wgs(64, 2) > 256) return pq_go<KIND, GOP_PLAIN, 4, 1, 2, 2, 4, 2>(a, x, st);
+  // 64 x 2 in four parts against 32 x 2: 2560 x 8192, 256 rows (160) q4 36 / 48, q8 40 / 52, 192
+  // rows (120) q4 35 / 31, q8 39 / 32
+  if (wgs(64, 2) >= 160) return pq_go<KIND, GOP_PLAIN, 4, 1, 2, 4, 4, 2>(a, x, st);
+  // 32 x 2 in four parts against 32 x 1 in eight: 2560 x 2560, 128 rows (320) q4 16 / 22, q8 16 /
+  // 21, 96 rows (240) q4 16 / 14, q8 16 / 14
+  if (wgs(32, 1) > 256) return pq_go<KIND, GOP_PLAIN, 2, 1, 2, 4, 8, 2>(a, x, st);
+  pq_go<KIND, GOP_PLAIN, 2, 1, 1, 8, 4, 2>(a, x, st);
+}
+
+static void pq_gateup(const GemmArgs& a, const PqX& x, hipStream_t st) {
+  const auto wgs = [&](int rows, int trs) {
+    return ((a.m_rows + rows - 1) / rows) * ((a.n_tr[0] + trs - 1) / trs);
+  };
+  // 128 rows x 4 pairs against 64 x 2 in two parts: 8192 x 2560, 400 rows (256) 55 / 64, 192
+  // rows (128) 51 / 39
+  if (wgs(128, 4) >= 192) return pq_go<4, GOP_GATEUP, 8, 2, 4, 1, 4, 2>(a, x, st);
+  // 64 x 2 against 32 x 2 in four parts: 2560 x 8192, 256 rows (160) 58 / 70, 192 rows (120)
+  // 58 / 44
+  if (wgs(64, 2) >= 160) return pq_go<4, GOP_GATEUP, 4, 2, 2, 2, 4, 2>(a, x, st);
+  // 32 x 2 against 32 x 1 in eight parts: 2560 x 2560, 128 rows (320) 23 / 28, 96 rows (240)
+  // 22 / 18
+  if (wgs(32, 1) > 256) return pq_go<4, GOP_GATEUP, 2, 2, 2, 4, 4, 2>(a, x, st);
+  pq_go<4, GOP_GATEUP, 2, 2, 1, 8, 4, 2>(a, x, st);
+}
+
+void pq_launch(int kind, int op, const GemmArgs& a, void* ws, hipStream_t st) {
+  PqX x;
+  const int tensors = op == GOP_GATEUP ? 2 : 1;
+  pq_layout(ws, kind, tensors, a.n_tr[0], a.k_t, a.m_rows, &x);
+  const bool norm = a.norm_w != nullptr;
+  if (kind == Q4NX_KIND_Q8) norm ? pq_prep<8, true>(a, x, tensors, st) : pq_prep<8, false>(a, x, tensors, st);
+  else norm ? pq_prep<4, true>(a, x, tensors, st) : pq_prep<4, false>(a, x, tensors, st);
+  if (op == GOP_GATEUP) pq_gateup(a, x, st);
+  else if (kind == Q4NX_KIND_Q4) pq_plain<4>(a, x, st);
+  else pq_plain<8>(a, x, st);
 }
 
 }  // namespace q4nx

@@ -324,7 +324,10 @@ def _free_minima(raw, rng):
 
 
 @pytest.mark.parametrize("m,n,k", [
-    (65, 32, 256),        # 32 x 1: one tile-row, seven of eight K parts empty
+    (65, 32, 768),        # 32 x 1: one tile-row, five of eight K parts empty
+    (66, 64, 1024),       # the pre-pass's last row length of a wave per row, of 256 threads, and
+    (67, 64, 4096),       # the first of 512
+    (67, 64, 4352),
     (80, 544, 2816),      # 32 x 1: 11 K-tiles over eight parts of two, the last ones empty
     (129, 2080, 768),     # 32 x 2 (325 workgroups of 32 x 1): a last workgroup with one tile-row
     (257, 2080, 1280),    # 64 x 2 in four parts: five K-tiles in parts of two, one empty
@@ -352,11 +355,89 @@ def test_gemm_fp16_operands_parity(dev, m, n, k):
     assert ((ssq.double() - want).abs() <= 16 * 2.0 ** -24 * want).all()
 
 
+@pytest.mark.parametrize("m,n,k", [
+    (65, 32, 768),        # 32 x 1: one tile-row, five of eight K parts empty
+    (66, 64, 1024),       # the pre-pass's last row length of a wave per row, of 256 threads, and
+    (67, 64, 4096),       # the first of 512
+    (67, 64, 4352),
+    (80, 544, 2816),      # 32 x 1: 11 K-tiles over eight parts of two, the last ones empty
+    (129, 2080, 768),     # 32 x 2: a last workgroup with one tile-row
+    (257, 2080, 1280),    # 64 x 2 in four parts: five K-tiles in parts of two, one empty
+    (449, 2592, 768),     # 64 x 2 in two parts, ragged rows
+    (1500, 2464, 256),    # 64 x 4 (480 workgroups): one K-tile, fewer steps than the ring's
+    (2900, 2208, 1024),   # 128 x 4, ragged rows, a last workgroup of one tile-row
+    (70, 131104, 256),    # 128 x 4, row blocks first: weights beyond the L2s, 1025 groups (no
+                          # multiple of eight), one tile-row in the last
+    (130, 66592, 512),    # the same with two row blocks
+    (130, 128, 8448),     # rows longer than the pre-pass keeps in registers
+])
+def test_gemm_q8_fp16_operands_parity(dev, m, n, k):
+    """q8 on every tile of the fp16-operand kernel and on both orders of its workgroups."""
+    raw, rng = _tiles("q8", n, k, 151 + m)
+    x = synth.random_bf16(rng, (m, k))
+    res = rng.standard_normal((m, n)).astype(np.float32)
+    w, xd, rd = _dev_u8(raw, dev), _dev_bf16(x, dev), torch.from_numpy(res).to(dev)
+    y = ops.gemm(w, "q8", xd, n // 32, k // 256, residual=rd)
+    rows = np.unique(np.concatenate([np.arange(0, m, max(1, m // (48 if n < 4096 else 4))), [m - 1]]))
+    ref = qo.gemv(raw, "q8", x[rows], n // 32, k // 256, acc=np.float64) + res[rows]
+    _check_rows(y.cpu().numpy()[rows], ref)
+    ssq = torch.full((m, n // 16), float("nan"), device=dev)
+    y2 = ops.gemv_ex(w, "q8", xd, n // 32, k // 256, residual=rd, ssq_out=ssq)
+    assert torch.equal(y, y2)
+    want = y2.double().view(m, -1, 16).square().sum(-1)
+    # 16 squares added in fp32: 16 roundings of 2^-24 at most
+    assert ((ssq.double() - want).abs() <= 16 * 2.0 ** -24 * want).all()
+
+
+@pytest.mark.parametrize("kind,m,n,k", [("q8", 256, 4096, 512), ("q8", 257, 4096, 512),
+                                        ("q4", 96, 2048, 512), ("q4", 97, 2048, 512),
+                                        ("q4", 200, 512, 512), ("q4", 200, 512, 768)])
+def test_gemm_short_k_either_side(dev, kind, m, n, k):
+    """Both sides of the short-K line between the batched and the fp16-operand kernel."""
+    raw, rng = _tiles(kind, n, k, 7 + m)
+    x = synth.random_bf16(rng, (m, k))
+    y = ops.gemm(_dev_u8(raw, dev), kind, _dev_bf16(x, dev), n // 32, k // 256).cpu().numpy()
+    _check_rows(y, qo.gemv(raw, kind, x, n // 32, k // 256, acc=np.float64))
+
+
+def test_gemm_q8_fp16_operands_range(dev):
+    """q8 scales over the whole bf16 exponent range between a tile's columns, zero scales, code
+    -128, rows of very different size; infinities and NaN stay in their rows."""
+    m, n, k = 72, 96, 768
+    raw, rng = _tiles("q8", n, k, 61)
+    raw = raw.copy()
+    e = (10.0 ** rng.uniform(-25, 25, (1, 1, 32))).astype(np.float32)   # one size per column
+    v = qo.bf16_to_f32(raw[:, :512].copy().view(np.uint16)).reshape(-1, 8, 32) * e
+    v[:, :, 5] = 0.0
+    raw[:, :512] = synth.f32_to_bf16_bits(v.reshape(-1, 256).astype(np.float32)).view(
+        np.uint8).reshape(-1, 512)
+    raw[:, 512::97] = 0x80
+    xf = rng.standard_normal((m, k)).astype(np.float32)
+    xf *= (10.0 ** rng.uniform(-6, 6, (m, 1))).astype(np.float32)
+    xf[3] = 0.0
+    x = qo.bf16_round(xf)
+    w, xd = _dev_u8(raw, dev), _dev_bf16(x, dev)
+    y = ops.gemm(w, "q8", xd, n // 32, k // 256).cpu().numpy().astype(np.float64)
+    ref = qo.gemv(raw, "q8", x, n // 32, k // 256, acc=np.float64)
+    assert (y[3] == 0).all() and (y[:, 5] == 0).all() and (y[:, 37] == 0).all()
+    # each output against its own terms' size, K roundings of 2^-24 at most
+    wabs = np.abs(qo.dequant_matrix(raw, "q8", n // 32, k // 256).astype(np.float64))
+    size = np.abs(qo.bf16_to_f32(x).astype(np.float64)) @ wabs.T
+    assert (np.abs(y - ref) <= k * 2.0 ** -24 * size).all()
+    bad = xd.clone()
+    bad[7, 100], bad[20, 3], bad[64, 511] = float("inf"), float("nan"), float("-inf")
+    yb = ops.gemm(w, "q8", bad, n // 32, k // 256).cpu().numpy()
+    hit = np.zeros(m, bool)
+    hit[[7, 20, 64]] = True
+    assert not np.isfinite(yb[hit]).any()
+    assert np.array_equal(yb[~hit].view(np.uint32), y[~hit].astype(np.float32).view(np.uint32))
+
+
 def test_gemm_fp16_operands_range(dev):
     """Scales over the whole bf16 exponent range between a tile's columns, zero scales and
     minima, all-zero rows and rows of very different size, exactly as the 64-bit result has
     them; an infinity or a NaN in a row of x reaches every output of that row and no other."""
-    m, n, k = 72, 96, 512
+    m, n, k = 72, 96, 768
     raw, rng = _tiles("q4", n, k, 61)
     raw = _free_minima(raw, rng)
     e = (10.0 ** rng.uniform(-25, 25, (1, 8, 32))).astype(np.float32)   # one size per column
@@ -389,6 +470,7 @@ def test_gemm_fp16_operands_range(dev):
 
 @pytest.mark.parametrize("batch,n,k,norm", [
     (65, 96, 256, False),      # 32 x 1 pairs
+    (67, 64, 4352, True),      # 512 threads per row of x
     (200, 1312, 768, True),    # 32 x 2 pairs (287 workgroups of 32 x 1)
     (300, 2080, 2816, True),   # 64 x 2 pairs in two parts
     (1300, 2464, 512, True),   # 128 x 4 pairs, ragged both ways
