@@ -41,7 +41,10 @@ namespace q4nx {
 // blocks of each group go to two workgroups, 8 apart (one XCD, so the metadata both stage
 // comes from one L2), each staging the metadata and its block's codes only and taking one
 // operand and one MFMA per tile-row and 32-K group.
-template <int KIND, int OP, int RT, int MT, int WK, int NWV, bool RB = false>
+// NORM (up to 8 rows, fused epilogues): the rows are the fp32 residual, normalised here to the bits
+// that xnorm_kernel would write -- every workgroup again, from L2 -- instead of by a launch before
+// this one (4 us at 8 rows; the line is at its dispatch).
+template <int KIND, int OP, int RT, int MT, int WK, int NWV, bool RB = false, bool NORM = false>
 __global__ __launch_bounds__(64 * NWV) void gemm_kernel(GemmArgs a) {
   constexpr int WM = NWV / WK;
   constexpr int NT = 64 * NWV;              // threads
@@ -52,6 +55,7 @@ __global__ __launch_bounds__(64 * NWV) void gemm_kernel(GemmArgs a) {
   constexpr int TW = RB ? 16 : 32;          // outputs per tile-row per workgroup
   constexpr int NW = RT * TW;               // outputs per row of X per workgroup
   static_assert(!RB || MT == 1, "row-block workgroups: one m-tile");
+  static_assert(!NORM || MT == 1, "RMSNorm prologue: one m-tile");
   static_assert(OP == GOP_PLAIN || RT == 2, "fused epilogues pair two tile-rows");
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   __shared__ int s_last;
@@ -201,8 +205,62 @@ __global__ __launch_bounds__(64 * NWV) void gemm_kernel(GemmArgs a) {
   const __amdgpu_buffer_rsrc_t xrs = make_rsrc(a.x, (uint32_t)((int64_t)a.m_rows * a.x_stride * 2));
   const uint32_t xoff = m0 + c < a.m_rows ? (uint32_t)(((int64_t)(m0 + c) * a.x_stride + 8 * s) * 2)
                                           : 0x80000000u;
+  // NORM: each wave adds up the sums of squares of every NWV-th row, in xnorm_kernel's order. The
+  // residual of a K-tile comes whole cache lines at a time (two rows of half a tile per load; rows
+  // past the batch lie outside the buffer; the operand's rows 8 to 15 repeat 0 to 7 and are never
+  // stored) and goes through the wave's slot, which the weights
+  // have not taken yet, into operand order.
+  constexpr int NROW = NORM ? (8 + NWV - 1) / NWV : 1;
+  constexpr int XROW = 272;                 // bytes of half a row there: 4 banks apart
+  static_assert(!NORM || 8 * XROW <= RT * SLOT, "the rows do not fit the staging slot");
+  __shared__ float s_inv[NORM ? 8 : 1];
+  const __amdgpu_buffer_rsrc_t hrs = make_rsrc(a.hres, (uint32_t)((int64_t)a.m_rows * a.x_stride * 4));
+  const __amdgpu_buffer_rsrc_t nrs = make_rsrc(a.norm_w, (uint32_t)a.k_t * (kTileK * 2u));
+  const int n_ss = a.k_t * (kTileK / kSsqRows);
+  float4 sq[NROW][2];
+  if constexpr (NORM) {
+#pragma unroll
+    for (int i = 0; i < NROW; ++i)
+      ssq_load<2>(a.ssq_in + (int64_t)min(wave + NWV * i, a.m_rows - 1) * n_ss, l, n_ss, sq[i]);
+    asm volatile("" ::: "memory");
+  }
   u32x4_t xa[8][MT];
+  v4i_t xh[NORM ? 8 : 1];
+  i32x2_t xw[2];
+  auto hload = [&](int kt) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const uint32_t o = (uint32_t)(kt * 1024 + h * 512 + 16 * (l & 31));
+      xw[h] = __builtin_bit_cast(i32x2_t, __builtin_amdgcn_raw_buffer_load_b64(nrs, (int)(o >> 1), 0, 0));
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        xh[4 * h + i] = __builtin_amdgcn_raw_buffer_load_b128(
+            hrs, (int)(o + (uint32_t)(2 * i + (l >> 5)) * (uint32_t)a.x_stride * 4u), 0, 0);
+    }
+  };
+  auto hnorm = [&] {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float inv = s_inv[2 * i + (l >> 5)];
+        const v4i_t v = xh[4 * h + i];
+        const uint32_t w0 = (uint32_t)xw[h].x, w1 = (uint32_t)xw[h].y;
+        *(uint2*)(slot + (2 * i + (l >> 5)) * XROW + (l & 31) * 8) =
+            make_uint2(pack_bf16x2((__int_as_float(v.x) * inv) * bf16lo(w0),
+                                   (__int_as_float(v.y) * inv) * bf16hi(w0)),
+                       pack_bf16x2((__int_as_float(v.z) * inv) * bf16lo(w1),
+                                   (__int_as_float(v.w) * inv) * bf16hi(w1)));
+      }
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb)
+        xa[4 * h + kb][0] = *(const u32x4_t*)(slot + (c & 7) * XROW + kb * 64 + s * 16);
+      __builtin_amdgcn_wave_barrier();
+    }
+  };
   auto xload = [&](int kt) {
+    if constexpr (NORM) return hload(kt);
 #pragma unroll
     for (int kb = 0; kb < 8; ++kb)
 #pragma unroll
@@ -219,6 +277,9 @@ __global__ __launch_bounds__(64 * NWV) void gemm_kernel(GemmArgs a) {
   // the first tile's weights, also in a wave with no tile (a clamped tile, never used): no
   // branch around the first loads, so the compiler's counts for the waits below stay exact
   // (after a branch they fall back to waiting for every load)
+  // (NORM: the rows first, normalised while the weights arrive)
+  if (NORM) xload(kbeg + wk);
+  asm volatile("" ::: "memory");
   u32x4_t pf[RT][NLD];
 #pragma unroll
   for (int r = 0; r < RT; ++r)
@@ -230,7 +291,7 @@ __global__ __launch_bounds__(64 * NWV) void gemm_kernel(GemmArgs a) {
   // latency followed the weights' in every one-tile wave, which is every wave of a decode
   // batch's launches; issued ahead of the weights they delayed the weight stream)
   // (a wave with no tile loads bytes it never uses: inside the rows' buffer, or zeros past it)
-  if (MT == 1) xload(kbeg + wk);
+  if (MT == 1 && !NORM) xload(kbeg + wk);
   asm volatile("" ::: "memory");
   if constexpr (PF_POS) {
     if (seg != 2) {
@@ -245,17 +306,29 @@ __global__ __launch_bounds__(64 * NWV) void gemm_kernel(GemmArgs a) {
     }
   }
 
-  for (int it = 0; it < n_it; ++it) {
+  if constexpr (NORM) {
+#pragma unroll
+    for (int i = 0; i < NROW; ++i) {
+      const float r = rms_inv(wave_sum(ssq_lane_sum<2>(sq[i], l, n_ss)), a.k_t * kTileK, a.eps);
+      if (l == 0 && wave + NWV * i < 8) s_inv[wave + NWV * i] = r;
+    }
+    // (the loads in flight stay in flight: only LDS is waited for)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  }
+  for (int it = 0; it < (NORM ? min(n_it, 1) : n_it); ++it) {
     const int kt = kbeg + wk + it * WK;
+    if constexpr (NORM) hnorm();
 #pragma unroll
     for (int r = 0; r < RT; ++r)
 #pragma unroll
       for (int i = 0; i < NLD; ++i) *(u32x4_t*)(slot + r * SLOT + 16 * (64 * i + l)) = pf[r][i];
     // activations of this tile first, then the next tile's weights: the in-order load
     // counter then lets the arithmetic start before the next tile arrives
-    if (MT != 1 || it > 0) xload(kt);
+    if (!NORM && (MT != 1 || it > 0)) xload(kt);
     asm volatile("" ::: "memory");
-    if (it + 1 < n_it) {   // wave-uniform: a one-iteration wave issues no second tile
+    if (!NORM && it + 1 < n_it) {   // wave-uniform: a one-iteration wave issues no second tile
       const size_t off = (size_t)(kt + WK) * TB;
 #pragma unroll
       for (int r = 0; r < RT; ++r)
@@ -541,6 +614,7 @@ __global__ __launch_bounds__(256) void xnorm_kernel(const float* __restrict__ h,
 struct GemmPlan {
   int rt, mt, wk, nwv, ksplit, kpp, mb, m_blocks, groups;
   bool rb;     // one m-tile: a workgroup per 16-row block of each group
+  bool norm;   // the kernel normalises its rows itself
   int units;   // workgroups along N (groups, or twice that with rb)
 };
 
@@ -610,6 +684,16 @@ static GemmPlan plan_gemm(int kind, int op, int n_units, int k_t, int m_rows, co
         break;
       }
   }
+  // Two m-tiles, at most a workgroup per CU (12288 x 4096 has 1.5: 32 rows 23.0 / 25.0): eight
+  // waves, where they find work -- with up to 32 rows all eight
+  // split K, so a part needs more K-tiles than waves (us, four / eight waves: [gate, up] 8192 x
+  // 2560, 32 rows 15.4 / 13.7, q8 8192 x 2560 12.2 / 11.7, but 2560 x 2560 in parts of four 7.6 /
+  // 8.1); with more, four of them do (q4 2560 x 8192, 33 rows 18.0 / 14.9, 64 rows 21.0 / 19.1,
+  // 1024 x 2048 9.7 / 8.8; q8's larger slots leave nothing: 8192 x 2560, 64 rows 18.4 / 18.6)
+  if (p.mt == 2 && p.wk > 1 && wgs <= 256 && (p.wk == 4 ? p.kpp > 8 : kind == Q4NX_KIND_Q4)) {
+    p.nwv = 8;
+    p.wk *= 2;
+  }
   // Row-block workgroups when the doubled grid still fits one workgroup per CU (measured at
   // 8 rows: the o-projection 2560->2560, 80 -> 160 workgroups, 6.79 -> 5.97 us and batch-8
   // decode 3736 -> 3790 tok/s; launches that already fill the chip lose, as each group's
@@ -636,7 +720,7 @@ static size_t gemm_split_bytes(const GemmPlan& p) {
   return part ? Q4NX_WS_COUNTER_BYTES + align256(part) : 0;
 }
 
-template <int KIND, int OP, int RT, int MT, int WK, int NWV = 4>
+template <int KIND, int OP, int RT, int MT, int WK, int NWV = 4, bool NORM = false>
 static void gemm_launch_t(const GemmArgs& a, const GemmPlan& p, hipStream_t st) {
   constexpr int lds = NWV * RT * GemmFmt<KIND>::kSlot;
   static_assert(NWV * 16 * MT * RT * 32 * 4 <= lds, "reduction does not fit the staging slots");
@@ -645,23 +729,32 @@ static void gemm_launch_t(const GemmArgs& a, const GemmPlan& p, hipStream_t st) 
     if (p.rb) {
       constexpr int lds_rb = NWV * RT * GemmFmt<KIND>::kSlotRB;
       static_assert(NWV * 16 * RT * 16 * 4 <= lds_rb, "reduction does not fit the staging slots");
-      hipLaunchKernelGGL((gemm_kernel<KIND, OP, RT, MT, WK, NWV, true>), grid, dim3(64 * NWV),
+      hipLaunchKernelGGL((gemm_kernel<KIND, OP, RT, MT, WK, NWV, true, NORM>), grid, dim3(64 * NWV),
                          lds_rb, st, a);
       return;
     }
   }
-  hipLaunchKernelGGL((gemm_kernel<KIND, OP, RT, MT, WK, NWV>), grid, dim3(64 * NWV), lds, st, a);
+  hipLaunchKernelGGL((gemm_kernel<KIND, OP, RT, MT, WK, NWV, false, NORM>), grid, dim3(64 * NWV), lds, st, a);
 }
 
 template <int KIND, int OP>
 static void gemm_launch_op(const GemmArgs& a, const GemmPlan& p, hipStream_t st) {
   constexpr int R1 = OP == GOP_PLAIN ? 1 : 2;
+  if constexpr (OP != GOP_PLAIN)
+    if (p.norm) {
+      if (p.nwv == 8) return gemm_launch_t<KIND, OP, R1, 1, 8, 8, true>(a, p, st);
+      if (p.nwv == 10) return gemm_launch_t<KIND, OP, R1, 1, 10, 10, true>(a, p, st);
+      return gemm_launch_t<KIND, OP, R1, 1, 4, 4, true>(a, p, st);
+    }
   if (p.mt == 1 && p.nwv == 8) gemm_launch_t<KIND, OP, R1, 1, 8, 8>(a, p, st);
   else if (p.mt == 1 && p.nwv == 10) gemm_launch_t<KIND, OP, R1, 1, 10, 10>(a, p, st);
   else if (p.mt == 1 && p.nwv == 16) {
     if constexpr (KIND == 4 && OP == GOP_PLAIN) gemm_launch_t<KIND, OP, 1, 1, 16, 16>(a, p, st);
   } else if (p.mt == 1) gemm_launch_t<KIND, OP, R1, 1, 4>(a, p, st);
-  else if (p.wk == 4) gemm_launch_t<KIND, OP, (OP == GOP_PLAIN ? 1 : 2), 2, 4>(a, p, st);
+  else if (p.nwv == 8 && p.wk == 8) gemm_launch_t<KIND, OP, R1, 2, 8, 8>(a, p, st);
+  else if (p.nwv == 8) {
+    if constexpr (KIND == 4) gemm_launch_t<KIND, OP, R1, 2, 4, 8>(a, p, st);
+  } else if (p.wk == 4) gemm_launch_t<KIND, OP, (OP == GOP_PLAIN ? 1 : 2), 2, 4>(a, p, st);
   else if (p.wk == 2) gemm_launch_t<KIND, OP, (OP == GOP_PLAIN ? 1 : 2), 2, 2>(a, p, st);
   else if (OP != GOP_PLAIN || p.rt == 2) gemm_launch_t<KIND, OP, 2, 2, 1>(a, p, st);
   else if constexpr (OP == GOP_PLAIN) gemm_launch_t<KIND, OP, 1, 2, 1>(a, p, st);
@@ -726,6 +819,13 @@ int mfma_launch(int kind, int op, GemmArgs& a, int n_units, void* ws, size_t ws_
     Q4NX_REQUIRE(K / kSsqRows <= 512, Q4NX_ERR_SHAPE, "%s: RMSNorm prologue supports K <= 8192", what);
     uint16_t* xn = a.xn_out;
     int64_t xs = a.x_stride;
+    // The kernel itself normalises the rows of a decode batch where nobody asks for them, every
+    // wave has at most one K-tile and the workgroups (each normalises all rows) are few. With
+    // xnorm_kernel before / in the kernel, us at 8 rows: [gate, up] 2048 x 1024 (64 groups) 6.8 /
+    // 5.5, 4096 x 2048 (128) 9.0 / 7.7, 8192 x 2560 (256) 12.3 / 12.8, 10240 x 2560 (320) 17.8 /
+    // 20.5
+    p.norm = xn == nullptr && a.m_rows <= 8 && op != GOP_PLAIN && p.groups <= 128 && p.kpp <= p.wk &&
+             (int64_t)a.m_rows * xs * 4 < ((int64_t)1 << 31);
     if (xn == nullptr) {
       Q4NX_REQUIRE(ws_ok && ws_bytes >= Q4NX_WS_COUNTER_BYTES + align256(split) + xn_b,
                    Q4NX_ERR_WS, "%s: workspace of %zu bytes needed for the normalised rows",
@@ -733,10 +833,12 @@ int mfma_launch(int kind, int op, GemmArgs& a, int n_units, void* ws, size_t ws_
       xn = (uint16_t*)((uint8_t*)ws + Q4NX_WS_COUNTER_BYTES + align256(split));
       xs = K;
     }
-    hipLaunchKernelGGL(xnorm_kernel, dim3(a.m_rows), dim3(256), 0, st, a.hres, a.x_stride,
-                       a.ssq_in, a.norm_w, a.eps, K, xn, xs);
-    a.x = xn;
-    a.x_stride = xs;
+    if (!p.norm) {
+      hipLaunchKernelGGL(xnorm_kernel, dim3(a.m_rows), dim3(256), 0, st, a.hres, a.x_stride,
+                         a.ssq_in, a.norm_w, a.eps, K, xn, xs);
+      a.x = xn;
+      a.x_stride = xs;
+    }
   }
   // one m-tile reads x through a buffer resource with 32-bit byte offsets
   Q4NX_REQUIRE(p.mt != 1 || (int64_t)a.m_rows * a.x_stride * 2 < ((int64_t)1 << 31),

@@ -237,6 +237,61 @@ def test_mfma_gate_up_swiglu(dev, mfma, batch, norm):
     assert_bf16_close(bits(hout), do.swiglu_from_raw(raw_np[:, :inter], raw_np[:, inter:]))
 
 
+@pytest.mark.parametrize("batch,hid,inter", [
+    (2, 256, 32),       # one K-tile: all waves but one without work; one group
+    (3, 1024, 1056),    # 33 groups, four waves
+    (8, 2048, 4096),    # 128 groups, eight waves: the last that normalise in the kernel
+    (8, 2048, 4128),    # 129 groups: the first with a launch for it
+    (7, 2560, 2048),    # row-block workgroups of ten waves
+    (5, 2816, 2048),    # 11 K-tiles in parts
+    (9, 2560, 2048),    # past eight rows
+])
+def test_mfma_norm_in_kernel_same_bits(dev, mfma, batch, hid, inter):
+    """[RMSNorm, gate, up, SwiGLU] and [RMSNorm, q, k, v, RoPE] with the normalised rows asked for
+    (a launch of their own) and without (normalised by the contraction where the launch is small):
+    the same bits, a row of zeros and a row with an infinity included."""
+    rng = np.random.default_rng(170 + batch + hid)
+    kt = hid // 256
+    d = lambda a: torch.from_numpy(a.reshape(-1)).to(dev)
+    x, ss, nw, _ = normed_input(rng, batch, hid, dev)
+    x[0] = 0.0
+    x[1, 5] = float("inf")
+    ss = x.view(batch, -1, 16).square().sum(-1).contiguous()
+    xn = torch.zeros((batch, hid), dtype=torch.bfloat16, device=dev)
+    wg, wu = d(synth.q4_tiles(rng, inter, hid)), d(synth.q4_tiles(rng, inter, hid))
+    run = lambda **kw: ops.gate_up_swiglu(wg, wu, inter // 32, kt, x, norm_w=nw, ssq_in=ss, **kw)
+    assert np.array_equal(bits(run()), bits(run(xn_out=xn)))
+    hq, hkv, lmax = 4, 2, 16
+    wq, wk, wv = (d(synth.q4_tiles(rng, h * 64, hid)) for h in (hq, hkv, hkv))
+    pos = torch.from_numpy(rng.integers(0, lmax, batch).astype(np.int32)).to(dev)
+    tab = ops.rope_table(lmax, 64, 10000.0)
+    got = []
+    for kw in ({}, {"xn_out": xn}):
+        kc = torch.zeros((batch, hkv, lmax, 64), dtype=torch.bfloat16, device=dev)
+        vc = torch.zeros_like(kc)
+        q = ops.qkv_rope(wq, wk, wv, hq, hkv, kt, x, pos, tab, kc, vc, norm_w=nw, ssq_in=ss, **kw)
+        got.append([bits(t) for t in (q, kc, vc)])
+    assert all(np.array_equal(a, b) for a, b in zip(*got))
+
+
+@pytest.mark.parametrize("kind", ["q4", "q8"])
+@pytest.mark.parametrize("rows,n,k", [
+    (17, 1056, 2304),    # nine K-tiles on eight waves that split K
+    (32, 512, 8192),     # the same in parts
+    (33, 544, 1280),     # two row blocks of waves, four (q4) on K
+    (64, 8192, 768),     # 256 groups, fewer K-tiles than waves
+    (64, 8224, 768),     # 257: four waves
+])
+def test_mfma_eight_waves(dev, mfma, kind, rows, n, k):
+    """17 to 64 rows on the eight-wave workgroups and at the edges of their rule."""
+    rng = np.random.default_rng(200 + rows + k)
+    raw = (synth.q4_tiles if kind == "q4" else synth.q8_tiles)(rng, n, k)
+    raw = raw.reshape(-1, qo.Q4_TILE_BYTES if kind == "q4" else qo.Q8_TILE_BYTES)
+    x = synth.random_bf16(rng, (rows, k))
+    y = ops.gemm(torch.from_numpy(raw.reshape(-1)).to(dev), kind, bf16_dev(x, dev), n // 32, k // 256)
+    rows_close(y.cpu().numpy(), qo.gemv(raw, kind, x, n // 32, k // 256, acc=np.float64), REL, COS)
+
+
 @pytest.mark.parametrize("parts", [1, 3])
 def test_mfma_rowblock_split_fused(dev, parts):
     """The fused epilogues on row-block workgroups (two per group: 32 [gate, up] groups and
