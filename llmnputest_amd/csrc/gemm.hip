@@ -684,13 +684,14 @@ static GemmPlan plan_gemm(int kind, int op, int n_units, int k_t, int m_rows, co
         break;
       }
   }
-  // Two m-tiles, at most a workgroup per CU (12288 x 4096 has 1.5: 32 rows 23.0 / 25.0): eight
+  // Two m-tiles, at most a workgroup per CU (12288 x 4096 has 1.5: 32 rows 23.0 / 25.0; [gate, up]
+  // 4096 x 2048 in three parts, 33 rows 17 / 22): eight
   // waves, where they find work -- with up to 32 rows all eight
   // split K, so a part needs more K-tiles than waves (us, four / eight waves: [gate, up] 8192 x
   // 2560, 32 rows 15.4 / 13.7, q8 8192 x 2560 12.2 / 11.7, but 2560 x 2560 in parts of four 7.6 /
   // 8.1); with more, four of them do (q4 2560 x 8192, 33 rows 18.0 / 14.9, 64 rows 21.0 / 19.1,
   // 1024 x 2048 9.7 / 8.8; q8's larger slots leave nothing: 8192 x 2560, 64 rows 18.4 / 18.6)
-  if (p.mt == 2 && p.wk > 1 && wgs <= 256 && (p.wk == 4 ? p.kpp > 8 : kind == Q4NX_KIND_Q4)) {
+  if (p.mt == 2 && p.wk > 1 && wgs * p.ksplit <= 256 && (p.wk == 4 ? p.kpp > 8 : kind == Q4NX_KIND_Q4)) {
     p.nwv = 8;
     p.wk *= 2;
   }
@@ -875,9 +876,15 @@ size_t q4nx_gemm_ws_bytes(int kind, int n_tile_rows, int k_tiles, int m_rows,
       m_rows < 1 || !resolve_policy_quiet(policy, &P))
     return 0;
   const size_t split = gemm_split_bytes(plan_gemm(kind, GOP_PLAIN, n_tile_rows, k_tiles, m_rows, P));
-  const size_t pq = m_rows >= kPqRows
-                        ? Q4NX_WS_COUNTER_BYTES + pq_ws_bytes(kind, GOP_PLAIN, n_tile_rows, k_tiles, m_rows) : 0;
-  return pq > split ? pq : split;
+  // a launch that fills the chip without a split: what the fp16-operand kernel keeps
+  return split ? split : q4nx_gemm_prompt_ws_bytes(kind, n_tile_rows, k_tiles, m_rows);
+}
+
+size_t q4nx_gemm_prompt_ws_bytes(int kind, int n_tile_rows, int k_tiles, int m_rows) {
+  if ((kind != Q4NX_KIND_Q4 && kind != Q4NX_KIND_Q8) || n_tile_rows < 1 || k_tiles < 1 ||
+      m_rows < kPqRows)
+    return 0;
+  return Q4NX_WS_COUNTER_BYTES + pq_ws_bytes(kind, GOP_PLAIN, n_tile_rows, k_tiles, m_rows);
 }
 
 int q4nx_gemm(int kind, const uint8_t* w, int n_tile_rows, int k_tiles, const uint16_t* x,

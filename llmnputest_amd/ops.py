@@ -197,7 +197,10 @@ def gemm(tiles: torch.Tensor, kind: str, x: torch.Tensor, n_tile_rows: int, k_ti
             raise ValueError("residual must have the shape of the output")
     ws = ws or default_workspace()
     pol = _pol(policy)
-    wp, wn = ws.get(_lib.lib().q4nx_gemm_ws_bytes(KIND[kind], n_tile_rows, k_tiles, m, pol))
+    need = _lib.lib().q4nx_gemm_ws_bytes(KIND[kind], n_tile_rows, k_tiles, m, pol)
+    if m > 64:
+        need = max(need, _lib.lib().q4nx_gemm_prompt_ws_bytes(KIND[kind], n_tile_rows, k_tiles, m))
+    wp, wn = ws.get(need)
     _lib.call("q4nx_gemm", KIND[kind], _ptr(tiles), n_tile_rows, k_tiles, _ptr(x2), x2.stride(0),
               m, _ptr(out), n, _ptr(residual), wp, wn, pol, _stream())
     return out.reshape(n) if squeeze else out
