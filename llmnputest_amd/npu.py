@@ -141,7 +141,11 @@ class NpuLmHead(torch.nn.Module):
             return self.fallback(h)
         t = time.perf_counter()
         d = self.design
-        x = h.detach().to(torch.float32).reshape(rows, -1).to(torch.bfloat16).to(d.device)
+        # bf16 rows on the device are read where they are (two conversions took 10 us of an 80 us
+        # call); anything else, and a view the kernels' 16-byte loads cannot take, is converted
+        x = h.detach().reshape(rows, -1).to(torch.bfloat16).to(d.device)
+        if not x.is_contiguous() or x.data_ptr() % 16:
+            x = x.clone(memory_format=torch.contiguous_format)
         y = ops.gemm(d.bos[0], d.meta["kind"], x, d.meta["tile_rows"], self.k // TILE_K)
         out = y.reshape(*h.shape[:-1], -1).to(h.device).to(h.dtype)
         if out.is_cuda:
