@@ -700,7 +700,7 @@ def main() -> int:
             "roofline_frac": round(dec["gbs"] / HBM_PEAK_GBS, 4),
             "cpu_baseline": dec_cpu,
         }
-        if dec_cpu is not None and dec.get("cpu") is not None:
+        if dec_cpu is not None and dec.get("cpu") is not None and dec_cpu is not dec["cpu"]:
             # the float64 oracle's own rate on the same workload, kept apart: it checks
             # results and is not a CPU decoder
             dec_cpu["float64_oracle"] = dec["cpu"]
