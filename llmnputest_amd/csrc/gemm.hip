@@ -29,6 +29,7 @@
 #include "common.h"
 #include "gemm.h"
 #include "gemm_fmt.h"
+#include "row_offset.h"
 
 namespace q4nx {
 
@@ -152,7 +153,7 @@ __global__ __launch_bounds__(64 * NWV) void gemm_kernel(GemmArgs a) {
   for (int r = 0; r < RT; ++r) wrs[r] = make_rsrc(wr[r], (uint32_t)(a.k_t * TB));
   auto wload = [&](int r, size_t off, int i) -> u32x4_t {
     if constexpr (RB && KIND == 4) {
-      const uint32_t o = ld_off[i] < 0 ? 0x80000000u : (uint32_t)(off + ld_off[i]);
+      const uint32_t o = ld_off[i] < 0 ? kOutOfRange : (uint32_t)(off + ld_off[i]);
       const v4i_t v = __builtin_amdgcn_raw_buffer_load_b128(wrs[r], (int)o, 0, 0);
       return u32x4_t{(uint32_t)v.x, (uint32_t)v.y, (uint32_t)v.z, (uint32_t)v.w};
     } else {
@@ -204,7 +205,7 @@ __global__ __launch_bounds__(64 * NWV) void gemm_kernel(GemmArgs a) {
   // a branch around those lanes' loads measured slower). Their outputs are never stored.
   const __amdgpu_buffer_rsrc_t xrs = make_rsrc(a.x, (uint32_t)((int64_t)a.m_rows * a.x_stride * 2));
   const uint32_t xoff = m0 + c < a.m_rows ? (uint32_t)(((int64_t)(m0 + c) * a.x_stride + 8 * s) * 2)
-                                          : 0x80000000u;
+                                          : kOutOfRange;
   // NORM: each wave adds up the sums of squares of every NWV-th row, in xnorm_kernel's order. The
   // residual of a K-tile comes whole cache lines at a time (two rows of half a tile per load; rows
   // past the batch lie outside the buffer; the operand's rows 8 to 15 repeat 0 to 7 and are never
@@ -227,6 +228,9 @@ __global__ __launch_bounds__(64 * NWV) void gemm_kernel(GemmArgs a) {
   u32x4_t xa[8][MT];
   v4i_t xh[NORM ? 8 : 1];
   i32x2_t xw[2];
+  uint32_t hrow[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) hrow[i] = row_offset(2 * i + (l >> 5), a.m_rows, (uint32_t)a.x_stride * 4u);
   auto hload = [&](int kt) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -235,7 +239,7 @@ __global__ __launch_bounds__(64 * NWV) void gemm_kernel(GemmArgs a) {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         xh[4 * h + i] = __builtin_amdgcn_raw_buffer_load_b128(
-            hrs, (int)(o + (uint32_t)(2 * i + (l >> 5)) * (uint32_t)a.x_stride * 4u), 0, 0);
+            hrs, (int)(hrow[i] + o), 0, 0);
     }
   };
   auto hnorm = [&] {

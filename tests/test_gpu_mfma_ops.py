@@ -274,6 +274,27 @@ def test_mfma_norm_in_kernel_same_bits(dev, mfma, batch, hid, inter):
     assert all(np.array_equal(a, b) for a, b in zip(*got))
 
 
+def test_mfma_norm_in_kernel_far_rows(dev, mfma):
+    """Two rows 0.8 GB apart, normalised by the contraction: the bits of adjacent rows. (Operand
+    rows past the batch have 32-bit offsets that would wrap to between the two.)"""
+    from llmnputest_amd import _lib
+    rng = np.random.default_rng(31)
+    batch, hid, inter, pitch = 2, 1024, 512, 200_000_000
+    d = lambda a: torch.from_numpy(a.reshape(-1)).to(dev)
+    x, ss, nw, _ = normed_input(rng, batch, hid, dev)
+    wg, wu = d(synth.q4_tiles(rng, inter, hid)), d(synth.q4_tiles(rng, inter, hid))
+    want = ops.gate_up_swiglu(wg, wu, inter // 32, hid // 256, x, norm_w=nw, ssq_in=ss)
+    far = torch.empty(batch * pitch, dtype=torch.float32, device=dev)
+    for r in range(batch):
+        far[r * pitch:r * pitch + hid] = x[r]
+    h = torch.zeros_like(want)
+    ws = ops.Workspace(4 << 20, device=dev)
+    _lib.call("q4nx_gate_up_swiglu", wg.data_ptr(), wu.data_ptr(), inter // 32, hid // 256,
+              far.data_ptr(), pitch, nw.data_ptr(), 1e-5, ss.data_ptr(), batch, h.data_ptr(), inter,
+              None, None, ws.buf.data_ptr(), ws.buf.numel(), None, ops._stream())
+    assert np.array_equal(bits(h), bits(want))
+
+
 @pytest.mark.parametrize("kind", ["q4", "q8"])
 @pytest.mark.parametrize("rows,n,k", [
     (17, 1056, 2304),    # nine K-tiles on eight waves that split K
