@@ -62,8 +62,9 @@ bool mfma_norm_fits(int k_t, int m_rows, size_t ws_bytes);
 constexpr int kPqRows = 65;
 // workspace bytes it keeps the fp16 x, sums and column terms in (past the counters)
 size_t pq_ws_bytes(int kind, int op, int n_tile_rows, int k_t, int m_rows);
-// whether a launch of op `op` described by `a` takes that kernel
-bool pq_use(int op, const GemmArgs& a);
+// whether a launch of op `op` described by `a` can take that kernel (its outputs' alignment and
+// strides; anything else is the batched kernel's, which reads and writes single values)
+bool pq_use(int kind, int op, const GemmArgs& a);
 // launches `a` on it (with its RMSNorm prologue, if any): the pre-pass over x into `ws`
 // (pq_ws_bytes of it, 256-byte aligned), then the contraction
 void pq_launch(int kind, int op, const GemmArgs& a, void* ws, hipStream_t st);

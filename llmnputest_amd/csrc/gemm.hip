@@ -807,7 +807,7 @@ int mfma_launch(int kind, int op, GemmArgs& a, int n_units, void* ws, size_t ws_
                                                                  : a.m_rows <= 96));
   // a prompt block: the fp16-operand kernel, when the workspace holds what it keeps
   // there (a K split that the policy names belongs to the batched kernel)
-  if (pq_use(op, a) && ws_ok && P.gemm_ksplit == 0 && !short_k &&
+  if (pq_use(kind, op, a) && ws_ok && P.gemm_ksplit == 0 && !short_k &&
       (a.norm_w == nullptr || (a.ssq_in != nullptr && K / kSsqRows <= 512)) &&
       ws_bytes >= Q4NX_WS_COUNTER_BYTES + pq_ws_bytes(kind, op, a.n_tr[0], a.k_t, a.m_rows)) {
     pq_launch(kind, op, a, (uint8_t*)ws + Q4NX_WS_COUNTER_BYTES, st);

@@ -1018,12 +1018,20 @@ size_t pq_ws_bytes(int kind, int op, int n_tile_rows, int k_t, int m_rows) {
   return pq_layout(nullptr, kind, op == GOP_GATEUP ? 2 : 1, n_tile_rows, k_t, m_rows, &x);
 }
 
-bool pq_use(int op, const GemmArgs& a) {
+bool pq_use(int kind, int op, const GemmArgs& a) {
   if (op == GOP_QKV || a.m_rows < kPqRows || a.argmax_keys != nullptr) return false;
-  // a lane's offset in its 16 rows has 32 bits; [gate, up] stores pairs of bf16 as one word
+  // a lane's offset in its 16 rows has 32 bits
   constexpr int64_t kMaxStride = 1 << 25;
-  if (op == GOP_PLAIN) return a.y_stride < kMaxStride;
-  return a.h_stride < kMaxStride && Q4NX_ALIGNED(a.h_out, 4) && a.h_stride % 2 == 0;
+  if (op == GOP_PLAIN) {
+    if (a.y_stride >= kMaxStride) return false;
+    // q4: a lane's two columns are adjacent and are read and written as one 8-byte pair (q8: they
+    // lie in different row blocks)
+    return kind == Q4NX_KIND_Q8 ||
+           (Q4NX_ALIGNED(a.y, 8) && Q4NX_ALIGNED(a.residual, 8) && a.y_stride % 2 == 0);
+  }
+  // pairs of bf16 as one word, pairs of fp32 as one 8-byte piece
+  return a.h_stride < kMaxStride && Q4NX_ALIGNED(a.h_out, 4) && a.h_stride % 2 == 0 &&
+         Q4NX_ALIGNED(a.raw_out, 8);
 }
 
 // Tile by the workgroups it gives a chip of 256 CUs, two on each: the largest that fills it.

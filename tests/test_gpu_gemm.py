@@ -509,3 +509,61 @@ def test_gate_up_fp16_operands(dev, batch, n, k, norm):
     want = (gv / (1 + torch.exp(-gv)) * uv)
     # one bf16 rounding (2^-9 of the value's binade) and the fp32 formula's own few ulps
     assert ((h_out.double() - want).abs() <= want.abs() * (2.0 ** -8 + 2.0 ** -20) + 1e-38).all()
+
+
+@pytest.mark.parametrize("kind", ["q4", "q8"])
+@pytest.mark.parametrize("off,odd", [(1, 0), (0, 1), (1, 1), (2, 2)])
+def test_prompt_block_outputs_at_any_float(dev, kind, off, odd):
+    """y and residual `off` floats past an aligned address, rows N + odd floats apart, as
+    q4nx_gemv_ex takes them: every row at the GEMV bar, the floats between the rows untouched. q4
+    pairs that no 8-byte access may touch give the batched kernel's bits (the call without a
+    workspace)."""
+    from llmnputest_amd import _lib
+    m, n, k = 200, 2592, 768         # (no K split on the batched kernel)
+    raw, rng = _tiles(kind, n, k, 91)
+    x = synth.random_bf16(rng, (m, k))
+    res = rng.standard_normal((m, n)).astype(np.float32)
+    w, xd = _dev_u8(raw, dev), _dev_bf16(x, dev)
+    code, ld = ops.KIND[kind], n + odd
+    rd = torch.zeros(off + m * ld, device=dev)
+    rd[off:].view(m, ld)[:, :n] = torch.from_numpy(res).to(dev)
+
+    def call(ws, out, ssq, o, stride, r):
+        _lib.call("q4nx_gemv_ex", code, w.data_ptr(), n // 32, k // 256, xd.data_ptr(), k, None, 0.0,
+                  None, m, out.data_ptr() + 4 * o, stride, r, ssq.data_ptr(), None,
+                  ws.buf.data_ptr() if ws else None, ws.buf.numel() if ws else 0, None,
+                  ops._stream())
+    ws = ops.Workspace(16 << 20, device=dev)
+    y = torch.full((off + m * ld,), -7.0, device=dev)
+    ssq = torch.zeros((m, n // 16), device=dev)
+    call(ws, y, ssq, off, ld, rd.data_ptr() + 4 * off)
+    got = y[off:].view(m, ld)
+    _check_rows(got[:, :n].cpu().numpy(),
+                qo.gemv(raw, kind, x, n // 32, k // 256, acc=np.float64) + res)
+    assert (y[:off] == -7).all() and (got[:, n:] == -7).all()
+    flat = torch.from_numpy(res).to(dev)
+    want, wssq = torch.empty((m, n), device=dev), torch.empty_like(ssq)
+    pair = kind == "q8" or (off % 2 == 0 and odd % 2 == 0)
+    call(ws if pair else None, want, wssq, 0, n, flat.data_ptr())
+    assert torch.equal(got[:, :n], want) and torch.equal(ssq, wssq)
+
+
+@pytest.mark.parametrize("off", [1, 2])
+def test_prompt_gate_up_raw_out_at_any_float(dev, off):
+    """raw_out of [gate, up] `off` floats past an aligned address: the bits of the batched kernel
+    where no 8-byte access may touch it, else those of the aligned call."""
+    from llmnputest_amd import _lib
+    m, n, k = 200, 6176, 512
+    raw, rng = _tiles("q4", n, k, 92)
+    w, xd = _dev_u8(raw, dev), _dev_bf16(synth.random_bf16(rng, (m, k)), dev)
+    ws = ops.Workspace(32 << 20, device=dev)
+    out = []
+    for o, work in ((off, True), (0, off % 2 == 0)):
+        h = torch.zeros((m, n), dtype=torch.bfloat16, device=dev)
+        r = torch.zeros(o + m * 2 * n, device=dev)
+        _lib.call("q4nx_gate_up_swiglu", w.data_ptr(), w.data_ptr(), n // 32, k // 256,
+                  xd.data_ptr(), k, None, 0.0, None, m, h.data_ptr(), n, r.data_ptr() + 4 * o, None,
+                  ws.buf.data_ptr() if work else None, ws.buf.numel() if work else 0, None,
+                  ops._stream())
+        out.append((h, r[o:]))
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
