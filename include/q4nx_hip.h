@@ -59,6 +59,9 @@ extern "C" {
 int q4nx_abi_version(void);
 /* Message of the last error on this thread ("" if none). */
 const char *q4nx_last_error(void);
+/* Id of the capture that `stream` is recording into a graph, 0 when it records none (or without
+ * a GPU). A workspace that a captured launch names belongs to that graph's replays. */
+unsigned long long q4nx_stream_capture_id(void *stream);
 
 /* ---------------------------------------------------------------- launch policy
  * Which kernel family takes a call and how its work is split, passed per call. No reference

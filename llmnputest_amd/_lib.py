@@ -56,6 +56,7 @@ c_pol = C.POINTER(Policy)
 SIGNATURES: dict[str, tuple] = {
     "q4nx_abi_version": (c_i, []),
     "q4nx_last_error": (C.c_char_p, []),
+    "q4nx_stream_capture_id": (C.c_ulonglong, [c_p]),
     "q4nx_dequant_q4": (c_i, [c_p, c_p, c_i, c_i, c_i, c_i, c_p]),
     "q4nx_dequant_q8": (c_i, [c_p, c_p, c_i, c_i, c_i, c_i, c_p]),
     "q4nx_policy_init": (None, [c_p]),

@@ -89,6 +89,16 @@ int q4nx_abi_version(void) { return Q4NX_ABI_VERSION; }
 
 const char* q4nx_last_error(void) { return q4nx::g_err; }
 
+unsigned long long q4nx_stream_capture_id(void* stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  if (hipStreamGetCaptureInfo((hipStream_t)stream, &status, &id) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  return status == hipStreamCaptureStatusActive ? id : 0;
+}
+
 // cos/sin of pos * theta^(-2i/hd) in float64, rounded once to float32.
 // The reference builds the same angles in float64 on the host
 // (designs/granite_gemv/granite_elementwise.py:135-138) but then rounds cos/sin to bf16.

@@ -14,8 +14,10 @@ variable (per thread / task), so callers that pass their own policy never see an
 
 from __future__ import annotations
 
+import collections
 import contextlib
 import contextvars
+import threading
 
 import numpy as np
 import torch
@@ -71,9 +73,12 @@ def _dev(t: torch.Tensor, name: str, dtype=None) -> None:
 
 
 class Workspace:
-    """Zero-filled device scratch shared by the split-K launches on one stream.
+    """Device scratch for the launches of one host thread on one stream, its arrival counters (the
+    first WS_COUNTER_BYTES) zero.
 
-    Kernels that use it leave its counters at zero, so it is zeroed only on (re)allocation.
+    Kernels that use it leave its counters at zero, so they are zeroed only on (re)allocation. An
+    op of two launches keeps its operands there between them: two threads, or two streams, need a
+    workspace each.
     """
 
     def __init__(self, nbytes: int = 0, device=None):
@@ -86,14 +91,56 @@ class Workspace:
         return self.buf.data_ptr(), self.buf.numel()
 
 
-_default_ws: dict = {}
+# What an op without ws= keeps for the next one: at most this many bytes for a stream (a larger
+# request is allocated for its call alone), for at most so many streams of a thread.
+DEFAULT_WS_BYTES = 256 << 20
+DEFAULT_WS_STREAMS = 16
+
+
+class _Defaults(threading.local):
+    """A host thread's default workspaces, by device and stream: given back when the thread ends.
+    A stream that records a graph has one of its own for that capture, which lies in the graph's
+    memory and is zeroed by its replays, so replays share no scratch with eager calls or with
+    another graph."""
+
+    def __init__(self):
+        self.by_stream: collections.OrderedDict = collections.OrderedDict()
+
+    def get(self, device: int, stream: int) -> Workspace:
+        key, capture = (device, stream), 0
+        if torch.cuda.is_current_stream_capturing():
+            capture = _lib.lib().q4nx_stream_capture_id(stream)
+            key = (device, stream, "capture")
+        held = self.by_stream.get(key)
+        if held is None or held[0] != capture:
+            held = self.by_stream[key] = (capture, Workspace(1 << 20, device=f"cuda:{device}"))
+            if len(self.by_stream) > DEFAULT_WS_STREAMS:
+                self.by_stream.popitem(last=False)
+        if len(self.by_stream) > 1:
+            self.by_stream.move_to_end(key)
+        return held[1]
+
+
+_defaults = _Defaults()
 
 
 def default_workspace() -> Workspace:
-    d = torch.cuda.current_device()
-    if d not in _default_ws:
-        _default_ws[d] = Workspace(1 << 20, device=f"cuda:{d}")
-    return _default_ws[d]
+    """What an op of this thread on the current stream uses without ws=."""
+    s = torch.cuda.current_stream()
+    return _defaults.get(s.device_index, s.cuda_stream)
+
+
+def _scratch(ws: Workspace | None, nbytes: int) -> tuple[Workspace, int, int, int]:
+    """The workspace of a call that needs nbytes, its address and size, and the current stream.
+    The caller holds the workspace until its launches are queued."""
+    s = torch.cuda.current_stream()
+    if ws is None:
+        ws = _defaults.get(s.device_index, s.cuda_stream)
+        if nbytes > max(DEFAULT_WS_BYTES, ws.buf.numel()):
+            ws = Workspace(device=ws.device)       # for this call alone: only its counters zeroed
+            ws.buf = torch.empty(nbytes, dtype=torch.uint8, device=ws.device)
+            ws.buf[:WS_COUNTER_BYTES].zero_()
+    return (ws, *ws.get(nbytes), s.cuda_stream)
 
 
 def _tiles(w: torch.Tensor, kind: str, n_tile_rows: int, k_tiles: int, name="w") -> None:
@@ -162,11 +209,11 @@ def gemv(tiles: torch.Tensor, kind: str, x: torch.Tensor, n_tile_rows: int, k_ti
         _dev(residual, "residual", torch.float32)
         if residual.numel() != b * n:
             raise ValueError("residual must have the shape of the output")
-    ws = ws or default_workspace()
     pol = _pol(policy)
-    wp, wn = ws.get(_lib.lib().q4nx_gemv_ws_bytes(KIND[kind], n_tile_rows, k_tiles, b, pol))
+    need = _lib.lib().q4nx_gemv_ws_bytes(KIND[kind], n_tile_rows, k_tiles, b, pol)
+    ws, wp, wn, stream = _scratch(ws, need)
     _lib.call(f"q4nx_gemv_{kind}", _ptr(tiles), _ptr(x2), _ptr(out), n_tile_rows, k_tiles, b,
-              k, n, _ptr(residual), wp, wn, pol, _stream())
+              k, n, _ptr(residual), wp, wn, pol, stream)
     return out.reshape(n) if squeeze else out
 
 
@@ -195,14 +242,13 @@ def gemm(tiles: torch.Tensor, kind: str, x: torch.Tensor, n_tile_rows: int, k_ti
         _dev(residual, "residual", torch.float32)
         if residual.numel() != m * n:
             raise ValueError("residual must have the shape of the output")
-    ws = ws or default_workspace()
     pol = _pol(policy)
     need = _lib.lib().q4nx_gemm_ws_bytes(KIND[kind], n_tile_rows, k_tiles, m, pol)
     if m > 64:
         need = max(need, _lib.lib().q4nx_gemm_prompt_ws_bytes(KIND[kind], n_tile_rows, k_tiles, m))
-    wp, wn = ws.get(need)
+    ws, wp, wn, stream = _scratch(ws, need)
     _lib.call("q4nx_gemm", KIND[kind], _ptr(tiles), n_tile_rows, k_tiles, _ptr(x2), x2.stride(0),
-              m, _ptr(out), n, _ptr(residual), wp, wn, pol, _stream())
+              m, _ptr(out), n, _ptr(residual), wp, wn, pol, stream)
     return out.reshape(n) if squeeze else out
 
 
@@ -239,12 +285,12 @@ def gemv_ex(tiles: torch.Tensor, kind: str, x: torch.Tensor, n_tile_rows: int, k
             raise ValueError("argmax_keys needs batch * N/16 entries")
     _ssq(ssq_in, "ssq_in", b, k_tiles * 16)
     _ssq(ssq_out, "ssq_out", b, n_tile_rows * 2)
-    ws = ws or default_workspace()
     pol = _pol(policy)
-    wp, wn = ws.get(_lib.lib().q4nx_gemv_ws_bytes(KIND[kind], n_tile_rows, k_tiles, b, pol))
+    need = _lib.lib().q4nx_gemv_ws_bytes(KIND[kind], n_tile_rows, k_tiles, b, pol)
+    ws, wp, wn, stream = _scratch(ws, need)
     _lib.call("q4nx_gemv_ex", KIND[kind], _ptr(tiles), n_tile_rows, k_tiles, _ptr(x2),
               x2.shape[1], _ptr(norm_w), float(eps), _ptr(ssq_in), b, _ptr(out), n,
-              _ptr(residual), _ptr(ssq_out), _ptr(argmax_keys), wp, wn, pol, _stream())
+              _ptr(residual), _ptr(ssq_out), _ptr(argmax_keys), wp, wn, pol, stream)
     return out
 
 
@@ -402,9 +448,9 @@ def qkv_rope(wq, wk, wv, n_q_heads: int, n_kv_heads: int, k_tiles: int, x: torch
         q_out = torch.empty((b, n_q_heads * 64), dtype=torch.bfloat16, device=x.device)
     if norm_w is not None:
         _dev(norm_w, "norm_w", torch.bfloat16)
-    ws = ws or default_workspace()
     pol = _pol(policy)
-    wp, wn = ws.get(_lib.lib().q4nx_qkv_rope_ws_bytes(n_q_heads, n_kv_heads, k_tiles, b, pol))
+    need = _lib.lib().q4nx_qkv_rope_ws_bytes(n_q_heads, n_kv_heads, k_tiles, b, pol)
+    ws, wp, wn, stream = _scratch(ws, need)
     _ssq(ssq_in, "ssq_in", b, k_tiles * 16)
     lmax = k_cache.shape[2]
     _lib.call("q4nx_qkv_rope", _ptr(wq), _ptr(wk), _ptr(wv), n_q_heads, n_kv_heads, k_tiles,
@@ -412,7 +458,7 @@ def qkv_rope(wq, wk, wv, n_q_heads: int, n_kv_heads: int, k_tiles: int, x: torch
               _ptr(table),
               table.shape[0] if table.shape[0] < lmax else lmax, _ptr(q_out), _ptr(k_cache),
               _ptr(v_cache), k_cache.stride(0), k_cache.stride(1), _ptr(raw_out), _ptr(xn_out),
-              wp, wn, pol, _stream())
+              wp, wn, pol, stream)
     return q_out
 
 
@@ -430,13 +476,13 @@ def gate_up_swiglu(wg, wu, n_tile_rows: int, k_tiles: int, x: torch.Tensor,
     n = n_tile_rows * 32
     if h_out is None:
         h_out = torch.empty((b, n), dtype=torch.bfloat16, device=x.device)
-    ws = ws or default_workspace()
     pol = _pol(policy)
-    wp, wn = ws.get(_lib.lib().q4nx_gate_up_ws_bytes(n_tile_rows, k_tiles, b, pol))
+    need = _lib.lib().q4nx_gate_up_ws_bytes(n_tile_rows, k_tiles, b, pol)
+    ws, wp, wn, stream = _scratch(ws, need)
     _ssq(ssq_in, "ssq_in", b, k_tiles * 16)
     _lib.call("q4nx_gate_up_swiglu", _ptr(wg), _ptr(wu), n_tile_rows, k_tiles, _ptr(x),
               x.shape[1], _ptr(norm_w), float(eps), _ptr(ssq_in), b, _ptr(h_out), h_out.stride(0),
-              _ptr(raw_out), _ptr(xn_out), wp, wn, pol, _stream())
+              _ptr(raw_out), _ptr(xn_out), wp, wn, pol, stream)
     return h_out
 
 
@@ -461,15 +507,14 @@ def gqa_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
     if out is None:
         out = torch.empty((b, hq, d), dtype=torch.bfloat16, device=q.device)
     of = torch.empty((b, hq, d), dtype=torch.float32, device=q.device) if want_f32 else None
-    ws = ws or default_workspace()
     pol = _pol(policy)
     need = _lib.lib().q4nx_gqa_decode_ws_bytes(b, hq, hkv, max_len, pol)
     if n_split:
         need = max(need, WS_COUNTER_BYTES + b * hkv * n_split * (hq // hkv) * 68 * 4)
-    wp, wn = ws.get(need)
+    ws, wp, wn, stream = _scratch(ws, need)
     _lib.call("q4nx_gqa_decode", _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), _ptr(of), b,
               hq, hkv, d, _ptr(lens), max_len, k_cache.stride(0), k_cache.stride(1),
-              float(scale), int(n_split), wp, wn, pol, _stream())
+              float(scale), int(n_split), wp, wn, pol, stream)
     return (out, of) if want_f32 else out
 
 
@@ -508,11 +553,10 @@ def gqa_decode_records(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Te
     max_len = lmax if max_len is None else min(max_len, lmax)
     g = hq // hkv
     pb = b * hkv * n_split * g * 68 * 4
-    ws = ws or default_workspace()
-    wp, wn = ws.get(WS_COUNTER_BYTES + pb)
+    ws, wp, wn, stream = _scratch(ws, WS_COUNTER_BYTES + pb)
     _lib.call("q4nx_gqa_decode_records", _ptr(q), _ptr(k_cache), _ptr(v_cache), b, hq, hkv, d,
               _ptr(lens), max_len, k_cache.stride(0), k_cache.stride(1), float(scale),
-              int(n_split), wp, wn, _pol(policy), _stream())
+              int(n_split), wp, wn, _pol(policy), stream)
     return ws.buf[WS_COUNTER_BYTES:WS_COUNTER_BYTES + pb].view(torch.float32).view(
         b, hkv, n_split, g, 68)
 
