@@ -574,9 +574,10 @@ __global__ __launch_bounds__(64 * WN * WK, OCC) void pq_kernel(GemmArgs a, PqX p
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[r][mt][0] = acc[r][mt][1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   // Short accumulation chains where the registers allow: a K-tile's sum starts from zero and is
-  // added to the total on the VALU (the matrix cores' own accumulation rounds more coarsely: K =
-  // 8192 in one chain is 5.9e-7 off the 64-bit result, in tiles 1.2e-7 .. 1.6e-7; the kernel of
-  // this shape before, 1.9e-6)
+  // added to the total on the VALU. The matrix cores' own accumulation rounds more coarsely: one
+  // chain over K = 1024 / 2560 / 8192 is 2.0 / 3.2 / 5.9e-7 off the 64-bit result, in K-tiles 1.0 /
+  // 1.1 / 1.4e-7. The 128-row q4 tile has no registers for that; in two K parts it is 1.4 / 2.2 /
+  // 4.1e-7 off, the batched kernel 1.9 / 2.6 / 4.2e-7 (which tile a launch may take: pq_plain).
   constexpr bool FLUSH = KIND == 4 && MT * RT <= 8;
   f32x4_t prt[FLUSH ? RT : 1][FLUSH ? MT : 1][2];
   const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
@@ -1034,6 +1035,9 @@ bool pq_use(int kind, int op, const GemmArgs& a) {
          Q4NX_ALIGNED(a.raw_out, 8);
 }
 
+// Whether w workgroups that take a CU each leave at most an eighth of their rounds idle
+static bool fills_cus(int w) { return w >= 224 && w * 8 >= (w + 255) / 256 * 256 * 7; }
+
 // Tile by the workgroups it gives a chip of 256 CUs, two on each: the largest that fills it.
 // Measured over N x K of 512 x 1024 to 12288 x 4096 (q8: to 248320 x 1024) and 65 to 3000 rows; us
 // at the side of each line where the two are closest (N x K, rows):
@@ -1044,12 +1048,21 @@ static void pq_plain(const GemmArgs& a, const PqX& x, hipStream_t st) {
   };
   const int w64 = wgs(64, 4);
   if constexpr (KIND == 4) {
-    // 128 rows x 8 tile-rows against 64 x 4: 8192 x 2560, 1000 rows (256) 57 / 61, 640 rows
-    // (160) 53 / 47; a short K does not repay the larger block's epilogue (6144 x 1024, 1500
-    // rows (288) 44 / 38), and with fewer rows than the block has the others are as fast and add
-    // up in shorter chains (the error against 64 bits 1.2e-7, not 2.8e-7)
+    // 128 rows x 8 tile-rows, eight waves with K in two parts, one workgroup per CU, against the
+    // same in one part and 64 x 4 (workgroups): 8192 x 2560 256 55.5 / 54.9 / 58.3, 512 100 / 86 /
+    // 103; 4096 x 4096 256 73.9 / 74.8 / 84.6; 2560 x 8192, 3000 rows (240) 133 / 140 / 161; one that
+    // leaves CUs idle in its last round loses (10240 x 4096 320 125 / 109 / 101). Its chains over K
+    // are half as long, so launches with sums of squares, formerly the batched kernel's, take it
+    // or 64 x 4 (768 144 / 148) where one chain is the less exact, from K = 1024 on.
+    const bool exact = a.ssq_out != nullptr && a.k_t >= 4;
     const int w0 = a.m_rows < 128 ? 0 : wgs(128, 8);
-    if (w0 >= 512 || (w0 >= 240 && a.k_t >= 8)) return pq_go<4, GOP_PLAIN, 8, 2, 4, 1, 4, 2>(a, x, st);
+    if (a.k_t >= 8 && fills_cus(w0) && (w0 <= 256 || exact))
+      return pq_go<4, GOP_PLAIN, 8, 2, 4, 2, 4, 2>(a, x, st);
+    // the same in one part against 64 x 4: 640 rows (160) 53 / 47; a short K does not repay the
+    // larger block's epilogue (6144 x 1024, 1500 rows (288) 44 / 38), and with fewer rows than the
+    // block has the others are as fast and nearer to the 64-bit result
+    if (!exact && (w0 >= 512 || (w0 >= 240 && a.k_t >= 8)))
+      return pq_go<4, GOP_PLAIN, 8, 2, 4, 1, 4, 2>(a, x, st);
     // 64 x 4 against 64 x 2 with K in two parts: 2560 x 8192, 1500 rows (480) 90 / 99, 1000 rows
     // (320) 80 / 72
     if (w64 >= 440) return pq_go<4, GOP_PLAIN, 4, 1, 4, 1, 8, 2>(a, x, st);
@@ -1077,9 +1090,21 @@ static void pq_gateup(const GemmArgs& a, const PqX& x, hipStream_t st) {
   const auto wgs = [&](int rows, int trs) {
     return ((a.m_rows + rows - 1) / rows) * ((a.n_tr[0] + trs - 1) / trs);
   };
-  // 128 rows x 4 pairs against 64 x 2 in two parts: 8192 x 2560, 400 rows (256) 55 / 64, 192
-  // rows (128) 51 / 39
-  if (wgs(128, 4) >= 192) return pq_go<4, GOP_GATEUP, 8, 2, 4, 1, 4, 2>(a, x, st);
+  // 128 rows x 4 pairs, eight waves with K in two parts, one workgroup per CU, against 64 x 4 in one
+  // part (128-row workgroups, us): 8192 x 2560 256 54.8 / 57.1, 1024 185 / 186; 4096 x 4096 224 67 /
+  // 76, 512 135 / 146; 2560 x 8192 480 240 / 278; 10240 x 4096 400 121 / 111, 960 253 / 277; 6144 x 1536
+  // 768 105 / 96. (In one part it takes 155 us for the 1024, but its chain over K is 3.2e-7 off at
+  // K = 2560 where the batched kernel was 2.6e-7.)
+  if (a.k_t >= 8 && a.m_rows >= 128 && fills_cus(wgs(128, 4)))
+    return pq_go<4, GOP_GATEUP, 8, 2, 4, 2, 4, 2>(a, x, st);
+  // 64 rows x 4 pairs, whole K, against 64 x 2 in two parts, which fill a last round of the 512
+  // workgroups the chip holds more evenly (64 x 4 workgroups): 8192 x 2560 448 54 / 59, 576 75 / 72,
+  // 640 76 / 74, 832 93 / 96; 4096 x 4096 320 72 / 66, 416 75 / 80, 608 110 / 102; 10240 x 4096 720
+  // 111 / 118; a short K does not repay the parts: 2048 x 1024 144 19.6 / 19.3, 384 28.6 / 30.9, 6144
+  // x 1536 144 26.2 / 26.7, 432 37 / 43
+  const int w64 = wgs(64, 4);
+  if (a.k_t <= 6 ? w64 >= 144 : w64 >= 400 && (w64 <= 512 || w64 >= 704))
+    return pq_go<4, GOP_GATEUP, 4, 2, 4, 1, 4, 2>(a, x, st);
   // 64 x 2 against 32 x 2 in four parts: 2560 x 8192, 256 rows (160) 58 / 70, 192 rows (120)
   // 58 / 44
   if (wgs(64, 2) >= 160) return pq_go<4, GOP_GATEUP, 4, 2, 2, 2, 4, 2>(a, x, st);

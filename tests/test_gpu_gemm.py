@@ -567,3 +567,68 @@ def test_prompt_gate_up_raw_out_at_any_float(dev, off):
                   ops._stream())
         out.append((h, r[o:]))
     assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+
+
+@pytest.mark.parametrize("m,n,k", [(500, 8192, 2560), (1000, 4096, 4096), (900, 2560, 8192),
+                                   (1500, 2560, 8192), (2048, 8192, 2560), (2048, 8192, 1024),
+                                   (2048, 12288, 768), (300, 4096, 1280)])
+@pytest.mark.parametrize("mean", [0.0, 0.5])
+def test_prompt_blocks_as_exact_as_batched(dev, m, n, k, mean):
+    """Prompt blocks that ran on the batched kernel ([gate, up], and projections that also give
+    sums of squares) are no further from the 64-bit result on the fp16-operand kernel: the 2-norm
+    of the difference, against that of the batched kernel (the same call without a workspace)."""
+    from llmnputest_amd import _lib
+    g = torch.Generator(device=dev)
+    g.manual_seed(m)
+    from llmnputest_amd.granite import random_q4_tiles
+    w = random_q4_tiles(n, k, g, dev)
+    x = (torch.randn((m, k), device=dev, generator=g) + mean).to(torch.bfloat16)
+    wm = ops.dequant(w, "q4", n // 32, k // 256, out_dtype=torch.float32, untile=True).double()
+    ref = x.double() @ wm.t().contiguous()
+    ws = ops.Workspace(96 << 20, device=dev)
+    gu, pl = [], []
+    for wp, wn in ((ws.buf.data_ptr(), ws.buf.numel()), (None, 0)):
+        h = torch.empty((m, n), dtype=torch.bfloat16, device=dev)
+        raw = torch.empty((m, 2 * n), device=dev)
+        _lib.call("q4nx_gate_up_swiglu", w.data_ptr(), w.data_ptr(), n // 32, k // 256, x.data_ptr(),
+                  k, None, 0.0, None, m, h.data_ptr(), n, raw.data_ptr(), None, wp, wn, None,
+                  ops._stream())
+        y = torch.empty((m, n), device=dev)
+        ssq = torch.empty((m, n // 16), device=dev)
+        _lib.call("q4nx_gemv_ex", 4, w.data_ptr(), n // 32, k // 256, x.data_ptr(), k, None, 0.0, None,
+                  m, y.data_ptr(), n, None, ssq.data_ptr(), None, wp, wn, None, ops._stream())
+        gu.append(((raw[:, :n].double() - ref).norm() / ref.norm()).item())
+        pl.append(((y.double() - ref).norm() / ref.norm()).item())
+    assert gu[0] <= gu[1] and pl[0] <= pl[1], (gu, pl)
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (2100, 4128, 2304),   # 128 x 8 in one part (289 workgroups), ragged both ways, nine K-tiles
+    (4100, 4000, 256),    # the same (528), one K-tile
+    (1900, 4320, 2304),   # 128 x 8 in two parts (255 workgroups), five and four K-tiles
+    (2000, 4064, 8448),   # the same, rows longer than the pre-pass keeps in registers
+])
+def test_gemm_large_tiles_parity(dev, m, n, k):
+    """The 128-row q4 tiles, plain and with sums of squares (which may take another tile)."""
+    raw, rng = _tiles("q4", n, k, 51 + m)
+    raw = _free_minima(raw, rng)
+    x = synth.random_bf16(rng, (m, k))
+    res = rng.standard_normal((m, n)).astype(np.float32)
+    w, xd, rd = _dev_u8(raw, dev), _dev_bf16(x, dev), torch.from_numpy(res).to(dev)
+    rows = np.unique(np.concatenate([np.arange(0, m, max(1, m // 32)), [m - 1]]))
+    ref = qo.gemv(raw, "q4", x[rows], n // 32, k // 256, acc=np.float64) + res[rows]
+    _check_rows(ops.gemm(w, "q4", xd, n // 32, k // 256, residual=rd).cpu().numpy()[rows], ref)
+    ssq = torch.full((m, n // 16), float("nan"), device=dev)
+    y = ops.gemv_ex(w, "q4", xd, n // 32, k // 256, residual=rd, ssq_out=ssq)
+    _check_rows(y.cpu().numpy()[rows], ref)
+    want = y.double().view(m, -1, 16).square().sum(-1)
+    assert ((ssq.double() - want).abs() <= 16 * 2.0 ** -24 * want).all()
+
+
+@pytest.mark.parametrize("batch,n,k", [
+    (1000, 3616, 2304),        # 128 x 4 pairs in two parts (232), ragged both ways, nine K-tiles
+    (900, 1984, 1280),         # 64 x 4 pairs (240), five K-tiles
+    (1700, 2592, 256),         # the same, one K-tile
+])
+def test_gate_up_large_tiles(dev, batch, n, k):
+    test_gate_up_fp16_operands(dev, batch, n, k, False)
