@@ -60,8 +60,9 @@ bool mfma_norm_fits(int k_t, int m_rows, size_t ws_bytes);
 // 38 / 21, [gate, up] 43 / 31; q8 2560 x 2560 20 / 14; at 64 rows q4 19 / 19, 22 / 20 and 28 /
 // 27, most shapes the batched kernel's).
 constexpr int kPqRows = 65;
-// workspace bytes it keeps the fp16 x, sums and column terms in (past the counters)
-size_t pq_ws_bytes(int kind, int op, int n_tile_rows, int k_t, int m_rows);
+// workspace bytes it keeps the fp16 x, sums and column terms in (past the counters); own_norm: with an
+// RMSNorm prologue whose rows the caller does not take
+size_t pq_ws_bytes(int kind, int op, int n_tile_rows, int k_t, int m_rows, bool own_norm);
 // whether a launch of op `op` described by `a` can take that kernel (its outputs' alignment and
 // strides; anything else is the batched kernel's, which reads and writes single values)
 bool pq_use(int kind, int op, const GemmArgs& a);

@@ -775,7 +775,7 @@ size_t mfma_ws_bytes(int kind, int op, int n_units, int k_t, int m_rows, const P
   // room for the split-K records and the normalised rows of an RMSNorm prologue or, for a prompt
   // block, for what the fp16-operand kernel keeps
   const size_t split = split_part_bytes(plan_gemm(kind, op, n_units, k_t, m_rows, P));
-  const size_t pq = op != GOP_QKV && m_rows >= kPqRows ? pq_ws_bytes(kind, op, n_units, k_t, m_rows) : 0;
+  const size_t pq = op != GOP_QKV && m_rows >= kPqRows ? pq_ws_bytes(kind, op, n_units, k_t, m_rows, k_t * kTileK / kSsqRows <= 512) : 0;
   const size_t b = align256(split) + align256((size_t)m_rows * k_t * kTileK * 2);
   return Q4NX_WS_COUNTER_BYTES + (pq > b ? pq : b);
 }
@@ -809,7 +809,7 @@ int mfma_launch(int kind, int op, GemmArgs& a, int n_units, void* ws, size_t ws_
   // there (a K split that the policy names belongs to the batched kernel)
   if (pq_use(kind, op, a) && ws_ok && P.gemm_ksplit == 0 && !short_k &&
       (a.norm_w == nullptr || (a.ssq_in != nullptr && K / kSsqRows <= 512)) &&
-      ws_bytes >= Q4NX_WS_COUNTER_BYTES + pq_ws_bytes(kind, op, a.n_tr[0], a.k_t, a.m_rows)) {
+      ws_bytes >= Q4NX_WS_COUNTER_BYTES + pq_ws_bytes(kind, op, a.n_tr[0], a.k_t, a.m_rows, xn_b != 0)) {
     pq_launch(kind, op, a, (uint8_t*)ws + Q4NX_WS_COUNTER_BYTES, st);
     return check_launch(what);
   }
@@ -888,7 +888,7 @@ size_t q4nx_gemm_prompt_ws_bytes(int kind, int n_tile_rows, int k_tiles, int m_r
   if ((kind != Q4NX_KIND_Q4 && kind != Q4NX_KIND_Q8) || n_tile_rows < 1 || k_tiles < 1 ||
       m_rows < kPqRows)
     return 0;
-  return Q4NX_WS_COUNTER_BYTES + pq_ws_bytes(kind, GOP_PLAIN, n_tile_rows, k_tiles, m_rows);
+  return Q4NX_WS_COUNTER_BYTES + pq_ws_bytes(kind, GOP_PLAIN, n_tile_rows, k_tiles, m_rows, false);
 }
 
 int q4nx_gemm(int kind, const uint8_t* w, int n_tile_rows, int k_tiles, const uint16_t* x,

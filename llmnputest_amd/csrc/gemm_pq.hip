@@ -13,8 +13,7 @@
 // of -(B + 7.5) d. d has 8 significant bits and A is a multiple of at most 128 of their last
 // place, so the result is a multiple of that place below 2^11 of them: exact. A's own rounding
 // is in o = -(B d + A), hence in u. x is an exact fp16 value under a power of two per row, d
-// under one per column (an entry 2^28 below its row's largest loses bits, 2^-39 of that
-// largest). The first sum is therefore v_mfma_f32_16x16x32_f16 alone, one per 16x16 block and
+// under one per column (what that leaves out: below, "Range"). The first sum is therefore v_mfma_f32_16x16x32_f16 alone, one per 16x16 block and
 // group with exact products: no per-group scale on the VALU, and no large offset to cancel
 // afterwards. The second sum is a contraction over the groups (32 per MFMA), S and u each in two
 // fp16 terms (the product of the two low terms, 2^-22, is left out). A one-hot row still gives
@@ -26,6 +25,16 @@
 // inner sum, which four FMAs per lane scale into the total. (Two MFMAs on s = s1 + s2, four bits
 // each, and no FMA took 555 us for 512 rows of 248320 x 1024, this 471.) x and s under powers of two
 // as above.
+//
+// Range. Under a row's power of two an entry of x is exact down to 2^-31 of the row's largest and
+// is rounded at 2^-39 of it below; d is exact down to 2^-22 of what the column's largest |m| and 8
+// |d| allow (d below 2^5, |m| below 2^8), S and u are kept to 2^-23 of themselves and 2^-33, 2^-39
+// of the largest. All of that is below the fp32 rounding of a sum to which the large groups
+// contribute: 16 d x of some group is within 2^-10 of the largest d times the largest x as soon as
+// either the row's or the column's groups all lie within 2^-10 of its largest one. The pre-pass marks
+// the rows and the columns of which that is not so, and a workgroup that has both adds up its tile
+// on bf16 operands with one fp32 scale per group instead (exact_tile): no loss at any range. (Marking
+// takes 0.3 to 0.4 us of the pre-pass, looking 0.3 to 3 us of the contraction.)
 //
 // What bounds it: see pq_kernel.
 #include "common.h"
@@ -47,9 +56,19 @@ __device__ __forceinline__ uint32_t pk_max_u16(uint32_t a, uint32_t b) {
   return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(us2_t, a),
                                                                 __builtin_bit_cast(us2_t, b)));
 }
-// two fp32 values that fp16 holds exactly (or far below the scale's largest), packed
-__device__ __forceinline__ uint32_t pk_f16(float lo, float hi) {
+__device__ __forceinline__ uint32_t pk_min_u16(uint32_t a, uint32_t b) {
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(us2_t, a),
+                                                                __builtin_bit_cast(us2_t, b)));
+}
+__device__ __forceinline__ uint32_t pk_add_u16(uint32_t a, uint32_t b) {
+  return __builtin_bit_cast(uint32_t, __builtin_bit_cast(us2_t, a) + __builtin_bit_cast(us2_t, b));
+}
+// two fp32 values as packed fp16, towards zero (one instruction); to nearest
+__device__ __forceinline__ uint32_t pk_f16z(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(lo, hi));
+}
+__device__ __forceinline__ uint32_t pk_f16(float lo, float hi) {
+  return h2_bits(half2_t{(_Float16)lo, (_Float16)hi});
 }
 // v = hi + lo to 2^-22: the two terms of a pair of values as packed fp16 words
 __device__ __forceinline__ void split2(float v0, float v1, uint32_t& hi, uint32_t& lo) {
@@ -68,6 +87,7 @@ constexpr int kPqWTop = 135;          // |u| of a column below 2^9, its 8 |d| be
 constexpr int kPqSum = 6;             // S is kept 2^6 below its row's scale, u 2^6 above its column's
 constexpr int kPqSTop = 131;          // a q8 column's largest scale in [2^4, 2^5)
 constexpr float kPqLow = -1031.5f, kPqHigh = -71.5f;   // A / d of the low and the high nibbles
+constexpr int kPqSpan = 10;           // a "wide" row or column: a group below 2^-10 of its largest
 constexpr int kPqSlack = 64 << 10;    // bytes after x that steps past its end read (never used)
 
 // The pre-pass's output (workspace), all in the order the contraction's operands take it: x as
@@ -78,8 +98,12 @@ struct PqX {
   u32x4_t* u;       // [tensor][tile-row][chunk][hi, lo][even, odd column][lane]
   uint2* scale;     // [tensor][tile-row][group][lane % 16]: fp16 d of the even and odd column, A
                     // (q4 only)
-  int* xshift;      // [row]: the power of two of x
-  int* wshift;      // [tensor][column]: that of d, A and u (q8: of s)
+  int* xshift;      // [row]: the power of two of x, times two, + 1 for a wide row
+  int* wshift;      // [tensor][column]: that of d, A and u (q8: of s), + 1 for a wide column
+  uint16_t* xe;     // with an RMSNorm whose rows the caller does not take: [row][K], wide rows only
+  const uint16_t* exact;    // bf16 rows for exact_tile, exact_stride entries apart: all of them,
+  int64_t exact_stride;     // or the wide ones
+  bool exact_all;
   int m_blocks, c_groups;   // the launch's row blocks, its groups of columns
   bool rows_first;  // the order of its workgroups: row blocks first, within an eighth of them
 };
@@ -97,6 +121,31 @@ __device__ __forceinline__ uint32_t rows_max(uint32_t v) {    // across the four
   return pk_max_u16(b[0], b[1]);
 }
 
+__device__ __forceinline__ uint32_t rows_min(uint32_t v) {
+  const auto a = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  v = pk_min_u16(a[0], a[1]);
+  const auto b = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  return pk_min_u16(b[0], b[1]);
+}
+// the smallest over the wave of 32-bit values that the four lanes of a quad share
+template <int CTRL>
+__device__ __forceinline__ uint32_t umin_dpp(uint32_t v) {
+  return min(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, false));
+}
+__device__ __forceinline__ uint32_t quads_min(uint32_t v) {
+  v = umin_dpp<kDppRor8>(umin_dpp<kDppHalfMirror>(v));
+  const auto a = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  v = min(a[0], a[1]);
+  const auto b = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  return min(b[0], b[1]);
+}
+// whether the smallest of a row's or column's groups lies more than kPqSpan binary orders below
+// its largest (bf16 exponent fields; 0 is the smallest normal numbers' binade or less, which the
+// largest power of two lifts whole into range)
+__device__ __forceinline__ int span_wide(int largest, int smallest) {
+  return max(largest, 1) - max(smallest, 1) > kPqSpan;
+}
+
 // 2^e as a float, -126 <= e <= 127
 __device__ __forceinline__ float exp2i(int e) { return __int_as_float((e + 127) << 23); }
 
@@ -106,9 +155,10 @@ __host__ __device__ constexpr int pq_chunks(int k_t) {
   return KIND == 4 ? (k_t + kPqChunkTiles - 1) / kPqChunkTiles : 0;
 }
 
-// One row of x per NT threads (a workgroup, or one wave of it): x (or RMSNorm of the fp32 residual, to bf16 first, as every
-// consumer rounds it) to fp16 under the row's power of two, and the sums per 32-K group. Each
-// thread keeps C chunks of 8 entries (K <= 8 NT C; longer rows are read again for the second
+// One row of x per NT threads (a workgroup, or one wave of it): x (or RMSNorm of the fp32 residual,
+// to bf16 first, as every consumer rounds it) to fp16 under the row's power of two, the sums per
+// 32-K group, and whether the row is wide (a wide row of a norm is also kept as bf16). Each thread
+// keeps C chunks of 8 entries (K <= 8 NT C; longer rows are read again for the second
 // pass). Every load is unconditional, through a buffer resource over the row: entries past its
 // end read zeros. Rows past m_rows stay unwritten: a row of an operand reaches its own row of
 // the result only. The code is kept short: a wave runs it once, so its instruction fetches are
@@ -132,10 +182,14 @@ __device__ __forceinline__ void prep_row(const GemmArgs& a, const PqX& o, int ro
       NORM ? make_rsrc(a.hres + (int64_t)row * a.x_stride, (uint32_t)K * 4u)
            : make_rsrc(a.x + (int64_t)row * a.x_stride, (uint32_t)K * 2u);
   u32x4_t v[C];
-  uint32_t mx = 0;
-  auto see = [&](const u32x4_t& w) {
+  uint32_t mx = 0, mn = ~0u;                    // the row's largest entry; the smallest group's
+  auto see = [&](const u32x4_t& w) {            // largest, less 1 (a group of zeros: none)
+    uint32_t g = 0;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) mx = pk_max_u16(mx, w[j] & 0x7FFF7FFFu);
+    for (int j = 0; j < 4; ++j) g = pk_max_u16(g, w[j] & 0x7FFF7FFFu);
+    mx = pk_max_u16(mx, g);
+    g = umax_dpp<kDppXor2>(umax_dpp<kDppXor1>(g));
+    mn = min(mn, max(g >> 16, g & 0xFFFFu) - 1u);
   };
   if constexpr (NORM) {
     const __amdgpu_buffer_rsrc_t wr = make_rsrc(a.norm_w, (uint32_t)K * 2u);
@@ -175,18 +229,29 @@ __device__ __forceinline__ void prep_row(const GemmArgs& a, const PqX& o, int ro
   mx = umax_dpp<kDppXor2>(mx);
   mx = umax_dpp<kDppHalfMirror>(mx);
   mx = rows_max(umax_dpp<kDppRor8>(mx));
+  mn = quads_min(mn);
   if constexpr (NT > 64) {
-    if (l == 0) smx[wave] = mx;
+    if (l == 0) smx[2 * wave] = mx, smx[2 * wave + 1] = mn;
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < NT / 64; ++i) mx = pk_max_u16(mx, smx[i]);
+    for (int i = 0; i < NT / 64; ++i) mx = pk_max_u16(mx, smx[2 * i]), mn = min(mn, smx[2 * i + 1]);
   }
   // exponent field of the row's largest entry; a row with an infinity or a NaN is left
   // unscaled (its sums carry the NaN into every output of the row)
   const int ex = (int)max(mx >> 16, mx & 0xFFFFu) >> 7;
   const int sh = ex == 255 ? 0 : min(kPqXTop - max(ex, 1), 127);
-  const float sc = exp2i(sh), ss = exp2i(sh - kPqSum);
-  if (tid == 0) o.xshift[row] = sh;
+  const float sc = exp2i(sh);
+  const int wide = ex < 255 && mn != ~0u && span_wide(ex, (int)(mn + 1) >> 7);
+  if (tid == 0) o.xshift[row] = 2 * sh + wide;
+  if constexpr (NORM) {
+    if (wide && a.xn_out == nullptr) {
+#pragma unroll
+      for (int i = 0; i < C; ++i) {
+        const int q = tid + NT * i;
+        if (q < n_q) *(u32x4_t*)(o.xe + (size_t)row * K + 8 * q) = v[i];
+      }
+    }
+  }
   const int r16 = row & 15, swz = (r16 >> 1) & 3;
   u32x4_t* xt = o.xt + (size_t)(row >> 4) * (a.k_t * 8 + n_ch * 2) * 64 + r16 * 4;
   u32x4_t* sm = xt + (size_t)a.k_t * 8 * 64;
@@ -203,9 +268,9 @@ __device__ __forceinline__ void prep_row(const GemmArgs& a, const PqX& o, int ro
       for (int j = 0; j < 4; ++j) {
         // entries k, k + 2 of a group of four share a word, as the codes do (below)
         const int e = j & 2;
-        const float x0 = (j & 1) ? bf16hi(w[e]) : bf16lo(w[e]);
-        const float x1 = (j & 1) ? bf16hi(w[e + 1]) : bf16lo(w[e + 1]);
-        h[j] = pk_f16(x0 * sc, x1 * sc);
+        const float x0 = ((j & 1) ? bf16hi(w[e]) : bf16lo(w[e])) * sc;
+        const float x1 = ((j & 1) ? bf16hi(w[e + 1]) : bf16lo(w[e + 1])) * sc;
+        h[j] = pk_f16(x0, x1);
         s += x0 + x1;
       }
       if (q < n_q) xt[(size_t)(q >> 2) * 64 + ((q & 3) ^ swz)] = h;
@@ -224,7 +289,7 @@ __device__ __forceinline__ void prep_row(const GemmArgs& a, const PqX& o, int ro
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         uint32_t th, tl;
-        split2(sg[8 * tid + 2 * j] * ss, sg[8 * tid + 2 * j + 1] * ss, th, tl);
+        split2(sg[8 * tid + 2 * j] * exp2i(-kPqSum), sg[8 * tid + 2 * j + 1] * exp2i(-kPqSum), th, tl);
         hi[j] = th;
         lo[j] = tl;
       }
@@ -248,6 +313,7 @@ __device__ __forceinline__ void prep_tile_row(const GemmArgs& a, const PqX& o, i
   const uint8_t* wr = a.w[tensor] + (size_t)tr * a.k_t * kQ4TileBytes +
                       2 * ((c >> 3) * 16 + 2 * (c & 7));
   uint32_t dv[CACHED][8], mv[CACHED][8], dm = 0, mm = 0;
+  uint32_t mn = ~0u;                            // the smallest group's larger of |m| and 8 |d|
   auto fetch = [&](int ch, uint32_t (&d)[8], uint32_t (&m)[8]) {
     const int kt = kPqChunkTiles * ch + s;
     const uint8_t* t = wr + (size_t)min(kt, a.k_t - 1) * kQ4TileBytes;
@@ -265,11 +331,14 @@ __device__ __forceinline__ void prep_tile_row(const GemmArgs& a, const PqX& o, i
       m[j] = in ? m[j] : 0u;
     }
   };
-  auto see = [&](const uint32_t (&d)[8], const uint32_t (&m)[8]) {
+  auto see = [&](int ch, const uint32_t (&d)[8], const uint32_t (&m)[8]) {
+    const uint32_t past = kPqChunkTiles * ch + s < a.k_t ? 0u : ~0u;   // groups past K: none
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      dm = pk_max_u16(dm, d[j] & 0x7FFF7FFFu);
-      mm = pk_max_u16(mm, m[j] & 0x7FFF7FFFu);
+      const uint32_t da = d[j] & 0x7FFF7FFFu, ma = m[j] & 0x7FFF7FFFu;
+      dm = pk_max_u16(dm, da);
+      mm = pk_max_u16(mm, ma);
+      mn = pk_min_u16(mn, pk_max_u16(pk_add_u16(da, 0x01800180u), ma) | past);
     }
   };
 #pragma unroll
@@ -279,36 +348,41 @@ __device__ __forceinline__ void prep_tile_row(const GemmArgs& a, const PqX& o, i
   for (int i = 0; i < CACHED; ++i)
     if (w + NW * i < n_ch) {
       clip(w + NW * i, dv[i], mv[i]);
-      see(dv[i], mv[i]);
+      see(w + NW * i, dv[i], mv[i]);
     }
   for (int ch = w + NW * CACHED; ch < n_ch; ch += NW) {
     uint32_t d[8], m[8];
     fetch(ch, d, m);
     clip(ch, d, m);
-    see(d, m);
+    see(ch, d, m);
   }
   dm = rows_max(dm);
   mm = rows_max(mm);
+  mn = rows_min(mn);
   if (l < 16) {
-    sm[w * 32 + l] = dm;
-    sm[w * 32 + 16 + l] = mm;
+    sm[w * 48 + l] = dm;
+    sm[w * 48 + 16 + l] = mm;
+    sm[w * 48 + 32 + l] = mn;
   }
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < NW; ++i) {
-    dm = pk_max_u16(dm, sm[i * 32 + c]);
-    mm = pk_max_u16(mm, sm[i * 32 + 16 + c]);
+    dm = pk_max_u16(dm, sm[i * 48 + c]);
+    mm = pk_max_u16(mm, sm[i * 48 + 16 + c]);
+    mn = pk_min_u16(mn, sm[i * 48 + 32 + c]);
   }
-  int sh[2];
+  int sh[2], wide[2];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     const int ed = (int)((dm >> (16 * h + 7)) & 0xFF), em = (int)((mm >> (16 * h + 7)) & 0xFF);
     // |u| <= |m| + 8 |d| < 2^(max(em, ed + 3) + 1 - 126)
-    sh[h] = ed < 255 && em < 255 ? min(kPqWTop - 1 - max(max(em, ed + 3), 1), 127 - kPqSum) : 0;
+    const bool finite = ed < 255 && em < 255;
+    sh[h] = finite ? min(kPqWTop - 1 - max(em, ed + 3), 127 - kPqSum) : 0;
+    wide[h] = finite && span_wide(max(em, ed + 3), (int)((mn >> (16 * h + 7)) & 0x1FF));
   }
   if (w == 0 && l < 16)
     *(int2*)(o.wshift + ((size_t)tensor * n_tr + tr) * 32 + (c >> 3) * 16 + 2 * (c & 7)) =
-        make_int2(sh[0], sh[1]);
+        make_int2(2 * sh[0] + wide[0], 2 * sh[1] + wide[1]);
   const float sd[2] = {exp2i(sh[0]), exp2i(sh[1])};
   auto put = [&](int ch, const uint32_t (&d)[8], const uint32_t (&m)[8]) {
     u32x4_t* du = o.u + ((((size_t)tensor * n_tr + tr) * n_ch + ch) * 4) * 64 + l;
@@ -321,7 +395,7 @@ __device__ __forceinline__ void prep_tile_row(const GemmArgs& a, const PqX& o, i
       for (int e = 0; e < 2; ++e) {
         const uint32_t dd = d[2 * j + e], mw = m[2 * j + e];
         const float d0 = bf16lo(dd) * sd[0], d1 = bf16hi(dd) * sd[1];
-        const uint32_t dp = pk_f16(d0, d1), ap = pk_f16(d0 * kPqLow, d1 * kPqHigh);
+        const uint32_t dp = pk_f16z(d0, d1), ap = pk_f16z(d0 * kPqLow, d1 * kPqHigh);
         const half2_t dh = as_h2(dp), ah = as_h2(ap);
         if (kPqChunkTiles * ch + s < a.k_t) ds[(2 * j + e) * 16] = make_uint2(dp, ap);
         u[0][e] = (bf16lo(mw) * sd[0] - fmaf(1024.f, (float)dh.x, (float)ah.x)) * (1 << kPqSum);
@@ -360,24 +434,35 @@ __device__ __forceinline__ void prep_tile_row_q8(const GemmArgs& a, const PqX& o
   const int l = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c = l & 15, s = l >> 4;
   const uint8_t* wr = a.w[0] + (size_t)tr * a.k_t * kQ8TileBytes + 128 * s + 4 * c;
-  uint32_t mx = 0;
+  uint32_t mx = 0, mn = ~0u;
   for (int kt = w; kt < a.k_t; kt += NW)
 #pragma unroll
-    for (int e = 0; e < 2; ++e)
-      mx = pk_max_u16(mx, *(const uint32_t*)(wr + (size_t)kt * kQ8TileBytes + 64 * e) & 0x7FFF7FFFu);
+    for (int e = 0; e < 2; ++e) {
+      const uint32_t v = *(const uint32_t*)(wr + (size_t)kt * kQ8TileBytes + 64 * e) & 0x7FFF7FFFu;
+      mx = pk_max_u16(mx, v);
+      mn = pk_min_u16(mn, v);
+    }
   mx = rows_max(mx);
-  if (l < 16) sm[w * 16 + l] = mx;
+  mn = rows_min(mn);
+  if (l < 16) {
+    sm[w * 32 + l] = mx;
+    sm[w * 32 + 16 + l] = mn;
+  }
   __syncthreads();
   if (w > 0 || l >= 16) return;
 #pragma unroll
-  for (int i = 1; i < NW; ++i) mx = pk_max_u16(mx, sm[16 * i + c]);
-  int sh[2];
+  for (int i = 1; i < NW; ++i) {
+    mx = pk_max_u16(mx, sm[32 * i + c]);
+    mn = pk_min_u16(mn, sm[32 * i + 16 + c]);
+  }
+  int sh[2], wide[2];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     const int e = (int)((mx >> (16 * h + 7)) & 0xFF);
     sh[h] = e < 255 ? min(kPqSTop - max(e, 1), 127) : 0;
+    wide[h] = e < 255 && span_wide(e, (int)((mn >> (16 * h + 7)) & 0xFF));
   }
-  *(int2*)(o.wshift + (size_t)tr * 32 + 2 * c) = make_int2(sh[0], sh[1]);
+  *(int2*)(o.wshift + (size_t)tr * 32 + 2 * c) = make_int2(2 * sh[0] + wide[0], 2 * sh[1] + wide[1]);
 }
 
 // First a weight tile-row per workgroup, over both tensors of [gate, up] -- the longer ones -- then
@@ -391,7 +476,7 @@ __device__ __forceinline__ void prep_tile_row_q8(const GemmArgs& a, const PqX& o
 template <int KIND, bool NORM, int C, int NT, int ROWS>
 __global__ __launch_bounds__(NT) void pq_prep_kernel(GemmArgs a, PqX o, int tile_rows) {
   __shared__ float sg[KIND == 4 ? NT / 4 * C : 1];
-  __shared__ uint32_t sm[NT / 2];
+  __shared__ uint32_t sm[NT / 64 * 48];         // (a tile-row's: 48 words of a wave)
   const int t = blockIdx.x, n = a.n_tr[0];
   if (t >= tile_rows) {
     constexpr int TR = NT / ROWS;                 // threads of a row: one wave, or all
@@ -436,6 +521,135 @@ template <int OFF>
 __device__ __forceinline__ void ldl4(const void* base, uint32_t voff, uint32_t lds, int add) {
   asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2 offset:%4"
                :: "s"(lds), "v"(voff), "s"(base), "i"(add - OFF), "i"(OFF) : "memory", "scc");
+}
+
+// A wave's tile without the powers of two, for rows and columns whose groups differ too far in size
+// (above, "Range"): per 32-K group the bf16 rows of x on exact bf16 codes (c - 8, or q) from zero, and
+// one FMA per output with the group's fp32 scale (q4: another with m + 8 d and the group's sum of x),
+// added up per K-tile. Everything comes through the caches as it is needed; the weights' tile goes
+// through the wave's LDS slot for the transposing read. All of K, MC m-tiles at a time, which the
+// waves of the K parts share out, each pass handed to `out`. One to two times the batched kernel's
+// time where every row is wide (8192 x 2560, 2048 rows 277 / 214 us, q8 324 / 349).
+template <int KIND, int MT, int RT, int WK, typename OUT>
+__device__ __forceinline__ void exact_tile(const GemmArgs& a, const PqX& p, uint8_t* slot,
+                                           const uint8_t* const (&wr)[RT], int m0, int wk, OUT&& out) {
+  constexpr int MW = MT > WK ? MT / WK : 1, MC = MW * RT > 4 ? 4 / RT : MW;
+  constexpr int TB = GemmFmt<KIND>::kTile, NLD = GemmFmt<KIND>::kLoads;
+  const int l = threadIdx.x & 63, c = l & 15, s = l >> 4;
+  const int tr_off = KIND == 4
+      ? GemmFmt<4>::kCodes + (c & 1) * 2048 + (8 * s + (c >> 1)) * 8
+      : GemmFmt<8>::kCodes + (8 * s + (c >> 1)) * 16 + (c & 1) * 8;
+  const int meta_off = KIND == 4 ? 2 * ((c >> 3) * 16 + 2 * (c & 7)) : 2 * c;
+  const int unit_steps = a.k_t * 8 + pq_chunks<KIND>(a.k_t) * 2;
+  const u32x4_t ones = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
+  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (int mp = wk * MC; mp < MT; mp += WK * MC) {
+    f32x4_t acc[RT][MC][2];
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int mt = 0; mt < MC; ++mt) acc[r][mt][0] = acc[r][mt][1] = zero;
+    // the lane's row of each m-tile: its bf16 entries, or (a row of a fused norm that is not wide)
+    // the pre-pass's fp16 ones under the power of two sh
+    const uint8_t* xr[MC];
+    int step[MC], sh[MC];
+#pragma unroll
+    for (int mt = 0; mt < MC; ++mt) {
+      const int row = min(m0 + 16 * (mp + mt) + c, a.m_rows - 1), r16 = row & 15;
+      const int x = p.exact_all ? 1 : p.xshift[row];
+      sh[mt] = x & 1 ? 256 : x >> 1;             // 256: bf16
+      step[mt] = x & 1 ? 64 : 1024;
+      xr[mt] = x & 1 ? (const uint8_t*)(p.exact + row * p.exact_stride + 8 * s)
+                     : (const uint8_t*)(p.xt + (size_t)(row >> 4) * unit_steps * 64 + r16 * 4 +
+                                        (s ^ ((r16 >> 1) & 3)));
+    }
+#pragma unroll 1
+    for (int kt = 0; kt < a.k_t; ++kt) {
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int i = 0; i < NLD; ++i) {
+          const int o = 16 * (64 * i + l);
+          if (o < TB) *(u32x4_t*)(slot + r * TB + o) = *(const u32x4_t*)(wr[r] + (size_t)kt * TB + o);
+        }
+      f32x4_t prt[RT][MC][2];
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int mt = 0; mt < MC; ++mt) prt[r][mt][0] = prt[r][mt][1] = zero;
+#pragma unroll 1
+      for (int kb = 0; kb < 8; ++kb) {
+        u32x4_t op[RT][2];
+        float d[RT][2], u[RT][2];
+#pragma unroll
+        for (int r = 0; r < RT; ++r) {
+          const uint8_t* sl = slot + r * TB;
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const i32x2_t cb = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
+                (lds_i32x2_t*)(sl + tr_off + (KIND == 4 ? kb * 256 : h * 4096 + kb * 512)));
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {        // entries 2 j and 2 j + 1
+              const uint32_t w = ((uint32_t)(j < 2 ? cb.x : cb.y)) >> (16 * (j & 1));
+              float f0, f1;
+              if constexpr (KIND == 4) {
+                f0 = (float)((w >> (4 * h)) & 15u) - 8.f;
+                f1 = (float)((w >> (8 + 4 * h)) & 15u) - 8.f;
+              } else {
+                f0 = (float)(int)(int8_t)w;
+                f1 = (float)(int)(int8_t)(w >> 8);
+              }
+              op[r][h][j] = perm(__float_as_uint(f1), __float_as_uint(f0), 0x07060302u);
+            }
+            if constexpr (KIND == 4) {
+              d[r][h] = bf16_to_f32(*(const uint16_t*)(sl + kb * 64 + meta_off + 2 * h));
+              u[r][h] = fmaf(8.f, d[r][h], bf16_to_f32(*(const uint16_t*)(sl + kMetaBytes + kb * 64 + meta_off + 2 * h)));
+            } else {
+              d[r][h] = bf16_to_f32(*(const uint16_t*)(sl + kb * 64 + h * 32 + meta_off));
+            }
+          }
+        }
+#pragma unroll
+        for (int mt = 0; mt < MC; ++mt) {
+          u32x4_t x = *(const u32x4_t*)(xr[mt] + (size_t)(kt * 8 + kb) * step[mt]);
+          if (sh[mt] < 256) {                    // entries k, k + 2 share a word there
+            u32x4_t y;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              const half2_t e0 = as_h2(x[j & 2]), e1 = as_h2(x[(j & 2) + 1]);
+              const float f0 = ldexpf((float)(j & 1 ? e0.y : e0.x), -sh[mt]);
+              const float f1 = ldexpf((float)(j & 1 ? e1.y : e1.x), -sh[mt]);
+              y[j] = perm(__float_as_uint(f1), __float_as_uint(f0), 0x07060302u);
+            }
+            x = y;
+          }
+          f32x4_t sx;
+          if constexpr (KIND == 4) sx = mfma_bf16(x, ones, zero);
+#pragma unroll
+          for (int r = 0; r < RT; ++r)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              const f32x4_t t = mfma_bf16(x, op[r][h], zero);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                prt[r][mt][h][e] = fmaf(d[r][h], t[e], prt[r][mt][h][e]);
+                if constexpr (KIND == 4) prt[r][mt][h][e] = fmaf(u[r][h], sx[e], prt[r][mt][h][e]);
+              }
+            }
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int mt = 0; mt < MC; ++mt)
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[r][mt][h][e] += prt[r][mt][h][e];
+    }
+    out(acc, m0 + 16 * mp);
+  }
 }
 
 // A workgroup of WN x WK waves takes 16 MT rows of X; wave (wn, wk) owns RT tile-rows (GATEUP:
@@ -587,9 +801,13 @@ __global__ __launch_bounds__(64 * WN * WK, OCC) void pq_kernel(GemmArgs a, PqX p
   int shw[RT][2];                              // the columns' powers of two
 #pragma unroll
   for (int r = 0; r < RT; ++r) {
-    shw[r][0] = p.wshift[(size_t)col0[r] * 32 + cols[0]];
-    shw[r][1] = p.wshift[(size_t)col0[r] * 32 + cols[1]];
+    shw[r][0] = p.wshift[(size_t)col0[r] * 32 + cols[0]] >> 1;
+    shw[r][1] = p.wshift[(size_t)col0[r] * 32 + cols[1]] >> 1;
   }
+  // whether a row of the block is wide: lane l looks at rows 2 l and 2 l + 1 (past X: anything)
+  const int row2 = m0 + 2 * min(l, 8 * MT - 1);
+  const int2 rows2 = *(const int2*)(p.xshift + row2);
+  const int wide_r = (row2 < a.m_rows ? rows2.x : 0) | (row2 + 1 < a.m_rows ? rows2.y : 0);
   // q8: the inner sums on their way to the totals (each LAG MFMAs after its own), the scales of
   // the steps of either parity, the columns' powers of two
   constexpr int LAG = 3;
@@ -674,8 +892,100 @@ __global__ __launch_bounds__(64 * WN * WK, OCC) void pq_kernel(GemmArgs a, PqX p
     pin_acc(acc[r][mt][h]);
   };
 
+  // ---- outputs: the lane's two columns are adjacent, so the 16 lanes of a row write 128
+  // contiguous bytes (64 of bf16; q8: 64 bytes per row block)
+  // (an output's address is a uniform row 16 mt + e plus the lane's 32-bit offset)
+  const uint32_t ly = (uint32_t)(4 * s * (OP == GOP_PLAIN ? a.y_stride : a.h_stride) + cols[0]);
+  // (v: RT x any number of m-tiles x 2, from row mb on; full: every row of them is one of X)
+  auto store_rows = [&](auto& v, int mb, auto fullc) {
+    constexpr bool FULL = decltype(fullc)::value;
+#pragma unroll
+    for (int mt = 0; mt < (int)(sizeof(v[0]) / sizeof(v[0][0])); ++mt)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int mu = mb + 16 * mt + e, m = mu + 4 * s;
+        const bool row_live = FULL || m < a.m_rows;
+        if constexpr (OP == GOP_PLAIN) {
+#pragma unroll
+          for (int r = 0; r < RT; ++r) {
+            if (tr[r] >= n_tr) continue;
+            const int64_t o = (int64_t)mu * a.y_stride + (int64_t)tr[r] * 32;
+            float2 o2 = make_float2(v[r][mt][0][e], v[r][mt][1][e]);
+            if (row_live) {
+              if (a.residual != nullptr) {
+                const float* rr = a.residual + o;
+                if constexpr (KIND == 4) {
+                  const float2 t = *(const float2*)(rr + ly);
+                  o2.x += t.x;
+                  o2.y += t.y;
+                } else {
+                  o2.x += rr[ly];
+                  o2.y += rr[ly + 16];
+                }
+              }
+              if (a.y != nullptr) {
+                float* yy = a.y + o;
+                if constexpr (KIND == 4) *(float2*)(yy + ly) = o2;
+                else {
+                  yy[ly] = o2.x;
+                  yy[ly + 16] = o2.y;
+                }
+              }
+            }
+            if (a.ssq_out != nullptr) {        // per 16-row block: 8 lanes (q8: 16, a column each)
+              float* so = a.ssq_out + (int64_t)m * n_tr * 2 + tr[r] * 2;
+              if constexpr (KIND == 4) {
+                float q = fmaf(o2.x, o2.x, o2.y * o2.y);
+                q += dpp<kDppXor1>(q);
+                q += dpp<kDppXor2>(q);
+                q += dpp<kDppHalfMirror>(q);
+                if (row_live && (c & 7) == 0) so[c >> 3] = q;
+              } else {
+                const float q0 = group16_sum(o2.x * o2.x), q1 = group16_sum(o2.y * o2.y);
+                if (row_live && c == 0) so[0] = q0, so[1] = q1;
+              }
+            }
+          }
+        } else {
+          if (tr[0] >= n_tr || !row_live) continue;
+          const int64_t N = (int64_t)n_tr * 32, n = (int64_t)tr[0] * 32;
+          const float g0 = v[0][mt][0][e], g1 = v[0][mt][1][e];
+          const float u0 = v[1][mt][0][e], u1 = v[1][mt][1][e];
+          *(uint32_t*)(a.h_out + (int64_t)mu * a.h_stride + n + ly) =
+              pack_bf16x2(swiglu(round_bf16_op(g0), round_bf16_op(u0)),
+                          swiglu(round_bf16_op(g1), round_bf16_op(u1)));
+          if (a.raw_out != nullptr) {
+            float* ro = a.raw_out + (int64_t)m * 2 * N + n + cols[0];
+            *(float2*)ro = make_float2(g0, g1);
+            *(float2*)(ro + N) = make_float2(u0, u1);
+          }
+        }
+      }
+  };
+  auto store = [&](auto& v, int mb, int rows) {
+    if (mb + rows <= a.m_rows) store_rows(v, mb, std::true_type{});
+    else store_rows(v, mb, std::false_type{});
+  };
+
   __builtin_amdgcn_s_waitcnt(vm_wait_pq(0));
   __syncthreads();
+  if (__builtin_expect(__any(wide_r & 1), 0)) {
+    // a column of the workgroup too: the tile by other means
+    int wide_c = 0;
+#pragma unroll
+    for (int i = 0; i < WN * RT * 32; i += 64) {
+      const int t = (i + l) >> 5;                // of the group's tile-rows (gate's, then up's)
+      const int ten = OP == GOP_PLAIN ? 0 : t / WN;
+      const int u = OP == GOP_PLAIN ? cgrp * WN * RT + t : cgrp * WN + t % WN;
+      if (i + l < WN * RT * 32 && u < n_tr) wide_c |= p.wshift[((size_t)ten * n_tr + u) * 32 + (l & 31)];
+    }
+    if (__any(wide_c & 1)) {
+      exact_tile<KIND, MT, RT, WK>(a, p, lds + wslot, wr, m0, wk, [&](auto& v, int mb) {
+        store_rows(v, mb, std::false_type{});
+      });
+      return;
+    }
+  }
   read_raw(0);
   read_raw(1);
 #pragma unroll
@@ -842,7 +1152,7 @@ __global__ __launch_bounds__(64 * WN * WK, OCC) void pq_kernel(GemmArgs a, PqX p
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     const int4 xs = *(const int4*)(p.xshift + m0 + 16 * mt + 4 * s);
-    const int xsh[4] = {xs.x, xs.y, xs.z, xs.w};
+    const int xsh[4] = {xs.x >> 1, xs.y >> 1, xs.z >> 1, xs.w >> 1};
 #pragma unroll
     for (int r = 0; r < RT; ++r)
 #pragma unroll
@@ -881,77 +1191,7 @@ __global__ __launch_bounds__(64 * WN * WK, OCC) void pq_kernel(GemmArgs a, PqX p
           }
   }
 
-  // ---- outputs: the lane's two columns are adjacent, so the 16 lanes of a row write 128
-  // contiguous bytes (64 of bf16; q8: 64 bytes per row block)
-  // (an output's address is a uniform row 16 mt + e plus the lane's 32-bit offset)
-  const uint32_t ly = (uint32_t)(4 * s * (OP == GOP_PLAIN ? a.y_stride : a.h_stride) + cols[0]);
-  auto store = [&](auto fullc) {               // full: every row of the block is one of X
-    constexpr bool FULL = decltype(fullc)::value;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int mu = m0 + 16 * mt + e, m = mu + 4 * s;
-        const bool row_live = FULL || m < a.m_rows;
-        if constexpr (OP == GOP_PLAIN) {
-#pragma unroll
-          for (int r = 0; r < RT; ++r) {
-            if (tr[r] >= n_tr) continue;
-            const int64_t o = (int64_t)mu * a.y_stride + (int64_t)tr[r] * 32;
-            float2 v = make_float2(acc[r][mt][0][e], acc[r][mt][1][e]);
-            if (row_live) {
-              if (a.residual != nullptr) {
-                const float* rr = a.residual + o;
-                if constexpr (KIND == 4) {
-                  const float2 t = *(const float2*)(rr + ly);
-                  v.x += t.x;
-                  v.y += t.y;
-                } else {
-                  v.x += rr[ly];
-                  v.y += rr[ly + 16];
-                }
-              }
-              if (a.y != nullptr) {
-                float* yy = a.y + o;
-                if constexpr (KIND == 4) *(float2*)(yy + ly) = v;
-                else {
-                  yy[ly] = v.x;
-                  yy[ly + 16] = v.y;
-                }
-              }
-            }
-            if (a.ssq_out != nullptr) {        // per 16-row block: 8 lanes (q8: 16, a column each)
-              float* so = a.ssq_out + (int64_t)m * n_tr * 2 + tr[r] * 2;
-              if constexpr (KIND == 4) {
-                float q = fmaf(v.x, v.x, v.y * v.y);
-                q += dpp<kDppXor1>(q);
-                q += dpp<kDppXor2>(q);
-                q += dpp<kDppHalfMirror>(q);
-                if (row_live && (c & 7) == 0) so[c >> 3] = q;
-              } else {
-                const float q0 = group16_sum(v.x * v.x), q1 = group16_sum(v.y * v.y);
-                if (row_live && c == 0) so[0] = q0, so[1] = q1;
-              }
-            }
-          }
-        } else {
-          if (tr[0] >= n_tr || !row_live) continue;
-          const int64_t N = (int64_t)n_tr * 32, n = (int64_t)tr[0] * 32;
-          const float g0 = acc[0][mt][0][e], g1 = acc[0][mt][1][e];
-          const float u0 = acc[1][mt][0][e], u1 = acc[1][mt][1][e];
-          *(uint32_t*)(a.h_out + (int64_t)mu * a.h_stride + n + ly) =
-              pack_bf16x2(swiglu(round_bf16_op(g0), round_bf16_op(u0)),
-                          swiglu(round_bf16_op(g1), round_bf16_op(u1)));
-          if (a.raw_out != nullptr) {
-            float* ro = a.raw_out + (int64_t)m * 2 * N + n + cols[0];
-            *(float2*)ro = make_float2(g0, g1);
-            *(float2*)(ro + N) = make_float2(u0, u1);
-          }
-        }
-      }
-  };
-  if (m0 + 16 * MT <= a.m_rows) store(std::true_type{});
-  else store(std::false_type{});
+  store(acc, m0, 16 * MT);
 }
 
 // ---------------------------------------------------------------- host side
@@ -960,7 +1200,7 @@ size_t pq_align(size_t b) { return (b + 255) & ~(size_t)255; }
 int pq_mtiles(int m_rows) { return (m_rows + 127) / 128 * 8; }   // whole 128-row blocks
 
 // The pre-pass's buffers in a workspace (nullptr: their total size)
-size_t pq_layout(void* ws, int kind, int tensors, int n_tr, int k_t, int m_rows, PqX* x) {
+size_t pq_layout(void* ws, int kind, int tensors, int n_tr, int k_t, int m_rows, bool xe, PqX* x) {
   const size_t mt = pq_mtiles(m_rows), tr = (size_t)tensors * n_tr;
   const size_t ch = kind == Q4NX_KIND_Q4 ? pq_chunks<4>(k_t) : pq_chunks<8>(k_t);
   size_t off = 0;
@@ -974,6 +1214,7 @@ size_t pq_layout(void* ws, int kind, int tensors, int n_tr, int k_t, int m_rows,
   x->scale = (uint2*)take(kind == Q4NX_KIND_Q4 ? tr * k_t * 1024 : 0);
   x->xshift = (int*)take(mt * 16 * 4);
   x->wshift = (int*)take(tr * 32 * 4);
+  x->xe = (uint16_t*)take(xe ? (size_t)m_rows * k_t * kTileK * 2 : 0);
   return off;
 }
 
@@ -1014,9 +1255,9 @@ void pq_prep(const GemmArgs& a, const PqX& x, int tensors, hipStream_t st) {
 
 }  // namespace
 
-size_t pq_ws_bytes(int kind, int op, int n_tile_rows, int k_t, int m_rows) {
+size_t pq_ws_bytes(int kind, int op, int n_tile_rows, int k_t, int m_rows, bool own_norm) {
   PqX x;
-  return pq_layout(nullptr, kind, op == GOP_GATEUP ? 2 : 1, n_tile_rows, k_t, m_rows, &x);
+  return pq_layout(nullptr, kind, op == GOP_GATEUP ? 2 : 1, n_tile_rows, k_t, m_rows, own_norm, &x);
 }
 
 bool pq_use(int kind, int op, const GemmArgs& a) {
@@ -1117,8 +1358,11 @@ static void pq_gateup(const GemmArgs& a, const PqX& x, hipStream_t st) {
 void pq_launch(int kind, int op, const GemmArgs& a, void* ws, hipStream_t st) {
   PqX x;
   const int tensors = op == GOP_GATEUP ? 2 : 1;
-  pq_layout(ws, kind, tensors, a.n_tr[0], a.k_t, a.m_rows, &x);
-  const bool norm = a.norm_w != nullptr;
+  const bool norm = a.norm_w != nullptr, own = norm && a.xn_out == nullptr;
+  pq_layout(ws, kind, tensors, a.n_tr[0], a.k_t, a.m_rows, own, &x);
+  x.exact = !norm ? a.x : own ? x.xe : a.xn_out;
+  x.exact_stride = own ? (int64_t)a.k_t * kTileK : a.x_stride;
+  x.exact_all = !own;
   if (kind == Q4NX_KIND_Q8) norm ? pq_prep<8, true>(a, x, tensors, st) : pq_prep<8, false>(a, x, tensors, st);
   else norm ? pq_prep<4, true>(a, x, tensors, st) : pq_prep<4, false>(a, x, tensors, st);
   if (op == GOP_GATEUP) pq_gateup(a, x, st);

@@ -632,3 +632,120 @@ def test_gemm_large_tiles_parity(dev, m, n, k):
 ])
 def test_gate_up_large_tiles(dev, batch, n, k):
     test_gate_up_fp16_operands(dev, batch, n, k, False)
+
+
+# ------------------------------------------------------------------ any range within a row or column
+# Under one power of two per row of x and per column of the weights an fp16 operand reaches some
+# 2^30 below the largest entry. Where both a row's and a column's 32-K groups lie further apart than
+# 2^10 the kernel adds the tile up with the groups' own fp32 scales.
+
+def _group_scaled(raw, f):
+    """Tiles with the scales (and minima) of every 32-K group divided by the power of two f[group]."""
+    q4 = raw.shape[1] == qo.Q4_TILE_BYTES
+    kt = f.size // 8
+    out = raw.copy()
+    for p in range(2 if q4 else 1):
+        v = qo.bf16_to_f32(raw[:, 512 * p:512 * p + 512].copy().view(np.uint16)).astype(np.float64)
+        v = v.reshape(-1, kt, 8, 32) / f.reshape(1, kt, 8, 1)
+        out[:, 512 * p:512 * p + 512] = synth.f32_to_bf16_bits(
+            v.astype(np.float32).reshape(raw.shape[0], 256)).view(np.uint8).reshape(-1, 512)
+    return out
+
+
+def _close_per_output(y, raw, kind, x, n_t, k_t, rows, d_weight):
+    """|y - ref| against the size of the output's own terms, 24 roundings of 2^-24: |x| on |w| and,
+    for q4, on the codes' offset times the group's own scale."""
+    w = qo.dequant_matrix(raw, kind, n_t, k_t).astype(np.float64)
+    xf = qo.bf16_to_f32(x[rows]).astype(np.float64)
+    size = np.abs(xf) @ (np.abs(w) + d_weight).T
+    err = np.abs(y[rows].astype(np.float64) - xf @ w.T)
+    assert (err <= 24 * 2.0 ** -24 * size).all(), float((err / size).max() * 2 ** 24)
+
+
+ANY_RANGE = [
+    (80, 544, 2816),      # 32 x 1, eight K parts
+    (129, 2080, 768),     # 32 x 2, four parts
+    (257, 2080, 1280),    # 64 x 2, four parts
+    (449, 2592, 768),     # 64 x 2, two parts
+    (130, 128, 8448),     # rows longer than the pre-pass keeps in registers
+    (1500, 2464, 256),    # 64 x 4
+    (2100, 4128, 768),    # 128 rows
+    (1900, 4320, 2304),   # 128 x 8, two parts (q4)
+    (2100, 4128, 2304),   # 128 x 8, one part (q4)
+]
+
+
+@pytest.mark.parametrize("kind", ["q4", "q8"])
+@pytest.mark.parametrize("m,n,k,spread", [(*c, s) for c in ANY_RANGE for s in (4, 10, 11, 30, 70)
+                                          if c[0] < 1000 or s in (10, 11, 70)])
+def test_prompt_blocks_any_range(dev, kind, m, n, k, spread):
+    """Groups of the weights up to 2^spread apart, x the other way round in two rows of three (every
+    group contributes as much) and as it was in the third."""
+    raw, rng = _tiles(kind, n, k, 300 + m + spread)
+    f = 2.0 ** (rng.integers(0, spread + 1, k // 32) - spread // 2)
+    f[:2] = 2.0 ** (spread - spread // 2), 2.0 ** -(spread // 2)
+    raw = _group_scaled(raw, f)
+    xf = rng.standard_normal((m, k))
+    xf[np.arange(m) % 3 < 2] *= np.repeat(f, 32)
+    x = qo.bf16_round(xf.astype(np.float32))
+    y = ops.gemm(_dev_u8(raw, dev), kind, _dev_bf16(x, dev), n // 32, k // 256).cpu().numpy()
+    rows = np.unique(np.concatenate([np.arange(0, m, max(1, m // 12)), [m - 2, m - 1]]))
+    ones = raw.copy()      # the group scales alone: every code 1 (and no minimum), times 16
+    if kind == "q4":
+        ones[:, 512:1024], ones[:, 1024:] = 0, 0x11
+        d = 16 * np.abs(qo.dequant_matrix(ones, kind, n // 32, k // 256).astype(np.float64))
+    else:
+        d = 0.0
+    _close_per_output(y, raw, kind, x, n // 32, k // 256, rows, d)
+
+
+@pytest.mark.parametrize("kind", ["q4", "q8"])
+def test_prompt_block_outlier_on_pruned_group(dev, kind):
+    """An entry 1e12 times the rest on a group whose weights are all zero leaves the others' sum."""
+    m, n, k = 200, 2592, 1024
+    raw, rng = _tiles(kind, n, k, 17)
+    raw = raw.copy().reshape(n // 32, k // 256, -1)
+    for p in range(2 if kind == "q4" else 1):          # group 3 of K-tile 1
+        raw[:, 1, 512 * p + 64 * 3:512 * p + 64 * 4] = 0
+    raw = raw.reshape(-1, raw.shape[-1])
+    xf = rng.standard_normal((m, k)).astype(np.float32)
+    xf[::2, 256 + 96 + 5] = 1e12
+    x = qo.bf16_round(xf)
+    y = ops.gemm(_dev_u8(raw, dev), kind, _dev_bf16(x, dev), n // 32, k // 256).cpu().numpy()
+    _check_rows(y, qo.gemv(raw, kind, x, n // 32, k // 256, acc=np.float64))
+
+
+@pytest.mark.parametrize("own", [True, False])
+@pytest.mark.parametrize("batch,n,k", [(65, 96, 1024), (300, 2080, 2816), (900, 1984, 1280),
+                                       (1000, 3616, 2304)])
+def test_gate_up_any_range_norm(dev, own, batch, n, k):
+    """[RMSNorm, gate, up] with the norm's weights and the tiles' scales 2^40 apart the other way
+    round, the normalised rows taken by the caller or not: raw_out per output, h from raw_out."""
+    rng = np.random.default_rng(400 + batch)
+    f = 2.0 ** (rng.integers(0, 41, k // 32) - 20)
+    g = _group_scaled(synth.q4_tiles(rng, n, k).reshape(-1, qo.Q4_TILE_BYTES), f)
+    u = _group_scaled(synth.q4_tiles(rng, n, k).reshape(-1, qo.Q4_TILE_BYTES), f)
+    h = rng.standard_normal((batch, k)).astype(np.float32)
+    h[1::3] /= np.repeat(f, 32)[None].astype(np.float32)   # rows that come out narrow
+    x = torch.from_numpy(h).to(dev)
+    nw = synth.f32_to_bf16_bits(np.repeat(f, 32).astype(np.float32))
+    kw = dict(norm_w=_dev_bf16(nw, dev), ssq_in=x.view(batch, -1, 16).square().sum(-1).contiguous())
+    raw_out = torch.empty((batch, 2 * n), device=dev)
+    xn = torch.zeros((batch, k), dtype=torch.bfloat16, device=dev)
+    wg, wu = _dev_u8(g, dev), _dev_u8(u, dev)
+    out = ops.gate_up_swiglu(wg, wu, n // 32, k // 256, x, raw_out=raw_out, **kw,
+                             **({} if own else {"xn_out": xn}))
+    if own:      # the rows it normalised, from a call that gives them
+        ops.gate_up_swiglu(wg, wu, n // 32, k // 256, x, xn_out=xn, **kw)
+    xb = xn.view(torch.int16).cpu().numpy().view(np.uint16)
+    rows = np.unique(np.concatenate([np.arange(0, batch, max(1, batch // 12)), [1, 4, batch - 1]]))
+    got = raw_out.cpu().numpy()
+    for w, o in ((g, 0), (u, n)):
+        ones = w.copy()
+        ones[:, 512:1024], ones[:, 1024:] = 0, 0x11
+        d = 16 * np.abs(qo.dequant_matrix(ones, "q4", n // 32, k // 256).astype(np.float64))
+        _close_per_output(got[:, o:o + n], w, "q4", xb, n // 32, k // 256, rows, d)
+    narrow = lambda t: t.to(torch.bfloat16).double()
+    gv, uv = narrow(raw_out[:, :n]), narrow(raw_out[:, n:])
+    want = gv / (1 + torch.exp(-gv)) * uv
+    assert ((out.double() - want).abs() <= want.abs() * (2.0 ** -8 + 2.0 ** -20) + 1e-38).all()
