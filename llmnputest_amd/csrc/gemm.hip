@@ -765,6 +765,26 @@ static void gemm_launch_op(const GemmArgs& a, const GemmPlan& p, hipStream_t st)
   else if constexpr (OP == GOP_PLAIN) gemm_launch_t<KIND, OP, 1, 2, 1>(a, p, st);
 }
 
+// Whether a prompt block is the fp16-operand kernel's, by its shape and the policy. That kernel takes
+// two launches; up to K = 512 they do not repay themselves while the batched kernel's one fits the
+// chip at once or the columns are few (a stream of calls, us, batched / fp16 operands; N x K, rows):
+// q8 1024 x 512, 1000 rows (256 workgroups) 10.8 / 12.4, 1500 rows (384) 15.0 / 13.1; q4 2048 x 512,
+// 96 rows 11.8 / 12.3, 128 rows 13.0 / 12.4; 512 x 512, 3000 rows q4 13.8 / 16.9, q8 15.1 / 15.9.
+// A K split that the policy names is the batched kernel's, but 1 asks for what this one does anyway,
+// and a projection that fills the chip without a split is not slowed down for it (8192 x 2560, 2048
+// rows 86 us, batched 214).
+static bool pq_wanted(int kind, int op, int n_tr, int k_t, int m_rows, bool ssq, const GemmPlan& p,
+                      const Policy& P) {
+  if (op == GOP_QKV || m_rows < kPqRows) return false;
+  const bool short_k = op == GOP_PLAIN && k_t <= 2 &&
+                       (n_tr <= 16 || (kind == Q4NX_KIND_Q8 ? p.groups * p.m_blocks <= 256
+                                                            : m_rows <= 96));
+  if (short_k) return false;
+  if (P.gemm_ksplit == 0) return true;
+  const bool fills = m_rows >= 128 && (int64_t)((n_tr + 3) / 4) * ((m_rows + 63) / 64) >= 512;
+  return op == GOP_PLAIN && (P.gemm_ksplit == 1 || (fills && !ssq));
+}
+
 // Whether `rows` rows of `kind` run on the matrix cores under the policy (mfma_rows: 0 never).
 bool mfma_use(int kind, int rows, const Policy& P) {
   const int t = P.mfma_rows[kind == Q4NX_KIND_Q8 ? 1 : 0];
@@ -774,8 +794,10 @@ bool mfma_use(int kind, int rows, const Policy& P) {
 size_t mfma_ws_bytes(int kind, int op, int n_units, int k_t, int m_rows, const Policy& P) {
   // room for the split-K records and the normalised rows of an RMSNorm prologue or, for a prompt
   // block, for what the fp16-operand kernel keeps
-  const size_t split = split_part_bytes(plan_gemm(kind, op, n_units, k_t, m_rows, P));
-  const size_t pq = op != GOP_QKV && m_rows >= kPqRows ? pq_ws_bytes(kind, op, n_units, k_t, m_rows, k_t * kTileK / kSsqRows <= 512) : 0;
+  const GemmPlan p = plan_gemm(kind, op, n_units, k_t, m_rows, P);
+  const size_t split = split_part_bytes(p);
+  const size_t pq = pq_wanted(kind, op, n_units, k_t, m_rows, false, p, P)
+                        ? pq_ws_bytes(kind, op, n_units, k_t, m_rows, k_t * kTileK / kSsqRows <= 512) : 0;
   const size_t b = align256(split) + align256((size_t)m_rows * k_t * kTileK * 2);
   return Q4NX_WS_COUNTER_BYTES + (pq > b ? pq : b);
 }
@@ -797,17 +819,8 @@ int mfma_launch(int kind, int op, GemmArgs& a, int n_units, void* ws, size_t ws_
   const size_t xn_b = a.norm_w != nullptr && a.xn_out == nullptr
                           ? align256((size_t)a.m_rows * K * 2) : 0;
   const bool ws_ok = ws != nullptr && Q4NX_ALIGNED(ws, 256);
-  // The fp16-operand kernel takes two launches; up to K = 512 they do not repay themselves while
-  // the batched kernel's one fits the chip at once or the columns are few (a stream of calls, us,
-  // batched / fp16 operands; N x K, rows): q8 1024 x 512, 1000 rows (256 workgroups) 10.8 / 12.4,
-  // 1500 rows (384) 15.0 / 13.1; q4 2048 x 512, 96 rows 11.8 / 12.3, 128 rows 13.0 / 12.4; 512 x
-  // 512, 3000 rows q4 13.8 / 16.9, q8 15.1 / 15.9
-  const bool short_k = op == GOP_PLAIN && a.k_t <= 2 &&
-                       (a.n_tr[0] <= 16 || (kind == Q4NX_KIND_Q8 ? p.groups * p.m_blocks <= 256
-                                                                 : a.m_rows <= 96));
-  // a prompt block: the fp16-operand kernel, when the workspace holds what it keeps
-  // there (a K split that the policy names belongs to the batched kernel)
-  if (pq_use(kind, op, a) && ws_ok && P.gemm_ksplit == 0 && !short_k &&
+  // a prompt block: the fp16-operand kernel, when the workspace holds what it keeps there
+  if (pq_use(kind, op, a) && ws_ok && pq_wanted(kind, op, a.n_tr[0], a.k_t, a.m_rows, a.ssq_out != nullptr, p, P) &&
       (a.norm_w == nullptr || (a.ssq_in != nullptr && K / kSsqRows <= 512)) &&
       ws_bytes >= Q4NX_WS_COUNTER_BYTES + pq_ws_bytes(kind, op, a.n_tr[0], a.k_t, a.m_rows, xn_b != 0)) {
     pq_launch(kind, op, a, (uint8_t*)ws + Q4NX_WS_COUNTER_BYTES, st);
@@ -871,22 +884,31 @@ int mfma_launch(int kind, int op, GemmArgs& a, int n_units, void* ws, size_t ws_
 
 using namespace q4nx;
 
+static bool gemm_shape_ok(int kind, int n_tile_rows, int k_tiles, int m_rows) {
+  return (kind == Q4NX_KIND_Q4 || kind == Q4NX_KIND_Q8) && n_tile_rows >= 1 && k_tiles >= 1 &&
+         m_rows >= 1;
+}
+
 extern "C" {
 
 size_t q4nx_gemm_ws_bytes(int kind, int n_tile_rows, int k_tiles, int m_rows,
                           const q4nx_policy* policy) {
   Policy P;
-  if ((kind != Q4NX_KIND_Q4 && kind != Q4NX_KIND_Q8) || n_tile_rows < 1 || k_tiles < 1 ||
-      m_rows < 1 || !resolve_policy_quiet(policy, &P))
-    return 0;
-  const size_t split = gemm_split_bytes(plan_gemm(kind, GOP_PLAIN, n_tile_rows, k_tiles, m_rows, P));
-  // a launch that fills the chip without a split: what the fp16-operand kernel keeps
-  return split ? split : q4nx_gemm_prompt_ws_bytes(kind, n_tile_rows, k_tiles, m_rows);
+  if (!gemm_shape_ok(kind, n_tile_rows, k_tiles, m_rows) || !resolve_policy_quiet(policy, &P)) return 0;
+  const GemmPlan p = plan_gemm(kind, GOP_PLAIN, n_tile_rows, k_tiles, m_rows, P);
+  const size_t split = gemm_split_bytes(p);
+  if (!pq_wanted(kind, GOP_PLAIN, n_tile_rows, k_tiles, m_rows, false, p, P)) return split;
+  const size_t pq = Q4NX_WS_COUNTER_BYTES + pq_ws_bytes(kind, GOP_PLAIN, n_tile_rows, k_tiles, m_rows, false);
+  // a launch that fills the chip without a split: what the fp16-operand kernel keeps; an automatic
+  // split: the batched kernel's records (q4nx_gemm_prompt_ws_bytes has the other)
+  return split == 0 ? pq : P.gemm_ksplit > 1 && pq > split ? pq : split;
 }
 
 size_t q4nx_gemm_prompt_ws_bytes(int kind, int n_tile_rows, int k_tiles, int m_rows) {
-  if ((kind != Q4NX_KIND_Q4 && kind != Q4NX_KIND_Q8) || n_tile_rows < 1 || k_tiles < 1 ||
-      m_rows < kPqRows)
+  Policy P;
+  if (!gemm_shape_ok(kind, n_tile_rows, k_tiles, m_rows) || !resolve_policy_quiet(nullptr, &P) ||
+      !pq_wanted(kind, GOP_PLAIN, n_tile_rows, k_tiles, m_rows, false,
+                 plan_gemm(kind, GOP_PLAIN, n_tile_rows, k_tiles, m_rows, P), P))
     return 0;
   return Q4NX_WS_COUNTER_BYTES + pq_ws_bytes(kind, GOP_PLAIN, n_tile_rows, k_tiles, m_rows, false);
 }

@@ -48,9 +48,9 @@ def policy_scope(policy: Policy | None):
         _POLICY.reset(tok)
 
 
-def current_policy() -> Policy:
-    """The policy an op called here without `policy=` would use."""
-    p = _POLICY.get()
+def current_policy(policy: Policy | None = None) -> Policy:
+    """The policy an op called here with this `policy=` would use."""
+    p = policy if policy is not None else _POLICY.get()
     return p if p is not None else Policy()
 
 
@@ -244,7 +244,7 @@ def gemm(tiles: torch.Tensor, kind: str, x: torch.Tensor, n_tile_rows: int, k_ti
             raise ValueError("residual must have the shape of the output")
     pol = _pol(policy)
     need = _lib.lib().q4nx_gemm_ws_bytes(KIND[kind], n_tile_rows, k_tiles, m, pol)
-    if m > 64:
+    if m > 64 and (pol is None or current_policy(policy).gemm_ksplit == 0):
         need = max(need, _lib.lib().q4nx_gemm_prompt_ws_bytes(KIND[kind], n_tile_rows, k_tiles, m))
     ws, wp, wn, stream = _scratch(ws, need)
     _lib.call("q4nx_gemm", KIND[kind], _ptr(tiles), n_tile_rows, k_tiles, _ptr(x2), x2.stride(0),

@@ -268,3 +268,22 @@ def test_rope_table_host_closed_forms():
         _lib.call("q4nx_rope_table_host", tab.ctypes.data, max_pos, hd, C.c_double(theta))
         return tab
     check_rope_frequencies(c_table)
+
+
+def test_prompt_workspace_queries_ask_for_what_is_used():
+    """Prompt blocks that the batched kernel takes (a named K split, a short K) ask for its own
+    workspace only; gemm_ksplit=1 and projections that fill the chip ask as by default."""
+    f, g = _lib.lib().q4nx_gemm_ws_bytes, _lib.lib().q4nx_gemm_prompt_ws_bytes
+    q4, q8 = 4, 8
+    full = f(q4, 256, 10, 2048, None)
+    assert full == g(q4, 256, 10, 2048) > 10 << 20
+    for parts in (1, 2, 8):
+        assert f(q4, 256, 10, 2048, pol(gemm_ksplit=parts)) >= full
+    assert f(q4, 80, 10, 100, pol(gemm_ksplit=1)) == g(q4, 80, 10, 100) > 0
+    # 80 groups of one row block in two parts: counters and 2 x 128 x 32 floats each, no more
+    assert f(q4, 80, 10, 100, pol(gemm_ksplit=2)) <= 65536 + 80 * 2 * 128 * 64 * 4
+    assert g(q8, 16, 2, 1000) == 0 and f(q8, 16, 2, 1000, None) == 0
+    assert g(q4, 64, 2, 96) == 0 and g(q4, 64, 2, 97) > 0
+    # [gate, up] under a named split is the batched kernel's: its normalised rows alone
+    h = _lib.lib().q4nx_gate_up_ws_bytes
+    assert h(256, 10, 500, pol(gemm_ksplit=1)) == 65536 + 500 * 2560 * 2 < h(256, 10, 500, None)

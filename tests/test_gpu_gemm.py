@@ -749,3 +749,19 @@ def test_gate_up_any_range_norm(dev, own, batch, n, k):
     gv, uv = narrow(raw_out[:, :n]), narrow(raw_out[:, n:])
     want = gv / (1 + torch.exp(-gv)) * uv
     assert ((out.double() - want).abs() <= want.abs() * (2.0 ** -8 + 2.0 ** -20) + 1e-38).all()
+
+
+@pytest.mark.parametrize("kind", ["q4", "q8"])
+@pytest.mark.parametrize("m,n,k,parts", [(2048, 8192, 512, 1), (2048, 8192, 512, 3), (100, 2560, 2560, 1)])
+def test_prompt_block_keeps_its_kernel_under_a_ksplit(dev, kind, m, n, k, parts):
+    """gemm_ksplit 1, and any on a projection that fills the chip by itself: the bits of the default
+    policy's kernel (which the batched kernel's differ from)."""
+    from llmnputest_amd import _lib
+    raw, rng = _tiles(kind, n, k, 77)
+    w, xd = _dev_u8(raw, dev), _dev_bf16(synth.random_bf16(rng, (m, k)), dev)
+    want = ops.gemm(w, kind, xd, n // 32, k // 256)
+    assert torch.equal(ops.gemm(w, kind, xd, n // 32, k // 256, policy=ops.Policy(gemm_ksplit=parts)), want)
+    y = torch.empty_like(want)
+    _lib.call("q4nx_gemm", ops.KIND[kind], w.data_ptr(), n // 32, k // 256, xd.data_ptr(), k, m,
+              y.data_ptr(), n, None, None, 0, None, ops._stream())
+    assert not torch.equal(y, want)
