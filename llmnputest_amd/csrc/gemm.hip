@@ -766,20 +766,26 @@ static void gemm_launch_op(const GemmArgs& a, const GemmPlan& p, hipStream_t st)
 }
 
 // Whether a prompt block is the fp16-operand kernel's, by its shape and the policy. That kernel takes
-// two launches; up to K = 512 they do not repay themselves while the batched kernel's one fits the
-// chip at once or the columns are few (a stream of calls, us, batched / fp16 operands; N x K, rows):
-// q8 1024 x 512, 1000 rows (256 workgroups) 10.8 / 12.4, 1500 rows (384) 15.0 / 13.1; q4 2048 x 512,
-// 96 rows 11.8 / 12.3, 128 rows 13.0 / 12.4; 512 x 512, 3000 rows q4 13.8 / 16.9, q8 15.1 / 15.9.
+// two launches; up to K = 512 they do not repay themselves while the batched kernel's one holds few
+// workgroups (groups x row blocks) or the columns are few. A stream of calls, us, batched / fp16
+// operands (N x K, rows, workgroups):
+//   K = 256: q4 8192, 512 rows (512) 14.1 / 13.7, 256 rows (256) 10.3 / 12.5; 49152, 96 rows (768)
+//   18.6 / 19.0, 128 rows 20.1 / 19.6; 1024, 6000 rows (752) 20.3 / 21.0; q8 4096, 512 rows (512) 10.3 /
+//   11.3, 1000 rows (1024) 15.7 / 13.0; 1024, 6000 rows (1504) 21.3 / 26.3
+//   K = 512: q4 16384, 96 rows (256) 12.8 / 13.8, 49152, 65 rows (768) 24.6 / 22.1, 2048, 128 rows 12.9 /
+//   9.7, 96 rows 11.9 / 9.6 (a program that makes these calls one by one from Python waits 2.5 us
+//   longer for the second launch: 11.8 / 12.3); q8 2048, 512 rows (256) 10.8 / 11.1, 1000 rows (512)
+//   15.5 / 12.8; 512 columns, 6000 rows q4 20.4 / 23.4, q8 20.8 / 22.6
 // A K split that the policy names is the batched kernel's, but 1 asks for what this one does anyway,
 // and a projection that fills the chip without a split is not slowed down for it (8192 x 2560, 2048
 // rows 86 us, batched 214).
 static bool pq_wanted(int kind, int op, int n_tr, int k_t, int m_rows, bool ssq, const GemmPlan& p,
                       const Policy& P) {
   if (op == GOP_QKV || m_rows < kPqRows) return false;
-  const bool short_k = op == GOP_PLAIN && k_t <= 2 &&
-                       (n_tr <= 16 || (kind == Q4NX_KIND_Q8 ? p.groups * p.m_blocks <= 256
-                                                            : m_rows <= 96));
-  if (short_k) return false;
+  const bool q8 = kind == Q4NX_KIND_Q8;
+  const int wgs = p.groups * p.m_blocks;
+  if (op == GOP_PLAIN && k_t == 1 && (n_tr <= 32 || wgs <= 512 || (!q8 && m_rows <= 96))) return false;
+  if (op == GOP_PLAIN && k_t == 2 && (n_tr <= 16 || (wgs <= 256 && (q8 || m_rows <= 96)))) return false;
   if (P.gemm_ksplit == 0) return true;
   const bool fills = m_rows >= 128 && (int64_t)((n_tr + 3) / 4) * ((m_rows + 63) / 64) >= 512;
   return op == GOP_PLAIN && (P.gemm_ksplit == 1 || (fills && !ssq));

@@ -284,6 +284,10 @@ def test_prompt_workspace_queries_ask_for_what_is_used():
     assert f(q4, 80, 10, 100, pol(gemm_ksplit=2)) <= 65536 + 80 * 2 * 128 * 64 * 4
     assert g(q8, 16, 2, 1000) == 0 and f(q8, 16, 2, 1000, None) == 0
     assert g(q4, 64, 2, 96) == 0 and g(q4, 64, 2, 97) > 0
+    # K <= 512 stays on the batched kernel up to a number of its workgroups, not of rows alone
+    assert g(q4, 512, 2, 96) == 0 and g(q4, 3136, 2, 96) > 0 and g(q4, 3136, 2, 65) > 0
+    assert g(q4, 256, 1, 256) == 0 and g(q4, 512, 1, 300) > 0 and g(q4, 32, 1, 6000) == 0
+    assert g(q8, 128, 1, 512) == 0 and g(q8, 128, 1, 513) > 0
     # [gate, up] under a named split is the batched kernel's: its normalised rows alone
     h = _lib.lib().q4nx_gate_up_ws_bytes
     assert h(256, 10, 500, pol(gemm_ksplit=1)) == 65536 + 500 * 2560 * 2 < h(256, 10, 500, None)

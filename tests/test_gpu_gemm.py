@@ -391,7 +391,10 @@ def test_gemm_q8_fp16_operands_parity(dev, m, n, k):
 
 @pytest.mark.parametrize("kind,m,n,k", [("q8", 256, 4096, 512), ("q8", 257, 4096, 512),
                                         ("q4", 96, 2048, 512), ("q4", 97, 2048, 512),
-                                        ("q4", 200, 512, 512), ("q4", 200, 512, 768)])
+                                        ("q4", 200, 512, 512), ("q4", 200, 512, 768),
+                                        ("q4", 90, 16384, 512), ("q4", 90, 16416, 512),
+                                        ("q4", 128, 16384, 256), ("q4", 300, 16448, 256),
+                                        ("q8", 512, 4096, 256), ("q8", 513, 4096, 256)])
 def test_gemm_short_k_either_side(dev, kind, m, n, k):
     """Both sides of the short-K line between the batched and the fp16-operand kernel."""
     raw, rng = _tiles(kind, n, k, 7 + m)
