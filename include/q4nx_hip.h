@@ -161,6 +161,9 @@ int q4nx_gemv_attn_q4(const uint8_t *w, int n_tile_rows, const float *att_rec, i
  *   fastest with q4nx_gemm_prompt_ws_bytes(...) bytes where that is more: the fp16-operand
  *   kernel keeps its form of x there; with less they take the batched kernel. */
 size_t q4nx_gemm_prompt_ws_bytes(int kind, int n_tile_rows, int k_tiles, int m_rows);
+/* The workgroup tile a prompt block takes with that workspace under the default policy: rows of x
+ * << 16 | tile-rows << 8 | K parts; 0: it is the batched kernel's. */
+int q4nx_gemm_prompt_tile(int kind, int n_tile_rows, int k_tiles, int m_rows);
 size_t q4nx_gemm_ws_bytes(int kind, int n_tile_rows, int k_tiles, int m_rows,
                           const q4nx_policy *policy);
 int q4nx_gemm(int kind, const uint8_t *w, int n_tile_rows, int k_tiles, const uint16_t *x,

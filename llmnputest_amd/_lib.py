@@ -67,6 +67,7 @@ SIGNATURES: dict[str, tuple] = {
                            c_p, c_p, c_p, c_sz, c_pol, c_p]),
     "q4nx_gemm_ws_bytes": (c_sz, [c_i, c_i, c_i, c_i, c_pol]),
     "q4nx_gemm_prompt_ws_bytes": (c_sz, [c_i, c_i, c_i, c_i]),
+    "q4nx_gemm_prompt_tile": (c_i, [c_i, c_i, c_i, c_i]),
     "q4nx_gemm": (c_i, [c_i, c_p, c_i, c_i, c_p, c_i64, c_i, c_p, c_i64, c_p, c_p, c_sz, c_pol,
                         c_p]),
     "q4nx_rmsnorm": (c_i, [c_p, c_i, c_p, c_p, c_p, c_i, c_i, c_f, c_p]),

@@ -66,6 +66,11 @@ size_t pq_ws_bytes(int kind, int op, int n_tile_rows, int k_t, int m_rows, bool 
 // whether a launch of op `op` described by `a` can take that kernel (its outputs' alignment and
 // strides; anything else is the batched kernel's, which reads and writes single values)
 bool pq_use(int kind, int op, const GemmArgs& a);
+// a workgroup's tile of a plain launch on it: rows of X, tile-rows, K parts
+struct PqTile {
+  int rows, tile_rows, parts;
+};
+PqTile pq_plain_tile(int kind, int n_tile_rows, int k_t, int m_rows, bool ssq);
 // launches `a` on it (with its RMSNorm prologue, if any): the pre-pass over x into `ws`
 // (pq_ws_bytes of it, 256-byte aligned), then the contraction
 void pq_launch(int kind, int op, const GemmArgs& a, void* ws, hipStream_t st);

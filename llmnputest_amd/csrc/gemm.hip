@@ -911,12 +911,19 @@ size_t q4nx_gemm_ws_bytes(int kind, int n_tile_rows, int k_tiles, int m_rows,
 }
 
 size_t q4nx_gemm_prompt_ws_bytes(int kind, int n_tile_rows, int k_tiles, int m_rows) {
+  return q4nx_gemm_prompt_tile(kind, n_tile_rows, k_tiles, m_rows)
+             ? Q4NX_WS_COUNTER_BYTES + pq_ws_bytes(kind, GOP_PLAIN, n_tile_rows, k_tiles, m_rows, false)
+             : 0;
+}
+
+int q4nx_gemm_prompt_tile(int kind, int n_tile_rows, int k_tiles, int m_rows) {
   Policy P;
   if (!gemm_shape_ok(kind, n_tile_rows, k_tiles, m_rows) || !resolve_policy_quiet(nullptr, &P) ||
       !pq_wanted(kind, GOP_PLAIN, n_tile_rows, k_tiles, m_rows, false,
                  plan_gemm(kind, GOP_PLAIN, n_tile_rows, k_tiles, m_rows, P), P))
     return 0;
-  return Q4NX_WS_COUNTER_BYTES + pq_ws_bytes(kind, GOP_PLAIN, n_tile_rows, k_tiles, m_rows, false);
+  const PqTile t = pq_plain_tile(kind, n_tile_rows, k_tiles, m_rows, false);
+  return t.rows << 16 | t.tile_rows << 8 | t.parts;
 }
 
 int q4nx_gemm(int kind, const uint8_t* w, int n_tile_rows, int k_tiles, const uint16_t* x,

@@ -17,7 +17,10 @@
 // group with exact products: no per-group scale on the VALU, and no large offset to cancel
 // afterwards. The second sum is a contraction over the groups (32 per MFMA), S and u each in two
 // fp16 terms (the product of the two low terms, 2^-22, is left out). A one-hot row still gives
-// the float32 dequantised column bit for bit.
+// the float32 dequantised column bit for bit, as long as u fits its two terms: |m| down to 2^-14 of
+// 8 |d|, below that it is kept to 2^-23 of 8 |d| (in fp32, m - 16 d was kept to 2^-24 of 16 |d|). The
+// 128-row tile adds the two terms one after the other to the codes' sum: one more rounding, none
+// where m = -8 d.
 //
 // Arithmetic, q8: y[m][n] = sum_g s[n][g] sum_{k in g} q[n][k] x[m][k]. s q has 15 bits, more than
 // one fp16 value holds, so the operand is the code alone (q = (1152 + q) - 1152, the byte under a
@@ -1282,48 +1285,66 @@ static bool fills_cus(int w) { return w >= 224 && w * 8 >= (w + 255) / 256 * 256
 // Tile by the workgroups it gives a chip of 256 CUs, two on each: the largest that fills it.
 // Measured over N x K of 512 x 1024 to 12288 x 4096 (q8: to 248320 x 1024) and 65 to 3000 rows; us
 // at the side of each line where the two are closest (N x K, rows):
-template <int KIND>
-static void pq_plain(const GemmArgs& a, const PqX& x, hipStream_t st) {
+PqTile pq_plain_tile(int kind, int n_tr, int k_t, int m_rows, bool ssq) {
   const auto wgs = [&](int rows, int trs) {
-    return ((a.m_rows + rows - 1) / rows) * ((a.n_tr[0] + trs - 1) / trs);
+    return ((m_rows + rows - 1) / rows) * ((n_tr + trs - 1) / trs);
   };
   const int w64 = wgs(64, 4);
-  if constexpr (KIND == 4) {
+  if (kind == Q4NX_KIND_Q4) {
     // 128 rows x 8 tile-rows, eight waves with K in two parts, one workgroup per CU, against the
     // same in one part and 64 x 4 (workgroups): 8192 x 2560 256 55.5 / 54.9 / 58.3, 512 100 / 86 /
     // 103; 4096 x 4096 256 73.9 / 74.8 / 84.6; 2560 x 8192, 3000 rows (240) 133 / 140 / 161; one that
     // leaves CUs idle in its last round loses (10240 x 4096 320 125 / 109 / 101). Its chains over K
     // are half as long, so launches with sums of squares, formerly the batched kernel's, take it
     // or 64 x 4 (768 144 / 148) where one chain is the less exact, from K = 1024 on.
-    const bool exact = a.ssq_out != nullptr && a.k_t >= 4;
-    const int w0 = a.m_rows < 128 ? 0 : wgs(128, 8);
-    if (a.k_t >= 8 && fills_cus(w0) && (w0 <= 256 || exact))
-      return pq_go<4, GOP_PLAIN, 8, 2, 4, 2, 4, 2>(a, x, st);
+    const bool exact = ssq && k_t >= 4;
+    const int w0 = m_rows < 128 ? 0 : wgs(128, 8);
+    if (k_t >= 8 && fills_cus(w0) && (w0 <= 256 || exact))
+      return {128, 8, 2};
     // the same in one part against 64 x 4: 640 rows (160) 53 / 47; a short K does not repay the
     // larger block's epilogue (6144 x 1024, 1500 rows (288) 44 / 38), and with fewer rows than the
     // block has the others are as fast and nearer to the 64-bit result
-    if (!exact && (w0 >= 512 || (w0 >= 240 && a.k_t >= 8)))
-      return pq_go<4, GOP_PLAIN, 8, 2, 4, 1, 4, 2>(a, x, st);
+    if (!exact && (w0 >= 512 || (w0 >= 240 && k_t >= 8)))
+      return {128, 8, 1};
     // 64 x 4 against 64 x 2 with K in two parts: 2560 x 8192, 1500 rows (480) 90 / 99, 1000 rows
     // (320) 80 / 72
-    if (w64 >= 440) return pq_go<4, GOP_PLAIN, 4, 1, 4, 1, 8, 2>(a, x, st);
+    if (w64 >= 440) return {64, 4, 1};
   } else {
     // 128 rows x 4 tile-rows (eight would take the LDS of both workgroups of a CU) against the
     // next: 8192 x 2560, 1000 rows (512) 68 / 79, 768 rows (384) 65 / 65, 640 rows (320) 64 / 60
-    if (wgs(128, 4) >= 384) return pq_go<8, GOP_PLAIN, 8, 1, 4, 1, 4, 2>(a, x, st);
+    if (wgs(128, 4) >= 384) return {128, 4, 1};
     // 64 x 4 when it fills the chip once, against 64 x 2 with K in two parts: 8192 x 2560, 400
     // rows (448) 40 / 43, 320 rows (320) 39 / 37, 640 rows (640) 62 / 60
-    if (w64 >= 440 && w64 <= 512) return pq_go<8, GOP_PLAIN, 4, 1, 4, 1, 8, 2>(a, x, st);
+    if (w64 >= 440 && w64 <= 512) return {64, 4, 1};
   }
   // two parts against four: 2560 x 8192, 400 rows (280) q4 50 / 56, q8 61 / 68, 256 rows (160)
   // q4 40 / 36, q8 46 / 40
-  if (wgs(64, 2) > 256) return pq_go<KIND, GOP_PLAIN, 4, 1, 2, 2, 4, 2>(a, x, st);
+  if (wgs(64, 2) > 256) return {64, 2, 2};
   // 64 x 2 in four parts against 32 x 2: 2560 x 8192, 256 rows (160) q4 36 / 48, q8 40 / 52, 192
   // rows (120) q4 35 / 31, q8 39 / 32
-  if (wgs(64, 2) >= 160) return pq_go<KIND, GOP_PLAIN, 4, 1, 2, 4, 4, 2>(a, x, st);
+  if (wgs(64, 2) >= 160) return {64, 2, 4};
   // 32 x 2 in four parts against 32 x 1 in eight: 2560 x 2560, 128 rows (320) q4 16 / 22, q8 16 /
   // 21, 96 rows (240) q4 16 / 14, q8 16 / 14
-  if (wgs(32, 1) > 256) return pq_go<KIND, GOP_PLAIN, 2, 1, 2, 4, 8, 2>(a, x, st);
+  if (wgs(32, 1) > 256) return {32, 2, 4};
+  return {32, 1, 8};
+}
+
+template <int KIND>
+static void pq_plain(const GemmArgs& a, const PqX& x, hipStream_t st) {
+  const PqTile t = pq_plain_tile(KIND, a.n_tr[0], a.k_t, a.m_rows, a.ssq_out != nullptr);
+  const auto is = [&](int rows, int trs, int parts) {
+    return t.rows == rows && t.tile_rows == trs && t.parts == parts;
+  };
+  if constexpr (KIND == 4) {
+    if (is(128, 8, 2)) return pq_go<4, GOP_PLAIN, 8, 2, 4, 2, 4, 2>(a, x, st);
+    if (is(128, 8, 1)) return pq_go<4, GOP_PLAIN, 8, 2, 4, 1, 4, 2>(a, x, st);
+  } else {
+    if (is(128, 4, 1)) return pq_go<8, GOP_PLAIN, 8, 1, 4, 1, 4, 2>(a, x, st);
+  }
+  if (is(64, 4, 1)) return pq_go<KIND, GOP_PLAIN, 4, 1, 4, 1, 8, 2>(a, x, st);
+  if (is(64, 2, 2)) return pq_go<KIND, GOP_PLAIN, 4, 1, 2, 2, 4, 2>(a, x, st);
+  if (is(64, 2, 4)) return pq_go<KIND, GOP_PLAIN, 4, 1, 2, 4, 4, 2>(a, x, st);
+  if (is(32, 2, 4)) return pq_go<KIND, GOP_PLAIN, 2, 1, 2, 4, 8, 2>(a, x, st);
   pq_go<KIND, GOP_PLAIN, 2, 1, 1, 8, 4, 2>(a, x, st);
 }
 

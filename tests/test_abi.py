@@ -288,6 +288,9 @@ def test_prompt_workspace_queries_ask_for_what_is_used():
     assert g(q4, 512, 2, 96) == 0 and g(q4, 3136, 2, 96) > 0 and g(q4, 3136, 2, 65) > 0
     assert g(q4, 256, 1, 256) == 0 and g(q4, 512, 1, 300) > 0 and g(q4, 32, 1, 6000) == 0
     assert g(q8, 128, 1, 512) == 0 and g(q8, 128, 1, 513) > 0
+    t = _lib.lib().q4nx_gemm_prompt_tile
+    assert t(q4, 80, 32, 333) == 64 << 16 | 2 << 8 | 4 and t(q4, 80, 32, 64) == 0
+    assert t(q8, 7760, 4, 512) == 128 << 16 | 4 << 8 | 1 and t(3, 80, 32, 333) == 0
     # [gate, up] under a named split is the batched kernel's: its normalised rows alone
     h = _lib.lib().q4nx_gate_up_ws_bytes
     assert h(256, 10, 500, pol(gemm_ksplit=1)) == 65536 + 500 * 2560 * 2 < h(256, 10, 500, None)

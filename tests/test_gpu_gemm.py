@@ -176,35 +176,38 @@ def test_gemm_q8_lm_head_prefill(dev):
     _check_rows(y[:, lo:hi], ref)
 
 
-# ------------------------------------------------------------------ prompt blocks (prefill kernel)
-# Launches that fill the chip go to the prefill kernel (raw codes on the matrix cores, the
-# group scale on the VALU, the minimum as a contraction over per-group sums of x): blocks of
-# 128 rows from 768 workgroups of four tile-rows, else 64-row blocks from 512; smaller
-# launches stay on the batched kernel above.
+# ------------------------------------------------------------------ prompt blocks
+# From 65 rows a launch goes to the fp16-operand kernel, whose workgroup tile (rows, tile-rows, K
+# parts) the library chooses by the workgroups each would give and names in a query. One shape per
+# tile, ragged both ways where it can be:
+TILE_SHAPES = {
+    "q4": {(32, 1, 8): (65, 32, 1024), (32, 2, 4): (129, 2080, 1024), (64, 2, 4): (257, 2080, 1280),
+           (64, 2, 2): (449, 2592, 1024), (64, 4, 1): (1500, 2464, 1024),
+           (128, 8, 1): (4100, 4128, 768), (128, 8, 2): (1900, 4320, 2304)},
+    "q8": {(32, 1, 8): (65, 32, 1024), (32, 2, 4): (129, 2080, 1024), (64, 2, 4): (257, 2080, 1280),
+           (64, 2, 2): (449, 2592, 1024), (64, 4, 1): (1500, 2464, 1024),
+           (128, 4, 1): (2900, 2208, 1024)},
+}
+EVERY_TILE = [(kind, t, *shape) for kind, d in TILE_SHAPES.items() for t, shape in d.items()]
 
-def _pf_workgroups(m, n, rows=128):
-    return -(-(n // 32) // 4) * -(-m // rows)
 
-
-def _pf_block_rows(m, n):
-    """Row-block size the library picks (0: not the prefill kernel)."""
-    if m >= 128 and _pf_workgroups(m, n, 128) >= 768:
-        return 128
-    if m >= 128 and _pf_workgroups(m, n, 64) >= 512:
-        return 64
-    return 0
+def _tile(kind, m, n, k):
+    """The tile of a prompt block (None: the batched kernel takes it)."""
+    from llmnputest_amd import _lib
+    v = _lib.lib().q4nx_gemm_prompt_tile(ops.KIND[kind], n // 32, k // 256, m)
+    return (v >> 16, v >> 8 & 255, v & 255) if v else None
 
 
 @pytest.mark.parametrize("kind", ["q4", "q8"])
 @pytest.mark.parametrize("m,n,k", [
     (4100, 2016, 512),   # 63 tile-rows: the last workgroup's fourth wave has none; ragged rows
     (2048, 4096, 1024),
-    (1544, 8192, 768),   # 128-row blocks; ragged rows, a partial chunk of groups (3 K-tiles)
-    (3100, 4064, 512),   # 128-row blocks, 127 tile-rows: the last workgroup's last wave has none
+    (1544, 8192, 768),   # ragged rows, a partial chunk of groups (3 K-tiles)
+    (3100, 4064, 512),   # 127 tile-rows: the last workgroup's last wave has none
 ])
 def test_gemm_prefill_parity(dev, kind, m, n, k):
     """Every row against the float64 oracle at the GEMV bar."""
-    assert _pf_block_rows(m, n) > 0
+    assert _tile(kind, m, n, k) == ((64, 4, 1) if kind == "q4" else (128, 4, 1))
     raw, rng = _tiles(kind, n, k, 21 + m)
     x = synth.random_bf16(rng, (m, k))
     y = ops.gemm(_dev_u8(raw, dev), kind, _dev_bf16(x, dev), n // 32, k // 256).cpu().numpy()
@@ -213,8 +216,9 @@ def test_gemm_prefill_parity(dev, kind, m, n, k):
 
 
 def test_gemm_prefill_long_k(dev):
-    """K = 8192 (32 tiles per wave, 256 pipelined steps): every row at the GEMV bar."""
+    """K = 8192 (16 tiles per wave and K part): every row at the GEMV bar."""
     m, n, k = 2048, 4096, 8192
+    assert _tile("q4", m, n, k) == (128, 8, 2)
     raw, rng = _tiles("q4", n, k, 23)
     x = synth.random_bf16(rng, (m, k))
     y = ops.gemm(_dev_u8(raw, dev), "q4", _dev_bf16(x, dev), n // 32, k // 256).cpu().numpy()
@@ -223,12 +227,12 @@ def test_gemm_prefill_long_k(dev):
 
 
 @pytest.mark.parametrize("kind", ["q4", "q8"])
-@pytest.mark.parametrize("n,m", [(2048, 4096), (8192, 1536)])   # 64- and 128-row blocks
+@pytest.mark.parametrize("n,m", [(2048, 4096), (8192, 1536)])
 def test_gemm_prefill_onehot_exact(dev, kind, n, m):
-    """One-hot rows reproduce the float32 dequantised column bit for bit: d (16 + c) (q4) or
-    s (q + 128) (q8) is exact, and so is its sum with the minimum term."""
+    """One-hot rows reproduce the float32 dequantised column bit for bit: the operand d c - o (q4)
+    or q under its scale (q8) is exact, and so is its sum with the minimum term."""
     k = 1024
-    assert _pf_block_rows(m, n) == (64 if n == 2048 else 128)
+    assert _tile(kind, m, n, k) == ((64, 4, 1) if kind == "q4" else (128, 4, 1))
     raw, _ = _tiles(kind, n, k, 3)
     cols = np.arange(m) * 5 % k
     x = np.zeros((m, k), np.float32)
@@ -241,12 +245,12 @@ def test_gemm_prefill_onehot_exact(dev, kind, n, m):
 
 @pytest.mark.parametrize("dist", ["student_t2", "outliers"])
 def test_gemm_prefill_heavy_tailed(dev, dist):
-    """Heavy-tailed activations on both row-block sizes: a few entries dwarf the rest of their
+    """Heavy-tailed activations on the three large tiles: a few entries dwarf the rest of their
     32-K group, so the group sums S carry most of the minimum term and the scaled code sums
     cancel against it."""
-    k = 1024
-    for m, n in ((1536, 8192), (2048, 2048)):
-        assert _pf_block_rows(m, n) > 0
+    for m, n, k, tile in ((1536, 8192, 1024, (64, 4, 1)), (2048, 2048, 1024, (64, 4, 1)),
+                          (2100, 4128, 2304, (128, 8, 1)), (1900, 4320, 2304, (128, 8, 2))):
+        assert _tile("q4", m, n, k) == tile
         raw, rng = _tiles("q4", n, k, 31 + m)
         if dist == "student_t2":
             xf = rng.standard_t(2.0, (m, k)).astype(np.float32)
@@ -261,10 +265,11 @@ def test_gemm_prefill_heavy_tailed(dev, dist):
 
 
 @pytest.mark.parametrize("scale", [1e-30, 1e30])
-def test_gemm_prefill_activation_range_residual_stride(dev, scale):
+@pytest.mark.parametrize("m,n,k,tile", [(4096, 2048, 512, (64, 4, 1)), (4100, 4128, 768, (128, 8, 1)),
+                                        (1900, 4320, 2304, (128, 8, 2))])
+def test_gemm_prefill_activation_range_residual_stride(dev, scale, m, n, k, tile):
     """Extreme activation ranges, rows with a stride longer than K and a residual."""
-    m, n, k = 4096, 2048, 512
-    assert _pf_block_rows(m, n) > 0
+    assert _tile("q4", m, n, k) == tile
     raw, rng = _tiles("q4", n, k, 14)
     xf = rng.standard_normal((m, k + 64)).astype(np.float32) * np.float32(scale)
     xfull = qo.bf16_round(xf)
@@ -278,11 +283,13 @@ def test_gemm_prefill_activation_range_residual_stride(dev, scale):
 
 
 @pytest.mark.parametrize("kind", ["q4", "q8"])
-@pytest.mark.parametrize("m,n,k", [(2048, 4096, 256), (1536, 8192, 512), (2048, 4096, 768)])
+@pytest.mark.parametrize("m,n,k", [(2048, 4096, 256), (1536, 8192, 512), (2048, 4096, 768),
+                                   (4100, 4128, 256), (4100, 4128, 512), (4100, 4128, 768)])
 def test_gemm_prefill_short_k(dev, kind, m, n, k):
-    """One to three K-tiles per tile-row: the first tile's reload, the clamped prefetch of the
-    tile after the last and the steps of x past the end all stay unused."""
-    assert _pf_block_rows(m, n) > 0
+    """One to three K-tiles per tile-row: the loads of tiles past the last and the steps of x past
+    the end all stay unused (the last three: the 128-row tile with its first wave of K alone)."""
+    assert _tile(kind, m, n, k) == ((128, 4, 1) if kind == "q8" else
+                                    (128, 8, 1) if m == 4100 else (64, 4, 1))
     raw, rng = _tiles(kind, n, k, 41 + k)
     x = synth.random_bf16(rng, (m, k))
     y = ops.gemm(_dev_u8(raw, dev), kind, _dev_bf16(x, dev), n // 32, k // 256).cpu().numpy()
@@ -291,11 +298,11 @@ def test_gemm_prefill_short_k(dev, kind, m, n, k):
 
 
 def test_gemm_prefill_without_workspace(dev):
-    """A prompt block with no workspace (NULL, 0), or one too small for the per-group sums of
-    x, runs on the batched kernel instead: every row at the same bar."""
+    """A prompt block with no workspace (NULL, 0), or one too small for the fp16 operands, runs on
+    the batched kernel instead: every row at the same bar."""
     from llmnputest_amd import _lib
     m, n, k = 2048, 4096, 512
-    assert _pf_block_rows(m, n) > 0
+    assert _tile("q4", m, n, k) is not None
     raw, rng = _tiles("q4", n, k, 43)
     x = synth.random_bf16(rng, (m, k))
     w, xd = _dev_u8(raw, dev), _dev_bf16(x, dev)
@@ -310,10 +317,7 @@ def test_gemm_prefill_without_workspace(dev):
 
 
 # ------------------------------------------------------------------ q4 prompt blocks on fp16 operands
-# From 65 rows q4 launches take the fp16-operand kernel, whose workgroup tile follows from the
-# workgroups each size would give: 128 rows x 8 tile-rows, 64 x 4, 64 x 2 with K in two or four
-# parts, 32 x 2 in four, 32 x 1 in eight. Its operands d (B + c) + A are exact and its sums fp32,
-# so every row is held to the GEMV bar; minima unrelated to the scales (every other case here has
+# The operands d (B + c) + A are exact and the sums fp32, so every row is held to the GEMV bar; minima unrelated to the scales (every other case here has
 # m = -8 d) make the minimum term carry a full share of the result.
 
 def _free_minima(raw, rng):
@@ -333,7 +337,7 @@ def _free_minima(raw, rng):
     (257, 2080, 1280),    # 64 x 2 in four parts: five K-tiles in parts of two, one empty
     (449, 2592, 768),     # 64 x 2 in two parts, ragged rows
     (1500, 2464, 256),    # 64 x 4: one K-tile, fewer steps than the ring holds ahead
-    (3900, 2016, 2048),   # 128 x 8, ragged rows, a last workgroup of seven tile-rows
+    (3900, 2016, 2048),   # 128 x 8 in two parts, ragged rows, a last workgroup of seven tile-rows
     (130, 128, 8448),     # rows longer than the pre-pass keeps in registers
 ])
 def test_gemm_fp16_operands_parity(dev, m, n, k):
@@ -768,3 +772,111 @@ def test_prompt_block_keeps_its_kernel_under_a_ksplit(dev, kind, m, n, k, parts)
     _lib.call("q4nx_gemm", ops.KIND[kind], w.data_ptr(), n // 32, k // 256, xd.data_ptr(), k, m,
               y.data_ptr(), n, None, None, 0, None, ops._stream())
     assert not torch.equal(y, want)
+
+
+# ------------------------------------------------------------------ every tile
+
+def _onehot_rows(m, k, dev):
+    cols = torch.from_numpy(np.arange(m) * 7 % k).to(dev)
+    x = torch.zeros((m, k), dtype=torch.bfloat16, device=dev)
+    x[torch.arange(m, device=dev), cols] = 1.0
+    return x, cols
+
+
+def _onehot_check(y, raw, kind, n, k, cols, dev, rows=0):
+    """Rows of y against the columns `cols` of the float32 dequantised matrix: the same bits; where a
+    q4 minimum is below 2^-14 of 8 d (its bits end past the two terms of u) or is added on top of
+    the codes' sum (minima other than -8 d on the 128-row tiles) to 2^-22 of 8 d, m and the value."""
+    column = lambda r: ops.dequant(_dev_u8(r, dev), kind, n // 32, k // 256, out_dtype=torch.float32,
+                                   untile=True)[:, cols].t()
+    want = column(raw)
+    if kind == "q8":
+        assert torch.equal(y, want)
+        return
+    lo, hi = raw.copy(), raw.copy()
+    lo[:, 1024:], hi[:, 1024:], hi[:, 512:1024] = 0, 0x11, 0     # the minimum; the scale
+    m, d8 = column(lo).abs(), 8 * column(hi).abs()
+    far = (m < 2.0 ** -14 * d8) | ((m != d8) & (rows == 128))
+    assert torch.equal(torch.where(far, want, y), want)
+    assert ((y - want).abs()[far] <= 2.0 ** -22 * (m + d8 + want.abs())[far]).all()
+
+
+@pytest.mark.parametrize("kind,tile,m,n,k,minima", [(*c, v) for c in EVERY_TILE
+                                                    for v in ("zero_point", "free")
+                                                    if c[0] == "q4" or v == "zero_point"])
+def test_every_tile_onehot_exact(dev, kind, tile, m, n, k, minima):
+    """One-hot rows on every tile (the K parts that do not hold the entry add zeros)."""
+    assert _tile(kind, m, n, k) == tile
+    raw, rng = _tiles(kind, n, k, 500 + m)
+    if minima == "free":
+        raw = _free_minima(raw, rng)
+    x, cols = _onehot_rows(m, k, dev)
+    y = ops.gemm(_dev_u8(raw, dev), kind, x, n // 32, k // 256)
+    _onehot_check(y, raw, kind, n, k, cols, dev, tile[0])
+
+
+@pytest.mark.parametrize("batch,n,k", [
+    (65, 96, 1024),            # 32 x 1 pairs
+    (200, 1312, 768),          # 32 x 2
+    (300, 2080, 2816),         # 64 x 2 in two parts
+    (900, 1984, 1280),         # 64 x 4
+    (1000, 3616, 2304),        # 128 x 4 in two parts
+])
+def test_gate_up_onehot_exact(dev, batch, n, k):
+    """The same for the gate and the up values of [gate, up]."""
+    rng = np.random.default_rng(600 + batch)
+    w = [synth.q4_tiles(rng, n, k).reshape(-1, qo.Q4_TILE_BYTES) for _ in range(2)]
+    w[1] = _free_minima(w[1], rng)
+    x, cols = _onehot_rows(batch, k, dev)
+    raw_out = torch.empty((batch, 2 * n), device=dev)
+    ops.gate_up_swiglu(_dev_u8(w[0], dev), _dev_u8(w[1], dev), n // 32, k // 256, x, raw_out=raw_out)
+    for t, o in ((w[0], 0), (w[1], n)):
+        _onehot_check(raw_out[:, o:o + n], t, "q4", n, k, cols, dev, 128 if batch == 1000 else 64)
+
+
+@pytest.mark.parametrize("kind", ["q4", "q8"])
+@pytest.mark.parametrize("m,n,k", [(65, 96, 1024), (70, 64, 2560), (300, 2080, 4096),
+                                   (449, 2592, 4352), (1500, 2464, 512)])
+def test_prompt_block_norm_prologue(dev, kind, m, n, k):
+    """A projection with its RMSNorm in the pre-pass (4, 1 and 1 rows per workgroup of 256, 256 and
+    512 threads) gives the bits of the projection of the rows that [RMSNorm, gate, up] normalises."""
+    raw, rng = _tiles(kind, n, k, 700 + m)
+    w = _dev_u8(raw, dev)
+    x = torch.from_numpy((rng.standard_normal((m, k)) * 3).astype(np.float32)).to(dev)
+    kw = dict(norm_w=_dev_bf16(synth.random_bf16(rng, k), dev),
+              ssq_in=x.view(m, -1, 16).square().sum(-1).contiguous())
+    xn = torch.zeros((m, k), dtype=torch.bfloat16, device=dev)
+    gate = _dev_u8(synth.q4_tiles(rng, 32, k), dev)
+    ops.gate_up_swiglu(gate, gate, 1, k // 256, x, xn_out=xn, **kw)
+    y = ops.gemv_ex(w, kind, x, n // 32, k // 256, **kw)
+    assert _tile(kind, m, n, k) is not None
+    assert torch.equal(y, ops.gemm(w, kind, xn, n // 32, k // 256))
+    xb = xn.view(torch.int16).cpu().numpy().view(np.uint16)
+    rows = np.unique(np.concatenate([np.arange(0, m, max(1, m // 24)), [m - 1]]))
+    _check_rows(y.cpu().numpy()[rows], qo.gemv(raw, kind, xb[rows], n // 32, k // 256, acc=np.float64))
+
+
+@pytest.mark.parametrize("m,n,k,gateup", [
+    (130, 26272, 2304, False),    # 64 x 4: 821 tile-rows, no multiple of eight tiles
+    (300, 26272, 2304, False),    # 128 x 8
+    (130, 13088, 2304, True),     # [gate, up]: 409 pairs
+    (1030, 13088, 2304, True),
+])
+def test_q4_weights_beyond_the_l2(dev, m, n, k, gateup):
+    """q4 weights of more than 32 MB: row blocks first within an XCD's share of the tiles."""
+    g = torch.Generator(device=dev)
+    g.manual_seed(m)
+    from llmnputest_amd.granite import random_q4_tiles
+    w = [random_q4_tiles(n, k, g, dev) for _ in range(1 + gateup)]
+    assert sum(t.numel() for t in w) > 32 << 20
+    x = torch.randn((m, k), device=dev, generator=g).to(torch.bfloat16)
+    if gateup:
+        y = torch.full((m, 2 * n), float("nan"), device=dev)
+        ops.gate_up_swiglu(w[0], w[1], n // 32, k // 256, x, raw_out=y)
+    else:
+        y = ops.gemm(w[0], "q4", x, n // 32, k // 256)
+    for i, t in enumerate(w):
+        wm = ops.dequant(t, "q4", n // 32, k // 256, out_dtype=torch.float32, untile=True).double()
+        ref = x.double() @ wm.t().contiguous()
+        err = (y[:, i * n:(i + 1) * n].double() - ref).abs()
+        assert (err <= REL * ref.abs().amax(1, keepdim=True)).all()
