@@ -26,7 +26,7 @@
 // one fp16 value holds, so the operand is the code alone (q = (1152 + q) - 1152, the byte under a
 // fixed exponent less a constant) and one MFMA from zero per 16x16 block and group gives the
 // inner sum, which four FMAs per lane scale into the total. (Two MFMAs on s = s1 + s2, four bits
-// each, and no FMA took 555 us for 512 rows of 248320 x 1024, this 471.) x and s under powers of two
+// each, and no FMA took 555 us for 512 rows of 248320 x 1024, this 406.) x and s under powers of two
 // as above.
 //
 // Range. Under a row's power of two an entry of x is exact down to 2^-31 of the row's largest and
@@ -661,14 +661,14 @@ __device__ __forceinline__ void exact_tile(const GemmArgs& a, const PqX& p, uint
 // x (a ring of RING 32-K steps) and the codes (a K-tile in two halves) go from memory to LDS by
 // direct loads, counted by hand, with no registers in between; the step's operands are built
 // beside its MFMAs, in 18 VALU instructions per tile-row, so the matrix cores set the pace.
-// What bounds it: two workgroups of the 128-row tile run the main loop at 1.76 PFLOP/s (an MFMA
-// loop with random operands and nothing else reaches 1.6-1.9 here, held by the power limit); the
-// pre-pass, the first loads and the outputs, all of a launch's at once, are not overlapped with
-// it. N x K, rows, before (scale after the MFMA, one FMA per output and group; below 512
-// workgroups the batched kernel) and now, pre-pass included: 8192 x 2560, 2048 rows 149 -> 95 us
-// (575 -> 905 TFLOP/s); 2560 x 8192, 333 rows 62 -> 37; [gate, up] 8192 x 2560, 500 rows 126 ->
-// 57 us, 2048 rows 477 -> 193. Error against 64 bits: 2048 rows, K = 2560 1.06e-6 -> 3.2e-7, 333
-// rows, K = 8192 3.1e-7 -> 1.2e-7.
+// What bounds it (2048 rows of 8192 x 2560, 83 us): more K adds at 1.23 to 1.30 PFLOP/s, with the
+// clock held at 2.0 to 2.1 GHz under that load and the matrix cores busy 0.51 of the time (0.59 at K
+// = 5120); 17 us of the launch -- the first loads and the outputs, all of its workgroups' at once --
+// and the pre-pass's 9 are not overlapped with it. Calls, pre-pass included, before (scale after the
+// MFMA, one FMA per output and group; below 512 workgroups and [gate, up] the batched kernel) and now,
+// us, N x K, rows: 8192 x 2560, 2048 rows 124 -> 86; 2560 x 8192, 333 rows 57 -> 31; [gate, up] 8192 x
+// 2560, 500 rows 126 -> 55, 2048 rows 477 -> 185. Error against 64 bits: 2048 rows, K = 2560 1.05e-6 ->
+// 3.2e-7, 333 rows, K = 8192 3.1e-7 -> 1.2e-7, [gate, up], K = 2560 2.6e-7 -> 2.2e-7.
 template <int KIND, int OP, int MT, int RT, int WN, int WK, int RING, int OCC>
 __global__ __launch_bounds__(64 * WN * WK, OCC) void pq_kernel(GemmArgs a, PqX p) {
   constexpr int TB = GemmFmt<KIND>::kTile, HALF = kPqHalf<KIND>;
@@ -1232,9 +1232,10 @@ void pq_go(const GemmArgs& a, PqX x, hipStream_t st) {
   x.c_groups = (units + WN - 1) / WN;
   // Weights beyond the eight L2s (4 MB each) would be read from memory again for every row block.
   // The dispatcher deals workgroups to the XCDs in turn, so each XCD then takes an eighth of the
-  // tiles, all row blocks of a group of columns before the next group. 512 x 248320 x 1024 (q8)
-  // 620 -> 562 us, 102 x 163200 x 2048 (q4) 146 -> 138; smaller weights stay in column order:
-  // 1000 x 2560 x 8192 (q4) 73, rows first 82.
+  // tiles, all row blocks of a group of columns before the next group. Columns first / rows first,
+  // us: 248320 x 1024 (q8, 258 MB), 512 rows 443..471 / 406, 200 rows 225 / 209; 163200 x 2048 (q4,
+  // 199 MB), 102 rows 143 / 134; 26272 x 2304 (q4, 36 MB), 300 rows 74.5 / 72.5; smaller weights stay
+  // in column order: 8192 x 4096 (q4, 20 MB), 1000 rows 75.3 / 74.8, 2560 x 8192 (12 MB) 70 / 81.
   x.rows_first = (size_t)a.n_tr[0] * (OP == GOP_PLAIN ? 1 : 2) * a.k_t * GemmFmt<KIND>::kTile > (32u << 20);
   const int tiles = x.c_groups * x.m_blocks;
   const dim3 grid((unsigned)((tiles + 7) / 8 * 8));
