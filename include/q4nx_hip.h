@@ -12,10 +12,11 @@
  *   - Tiled weights are raw q4nx bytes, [n_tile_rows][k_tiles][tile], exactly as stored
  *     in a .q4nx file (tools/q4nx.py:1-18): q4 tiles are 5120 B, q8 tiles 8704 B.
  *   - Workspaces (`ws`) are laid out as Q4NX_WS_COUNTER_BYTES of arrival counters
- *     followed by fp32 partial sums. They must be zero-filled once before their first
- *     use; every call leaves the counters at zero again, whatever the shapes of the
- *     calls that share the workspace. Calls that share a workspace must be ordered on
- *     one stream. Any entry point's ws_bytes query includes the counter region.
+ *     followed by fp32 partial sums or a prompt block's operands. They must be zero-filled
+ *     once before their first use; every call leaves the counters at zero again, whatever
+ *     the shapes of the calls that share the workspace. Calls that share a workspace must be
+ *     ordered on one stream and not be issued by two host threads at once (a call may be two
+ *     launches that meet there). Any entry point's ws_bytes query includes the counter region.
  *   - Entry points that choose between kernel families or work splits take a
  *     `const q4nx_policy *policy` (NULL = the defaults of q4nx_policy_init). The library
  *     keeps no mutable state of its own: calls with different policies, from any thread,
